@@ -16,8 +16,12 @@
 // kNN: one lane per query.  Per depth level the lane keeps in LDS the first child and the
 // children still to visit in increasing box distance (so the search reaches the query's own
 // leaves first and the k-th distance bound tightens early); small subtrees are scanned as
-// contiguous point ranges.  Candidates are kept in registers as a sorted array of 64-bit keys
-// (distance bits << 32 | sorted point index).  Ball: one walk per wavefront over the union of
+// contiguous point ranges.  Candidates within the bound are buffered in LDS and merged, by all lanes
+// of a wavefront together, into a sorted array of 64-bit keys in registers (distance bits << 32 |
+// sorted point index).  The kernel is bound by vector instructions (VALU 94 % busy, k = 32): merging
+// together runs the insertion about as often as the fullest lane needs it instead of once per point
+// that any lane takes (k = 32, 5M points, 4M queries, FP32C: 12.0 ms a step with 64-bit integer
+// compares, 7.7 with keys as doubles, 5.9 with the buffers).  Ball: one walk per wavefront over the union of
 // its lanes' balls (k_ball_wave).
 #include <cfloat>
 #include <cmath>
@@ -48,24 +52,35 @@ __device__ __forceinline__ float kd_d2(float4 p, V3<float> q) {
   return (dx * dx + dy * dy) + dz * dz;
 }
 
-// Squared distance from q to a node's closed box (a lower bound for all its points).
-__device__ __forceinline__ float box_d2(const float* __restrict__ box, uint32_t c, V3<float> q) {
-  const float2 a = *reinterpret_cast<const float2*>(box + 6 * (size_t)c);
-  const float2 b = *reinterpret_cast<const float2*>(box + 6 * (size_t)c + 2);
-  const float2 e = *reinterpret_cast<const float2*>(box + 6 * (size_t)c + 4);
-  // a = (lo.x, lo.y), b = (lo.z, hi.x), e = (hi.y, hi.z)
-  const float dx = fmaxf(fmaxf(a.x - q.x, q.x - b.y), 0.f);
-  const float dy = fmaxf(fmaxf(a.y - q.y, q.y - e.x), 0.f);
-  const float dz = fmaxf(fmaxf(b.x - q.z, q.z - e.y), 0.f);
+// A lower bound of the squared distance from q to the points of a node, from the node's centre (one
+// 16-byte record) and the half extents of its depth: `h` holds the root's half extents over 2^depth,
+// grown by what float rounding moves a cell's bounds and centre (HalfBox), so the box it spans
+// contains the cell.  The cell's own bounds are 24 bytes in three loads (k = 32, 5M points, 4M
+// queries: 7.7 ms a step with them, 7.4 with the centres).
+struct HalfBox {
+  float x, y, z, eps;  // the root's half extents; the rounding margin
+};
+__device__ __forceinline__ V3<float> half_at(HalfBox hb, uint32_t depth) {
+  return V3<float>{ldexpf(hb.x, -(int)depth) + hb.eps, ldexpf(hb.y, -(int)depth) + hb.eps,
+                   ldexpf(hb.z, -(int)depth) + hb.eps};
+}
+__device__ __forceinline__ float cell_d2(float4 g, V3<float> h, V3<float> q) {
+  const float dx = fmaxf(fabsf(q.x - g.x) - h.x, 0.f);
+  const float dy = fmaxf(fabsf(q.y - g.y) - h.y, 0.f);
+  const float dz = fmaxf(fabsf(q.z - g.z) - h.z, 0.f);
   return (dx * dx + dy * dy) + dz * dz;
 }
 
 // Bound slack: box distances are float-rounded, so a node is kept while its bound is within
-// a relative 1e-5 of the search radius (a superset of the exact test).
+// a relative 1e-4 of the squared search radius (a superset of the exact test).
 constexpr float kSlack = 1.0001f;
 
 // kNN: subtrees of at most this many points are scanned rather than walked.
 constexpr uint32_t kScanPointsKnn = 8;
+// kNN: candidates within the bound are buffered in LDS and merged into the sorted keys by all lanes
+// of a wavefront together, once one of them holds kBufFill; a lane scans at most kBufFill points
+// between two merges.
+constexpr uint32_t kBufFill = 8, kBufCap = 2 * kBufFill - 1;
 
 // Weighted sums of the neighbours (CPUUtils.cpp:719-731): unit area, raw p and n.
 struct SumF {  // plain FP32
@@ -241,48 +256,64 @@ __device__ __forceinline__ void fit_step(const typename Sums<FORM>::S& s, V3<dou
   }
 }
 
-// Sorted (ascending) candidate keys of the k nearest, in registers.  Real keys are
-// (distance bits << 32) | (sorted point index + 1); the first KMAX - k slots hold the
-// sentinel 0, smaller than every real key and never displaced, so the k-th smallest real key
-// is always the last slot (a static register index).
+// Sorted (ascending) candidate keys of the k nearest, in registers.  A key is
+// (distance bits << 32) | (sorted point index + 1) held as a double: distance bits are those of a
+// non-negative float (a NaN is cut to 0x7fc00000), so every key is a finite non-negative double and
+// doubles order as the 64-bit integers do.  One slot of the insertion is then v_max_f64 and
+// v_min_f64 (full rate on this chip) instead of two 64-bit integer compares and four selects: 64
+// vector instructions an insertion at k = 32 against 192.  The first KMAX - k slots hold the
+// sentinel 0, smaller than every real key and never displaced, so the k-th smallest real key is
+// always the last slot (a static register index); empty slots hold +inf.  Both have a zero low word.
+__device__ __forceinline__ double min_key(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double max_key(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double make_key(float d2, uint32_t j) {
+  const uint32_t hi = min(__float_as_uint(d2) & 0x7fffffffu, 0x7fc00000u);
+  return __hiloint2double((int)hi, (int)(j + 1u));
+}
+
 template <int KMAX>
 struct TopK {
-  uint64_t key[KMAX];
+  double key[KMAX];
   __device__ __forceinline__ void clear(uint32_t k) {
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) key[j] = (uint32_t)j < KMAX - k ? 0ull : ~0ull;
+    for (int j = 0; j < KMAX; ++j) key[j] = (uint32_t)j < KMAX - k ? 0.0 : (double)INFINITY;
   }
-  __device__ __forceinline__ void insert(uint64_t x) {
-    if (x >= key[KMAX - 1]) return;
+  __device__ __forceinline__ void insert(double x) {
+    if (!(x < key[KMAX - 1])) return;
 #pragma unroll
-    for (int j = KMAX - 1; j > 0; --j) {
-      const uint64_t lo = key[j - 1] < x ? x : key[j - 1];  // max(key[j-1], x)
-      key[j] = key[j] < lo ? key[j] : lo;                   // min(key[j], max(key[j-1], x))
-    }
-    key[0] = key[0] < x ? key[0] : x;
+    for (int j = KMAX - 1; j > 0; --j) key[j] = min_key(key[j], max_key(key[j - 1], x));
+    key[0] = min_key(key[0], x);
   }
-  // removes and returns the smallest key (register shift, static indices only)
-  __device__ __forceinline__ uint64_t pop_front() {
-    const uint64_t v = key[0];
-#pragma unroll
-    for (int j = 0; j < KMAX - 1; ++j) key[j] = key[j + 1];
-    key[KMAX - 1] = ~0ull;
-    return v;
+  // squared distance of the k-th candidate, infinite while there are fewer
+  __device__ __forceinline__ float bound() const {
+    const uint32_t hi = (uint32_t)__double2hiint(key[KMAX - 1]);
+    return hi == 0x7ff00000u ? INFINITY : __uint_as_float(hi);
   }
-  __device__ __forceinline__ uint64_t kth() const { return key[KMAX - 1]; }
 };
 
 template <int FORM, int KT, int KMAX>
-// The 32 sorted 64-bit keys take 64 VGPRs; the FP32 forms are held to three waves per SIMD (the
-// compensated form then spills ~64 B per lane, cheaper than the lost wave), the FP64 form keeps two.
+// The 32 sorted 64-bit keys take 64 VGPRs; the FP32 forms fit four waves per SIMD (119 VGPRs).
 __global__ __launch_bounds__(NBS) __attribute__((amdgpu_waves_per_eu(FORM == 2 ? 1 : 3)))
-void k_knn(TreeView tv, const float* __restrict__ box, KParams kp,
+void k_knn(TreeView tv, HalfBox hb, KParams kp,
                                              float4* __restrict__ q, float4* __restrict__ qn,
                                              const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit, uint32_t nIter,
                                              uint32_t k) {
-  __shared__ uint32_t sFirst[kLevels][NBS];
-  __shared__ uint32_t sOrder[kLevels][NBS];  // children still to visit, nearest first, 4 bits each
-  __shared__ uint8_t sLeft[kLevels][NBS];    // how many
+  // per lane: the search's stack (two words a level) and the buffered candidates, then the found
+  // indices of the step
+  constexpr int kStack = 2 * kLevels, kWords = KMAX > kStack + kBufCap ? KMAX : kStack + kBufCap;
+  __shared__ uint32_t sWords[kWords][NBS];
+  uint32_t (*sFirst)[NBS] = sWords;            // first child
+  uint32_t (*sOrder)[NBS] = sWords + kLevels;  // waiting children, nearest first, 3 bits each; their
+                                               // number << 24; their depth << 28
+  uint32_t (*sBuf)[NBS] = sWords + kStack;
   const int tid = threadIdx.x;
   const uint32_t i = xcd_block() * NBS + tid;
   if (i >= m) return;
@@ -294,39 +325,52 @@ void k_knn(TreeView tv, const float* __restrict__ box, KParams kp,
     const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
     TopK<KMAX> top;
     top.clear(k);
-    float bound = INFINITY;  // squared distance of the current k-th candidate
-    const uint4 h0 = tv.hdr[0];
+    float bound = INFINITY;  // squared distance of the k-th candidate when last merged
+    uint32_t cnt = 0;        // buffered candidates
+    // inserts the buffered candidates of every lane (their distances are computed again: the points
+    // were just read)
+    const auto merge = [&]() {
+#pragma unroll 1
+      for (uint32_t b = 0; b < cnt; ++b) {
+        const uint32_t j = sBuf[b][tid];
+        top.insert(make_key(kd_d2(tv.pts[j], qf), j));
+      }
+      cnt = 0;
+      bound = top.bound();
+    };
     int lvl = -1;
-    uint32_t cur = 0;  // node to expand next (root first)
+    uint32_t cur = 0;         // node to expand next (root first)
+    uint32_t sa = 0, sb = 0;  // points still to scan
     bool have = true;
     while (true) {
       if (have) {
-        const uint4 h = cur == 0 ? h0 : tv.hdr[cur];
+        const uint4 h = tv.hdr[cur];
         const uint2 sp = tv.span[cur];
+        have = false;
         if (hdr_leaf(h.y) || sp.y - sp.x <= kScanPointsKnn) {
           // a leaf or a small subtree: every point is a candidate (the k nearest do not depend
           // on the order they are offered in)
-          for (uint32_t j = sp.x; j < sp.y; ++j) {
-            const float d2 = kd_d2(tv.pts[j], qf);
-            top.insert(((uint64_t)__float_as_uint(d2) << 32) | (j + 1u));
-          }
-          const uint64_t kk = top.kth();
-          bound = kk == ~0ull ? INFINITY : __uint_as_float((uint32_t)(kk >> 32));
+          sa = sp.x;
+          sb = sp.y;
         } else {
           // children whose box reaches the bound, visited nearest box first, so that the
           // first leaves reached are the query's own and the bound tightens at once
           const uint32_t first = h.x, nc = hdr_count(h.y);
+          const V3<float> hc = half_at(hb, hdr_depth(h.y) + 1u);
           // keys: the box distance's bits (non-negative floats order as integers) with the child
           // slot in the low 3 bits, children beyond the bound last; an 8-input sorting network
           // (19 compare-exchanges) orders them.  The visiting order only steers the search: the
-          // k nearest do not depend on it
-          uint32_t key[8], cnt = 0;
+          // k nearest do not depend on it.  All eight centres are loaded before the first is used
+          float4 g[8];
+#pragma unroll
+          for (uint32_t c = 0; c < 8; ++c) g[c] = tv.geo[first + min(c, nc - 1u)];
+          uint32_t key[8], n = 0;
 #pragma unroll
           for (uint32_t c = 0; c < 8; ++c) {
-            const float d = c < nc ? box_d2(box, first + c, qf) : INFINITY;
+            const float d = cell_d2(g[c], hc, qf);
             const bool in = c < nc && d <= bound * kSlack;
             key[c] = in ? (__float_as_uint(d) & ~7u) | c : 0xffffffffu;
-            cnt += in ? 1u : 0u;
+            n += in ? 1u : 0u;
           }
           const auto cx = [&](int a, int b) {
             const uint32_t lo = min(key[a], key[b]), hi = max(key[a], key[b]);
@@ -334,39 +378,47 @@ void k_knn(TreeView tv, const float* __restrict__ box, KParams kp,
           };
           cx(0, 2), cx(1, 3), cx(4, 6), cx(5, 7), cx(0, 4), cx(1, 5), cx(2, 6), cx(3, 7), cx(0, 1), cx(2, 3);
           cx(4, 5), cx(6, 7), cx(2, 4), cx(3, 5), cx(1, 4), cx(3, 6), cx(1, 2), cx(3, 4), cx(5, 6);
-          uint32_t order = 0;
+          uint32_t order = (hdr_depth(h.y) + 1u) << 28 | n << 24;
 #pragma unroll
-          for (uint32_t r = 0; r < 8; ++r) order |= (key[r] & 7u) << (4u * r);
-          ++lvl;
-          sFirst[lvl][tid] = first;
-          sOrder[lvl][tid] = order;
-          sLeft[lvl][tid] = (uint8_t)cnt;
+          for (uint32_t r = 0; r < 8; ++r) order |= (key[r] & 7u) << (3u * r);
+          if (n) {
+            ++lvl;
+            sFirst[lvl][tid] = first;
+            sOrder[lvl][tid] = order;
+          }
         }
-        have = false;
       }
+      // scan at most kBufFill points: those that the bound does not rule out are buffered
+      for (uint32_t e = min(sb, sa + kBufFill); sa < e; ++sa) {
+        if (!(kd_d2(tv.pts[sa], qf) > bound)) {
+          sBuf[cnt][tid] = sa;
+          ++cnt;
+        }
+      }
+      if (__any(cnt >= kBufFill)) merge();
+      if (sa < sb) continue;
       if (lvl < 0) break;
-      const uint32_t left = sLeft[lvl][tid];
-      if (left == 0) {
-        --lvl;
-        continue;
-      }
-      const uint32_t order = sOrder[lvl][tid];
-      sOrder[lvl][tid] = order >> 4;
-      sLeft[lvl][tid] = (uint8_t)(left - 1u);
-      const uint32_t c = sFirst[lvl][tid] + (order & 15u);
-      if (box_d2(box, c, qf) <= bound * kSlack) {  // the bound may have shrunk since the push
+      const uint32_t w = sOrder[lvl][tid];
+      const uint32_t c = sFirst[lvl][tid] + (w & 7u);
+      const uint32_t rest = ((w & 0xffffffu) >> 3) + (w & 0xff000000u) - (1u << 24);
+      sOrder[lvl][tid] = rest;
+      if (!(rest & 0x0f000000u)) --lvl;
+      if (cell_d2(tv.geo[c], half_at(hb, w >> 28), qf) <= bound * kSlack) {  // the bound may have shrunk since the push
         cur = c;
         have = true;
       }
     }
+    merge();
+    // the found indices through this lane's own LDS column (a rolled loop cannot index registers),
+    // summed nearest first
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) sWords[j][tid] = (uint32_t)__double2loint(top.key[j]);
     typename Sums<FORM>::S s{};
 #pragma unroll 1
-    for (uint32_t j = 0; j < KMAX; ++j) {
-      const uint64_t key = top.pop_front();
-      if (key == 0ull) continue;  // sentinel
-      if (key == ~0ull) break;    // fewer than k points in the cloud
-      const uint32_t pj = (uint32_t)key - 1u;
-      add_nb<FORM, KT>(s, kp, tv.pts[pj], tv.nrm[pj], qd, qf);
+    for (uint32_t j = KMAX - k; j < KMAX; ++j) {
+      const uint32_t pj = sWords[j][tid];
+      if (pj == 0u) break;  // fewer than k points (of a finite distance) found
+      add_nb<FORM, KT>(s, kp, tv.pts[pj - 1u], tv.nrm[pj - 1u], qd, qf);
     }
     fit_step<FORM>(s, qd, qf, nout);
   }
@@ -500,6 +552,20 @@ __global__ __launch_bounds__(NBS) void k_ball_wave(TreeView tv, const float* __r
   }
 }
 
+// The root's half extents and the rounding margin of a cell's bounds.  Every bound of a cell is the
+// root's or a split rounded to float, so it is within 2^-24 M of the exact halving of its own
+// level's bounds (M: the largest |coordinate| of the root box); those errors halve from level to
+// level, so an extent is within 4 * 2^-24 M of the root's over 2^depth, and the centre is rounded once
+// more.  The products and sums here and in the kernel round too: 16 * 2^-24 M covers them all.
+HalfBox half_box(const mlod_tree* t) {
+  float m = 0.f, h[3];
+  for (int a = 0; a < 3; ++a) {
+    m = fmaxf(m, fmaxf(fabsf(t->bb[a]), fabsf(t->BB[a])));
+    h[a] = 0.5f * (t->BB[a] - t->bb[a]);
+  }
+  return HalfBox{h[0], h[1], h[2], m * (16.f / 16777216.f)};
+}
+
 template <int FORM, int KT>
 int launch_form(mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter, hipStream_t s) {
   const uint32_t m = t->qs.m;
@@ -507,13 +573,13 @@ int launch_form(mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter,
   if (t->mode == MLOD_MODE_KNN) {
     const uint32_t k = t->knn < t->n ? t->knn : t->n;
     if (k <= 8)
-      k_knn<FORM, KT, 8><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
+      k_knn<FORM, KT, 8><<<grid, NBS, 0, s>>>(t->view(), half_box(t), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
     else if (k <= 16)
-      k_knn<FORM, KT, 16><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
+      k_knn<FORM, KT, 16><<<grid, NBS, 0, s>>>(t->view(), half_box(t), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
     else if (k <= 32)
-      k_knn<FORM, KT, 32><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
+      k_knn<FORM, KT, 32><<<grid, NBS, 0, s>>>(t->view(), half_box(t), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
     else if (k <= 64)
-      k_knn<FORM, KT, 64><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
+      k_knn<FORM, KT, 64><<<grid, NBS, 0, s>>>(t->view(), half_box(t), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, k);
     else
       return fail(MLOD_ERR_UNSUPPORTED, "kNN supports k <= 64");
   } else {
