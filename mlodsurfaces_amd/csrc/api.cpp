@@ -29,7 +29,7 @@ int hip_fail(hipError_t e, const char* what, const char* file, int line) {
 static void free_tree(mlod_tree* t) {
   if (!t) return;
   queries_free(t);
-  void* bufs[] = {t->geo, t->hdr, t->momP, t->momC, t->momD, t->AD, t->pts, t->nrm, t->order, t->box, t->area, t->span};
+  void* bufs[] = {t->geo, t->hdr, t->recP, t->recC, t->momD, t->AD, t->pts, t->nrm, t->order, t->box, t->area, t->span};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
   delete t;

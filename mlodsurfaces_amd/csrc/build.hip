@@ -485,8 +485,9 @@ struct KSum {
 };
 
 __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint4* __restrict__ hdr,
-                                                const float4* __restrict__ pts, const float4* __restrict__ nrm,
-                                                float4* __restrict__ momP, float4* __restrict__ momC,
+                                                const float4* __restrict__ geo, const float4* __restrict__ pts,
+                                                const float4* __restrict__ nrm, float4* __restrict__ recP,
+                                                float4* __restrict__ recC,
                                                 double4* __restrict__ momD, double* __restrict__ AD) {
   const uint32_t k = beg + blockIdx.x * BS + threadIdx.x;
   if (k >= end) return;
@@ -532,7 +533,7 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
   } else {
     // plain sums in child slot order (CPUUtils.cpp:379-396)
     for (uint32_t j = first; j < first + cnt; ++j) {
-      const float4 m0 = momP[2 * (uint64_t)j], m1 = momP[2 * (uint64_t)j + 1];
+      const float4 m0 = recP[4 * (uint64_t)j + 2], m1 = recP[4 * (uint64_t)j + 3];
       const M9f o{__uint_as_float(hdr[j].z), m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, m0.w, m1.w};
       add_f(sf, o);
       const double4 d0 = momD[2 * (uint64_t)j], d1 = momD[2 * (uint64_t)j + 1];
@@ -540,11 +541,11 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
       add_d(sd, od);
     }
     // centred merge: mean, then parallel-axis terms
-    const float4 c00 = momC[2 * (uint64_t)first];
+    const float4 c00 = recC[4 * (uint64_t)first + 2];
     const float A = sf.a;
     KSum D[3];
     for (uint32_t j = first; j < first + cnt; ++j) {
-      const float4 c0 = momC[2 * (uint64_t)j], c1 = momC[2 * (uint64_t)j + 1];
+      const float4 c0 = recC[4 * (uint64_t)j + 2], c1 = recC[4 * (uint64_t)j + 3];
       const float Aj = __uint_as_float(hdr[j].z);
       D[0].add(Aj * (c0.x - c00.x));
       D[1].add(Aj * (c0.y - c00.y));
@@ -558,7 +559,7 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
     pb[2] = c00.z + D[2].val() / A;
     KSum Ck, Vk;
     for (uint32_t j = first; j < first + cnt; ++j) {
-      const float4 c0 = momC[2 * (uint64_t)j], c1 = momC[2 * (uint64_t)j + 1];
+      const float4 c0 = recC[4 * (uint64_t)j + 2], c1 = recC[4 * (uint64_t)j + 3];
       const float Aj = __uint_as_float(hdr[j].z);
       const float dx = c0.x - pb[0], dy = c0.y - pb[1], dz = c0.z - pb[2];
       Ck.add(c0.w);
@@ -571,10 +572,20 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
   }
   h.z = __float_as_uint(sf.a);
   hdr[k] = h;
-  momP[2 * (uint64_t)k] = make_float4(sf.px, sf.py, sf.pz, sf.pn);
-  momP[2 * (uint64_t)k + 1] = make_float4(sf.nx, sf.ny, sf.nz, sf.pp);
-  momC[2 * (uint64_t)k] = make_float4(pb[0], pb[1], pb[2], Cc);
-  momC[2 * (uint64_t)k + 1] = make_float4(Nk[0].val(), Nk[1].val(), Nk[2].val(), Vc);
+  const float4 g = geo[k];
+  float4* rp = recP + 4 * (uint64_t)k;
+  float4* rc = recC + 4 * (uint64_t)k;
+  rp[0] = g;
+  // the walk's header: a leaf's depth gives way to a flag for a leaf of one point, the father to the
+  // reciprocal of A (rounded as a division for the plain form, the hardware's for the other)
+  const uint32_t code = !hdr_leaf(h.y) ? h.y : kLeafBit | (cnt == 1 ? kSingleBit : 0u) | cnt;
+  reinterpret_cast<uint4*>(rp)[1] = make_uint4(first, code, h.z, __float_as_uint((float)(1.0 / (double)sf.a)));
+  rp[2] = make_float4(sf.px, sf.py, sf.pz, sf.pn);
+  rp[3] = make_float4(sf.nx, sf.ny, sf.nz, sf.pp);
+  rc[0] = g;
+  reinterpret_cast<uint4*>(rc)[1] = make_uint4(first, code, h.z, __float_as_uint(__builtin_amdgcn_rcpf(sf.a)));
+  rc[2] = make_float4(pb[0], pb[1], pb[2], Cc);
+  rc[3] = make_float4(Nk[0].val(), Nk[1].val(), Nk[2].val(), Vc);
   momD[2 * (uint64_t)k] = make_double4(sd.px, sd.py, sd.pz, sd.pn);
   momD[2 * (uint64_t)k + 1] = make_double4(sd.nx, sd.ny, sd.nz, sd.pp);
   AD[k] = sd.a;
@@ -698,7 +709,7 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
   }
   lev.v[kMaxDepth + 1] = (uint32_t)tot;
   t->level_off[kMaxDepth + 1] = (uint32_t)tot;
-  // kernels address node records with 32-bit byte offsets (32-byte moment pairs)
+  // kernels address node headers with 32-bit byte offsets, and a header's count and depth share a word
   if (tot >= (1ull << 27)) return fail(MLOD_ERR_UNSUPPORTED, "octree has 2^27 nodes or more");
   t->nn = (uint32_t)tot;
   const uint32_t nn = t->nn;
@@ -709,7 +720,7 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
       (r = sc.alloc(&areaOrig, n)))
     return r;
   if ((r = dalloc(&t->geo, nn, &t->bytes)) || (r = dalloc(&t->hdr, nn, &t->bytes)) ||
-      (r = dalloc(&t->momP, 2 * (size_t)nn, &t->bytes)) || (r = dalloc(&t->momC, 2 * (size_t)nn, &t->bytes)) ||
+      (r = dalloc(&t->recP, 4 * (size_t)nn, &t->bytes)) || (r = dalloc(&t->recC, 4 * (size_t)nn, &t->bytes)) ||
       (r = dalloc(&t->momD, 2 * (size_t)nn, &t->bytes)) || (r = dalloc(&t->AD, nn, &t->bytes)) ||
       (r = dalloc(&t->box, 6 * (size_t)nn, &t->bytes)) || (r = dalloc(&t->pts, n, &t->bytes)) ||
       (r = dalloc(&t->nrm, n, &t->bytes)) || (r = dalloc(&t->area, n, &t->bytes)) ||
@@ -728,7 +739,7 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
   for (int d = (int)t->depth; d >= 0; --d) {
     const uint32_t beg = lev.v[d], end = lev.v[d + 1];
     if (end <= beg) continue;
-    k_moments<<<(end - beg + BS - 1) / BS, BS, 0, s>>>(beg, end, t->hdr, t->pts, t->nrm, t->momP, t->momC, t->momD, t->AD);
+    k_moments<<<(end - beg + BS - 1) / BS, BS, 0, s>>>(beg, end, t->hdr, t->geo, t->pts, t->nrm, t->recP, t->recC, t->momD, t->AD);
     LAUNCH_CHECK();
   }
   unsigned long long hties = 0;
@@ -742,14 +753,14 @@ int dump_tree(const mlod_tree* t, int32_t* depth, float* bb6, float* center3, fl
               int32_t* first_child, int32_t* next_brother, int32_t* num_children, uint32_t* leaf_count,
               uint32_t* leaf_idx, float* areas, float* moments9) {
   const uint32_t nn = t->nn, n = t->n;
-  std::vector<float4> geo(nn), momP(2 * (size_t)nn);
+  std::vector<float4> geo(nn), recP(moments9 ? 4 * (size_t)nn : 0);
   std::vector<uint4> hdr(nn);
   std::vector<float> box(6 * (size_t)nn);
   std::vector<uint32_t> order(n);
   MLOD_HIP(hipDeviceSynchronize());
   MLOD_HIP(hipMemcpy(geo.data(), t->geo, nn * sizeof(float4), hipMemcpyDeviceToHost));
   MLOD_HIP(hipMemcpy(hdr.data(), t->hdr, nn * sizeof(uint4), hipMemcpyDeviceToHost));
-  MLOD_HIP(hipMemcpy(momP.data(), t->momP, 2 * (size_t)nn * sizeof(float4), hipMemcpyDeviceToHost));
+  if (moments9) MLOD_HIP(hipMemcpy(recP.data(), t->recP, 4 * (size_t)nn * sizeof(float4), hipMemcpyDeviceToHost));
   MLOD_HIP(hipMemcpy(box.data(), t->box, 6 * (size_t)nn * sizeof(float), hipMemcpyDeviceToHost));
   MLOD_HIP(hipMemcpy(order.data(), t->order, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (areas) MLOD_HIP(hipMemcpy(areas, t->area, n * sizeof(float), hipMemcpyDeviceToHost));
@@ -775,7 +786,7 @@ int dump_tree(const mlod_tree* t, int32_t* depth, float* bb6, float* center3, fl
     if (leaf && leaf_idx)
       for (uint32_t j = 0; j < c; ++j) leaf_idx[lo++] = order[h.x + j];
     if (moments9) {
-      const float4 m0 = momP[2 * (size_t)k], m1 = momP[2 * (size_t)k + 1];
+      const float4 m0 = recP[4 * (size_t)k + 2], m1 = recP[4 * (size_t)k + 3];
       float A;
       std::memcpy(&A, &h.z, sizeof(float));
       const float v[9] = {A, m0.x, m0.y, m0.z, m1.x, m1.y, m1.z, m0.w, m1.w};

@@ -8,9 +8,15 @@
 //            first  = first child (internal) or first sorted point (leaf)
 //            count  = #children or #points, bits 27..30 depth, bit 31 leaf
 //            A      = sum of point areas (float bits, reference summation order)
-//     momP float4 x2 {ap, apn}, {an, app}     plain moments (global frame, FP32)
-//     momC float4 x2 {pbar, C}, {N, V}        centred moments: mean point, sum a n,
-//                                              sum a (p - pbar).n, sum a |p - pbar|^2
+//     recP float4 x4 {geo}, {first, code, A, 1/A}, {ap, apn}, {an, app}   the node's 64-byte record
+//                                              for the plain FP32 form: its cell, the walk's
+//                                              header and its plain moments (global frame);
+//                                              code = hdr's word, but a leaf's holds leaf bit,
+//                                              kSingleBit for one point, and #points
+//     recC float4 x4 {geo}, {first, code, A, 1/A}, {pbar, C}, {N, V}      the same for the compensated
+//                                              form: centred moments (mean point, sum a n,
+//                                              sum a (p - pbar).n, sum a |p - pbar|^2)
+//            A walk that needs a whole node takes it in one 64-byte segment.
 //     momD double4 x2 + double                plain moments in FP64
 //   points, in leaf (sorted) order: pts float4 {p, a}, nrm float4 {n, 0}; order maps a
 //   sorted position to the input index.
@@ -27,6 +33,7 @@ namespace mlod {
 
 constexpr int kMaxDepth = 12;          // MAX_DEPTH, sources/apss/CPUUtils.h:20
 constexpr uint32_t kLeafBit = 1u << 31;
+constexpr uint32_t kSingleBit = 1u << 30;  // in a record's code, of a leaf: it holds one point
 constexpr uint32_t kCountMask = (1u << 27) - 1;
 
 __host__ __device__ inline uint32_t hdr_count(uint32_t c) { return c & kCountMask; }
@@ -37,8 +44,8 @@ __host__ __device__ inline bool hdr_leaf(uint32_t c) { return (c & kLeafBit) != 
 struct TreeView {
   const float4* geo;
   const uint4* hdr;
-  const float4* momP;
-  const float4* momC;
+  const float4* recP;
+  const float4* recC;
   const double4* momD;
   const double* AD;
   const float4* pts;
@@ -117,8 +124,8 @@ struct mlod_tree {
   // device buffers
   float4* geo = nullptr;
   uint4* hdr = nullptr;
-  float4* momP = nullptr;
-  float4* momC = nullptr;
+  float4* recP = nullptr;
+  float4* recC = nullptr;
   double4* momD = nullptr;
   double* AD = nullptr;
   float4* pts = nullptr;
@@ -140,7 +147,7 @@ struct mlod_tree {
   float ball_radius = 0.1f;
   mlod::QueryState qs;
   mlod::TreeView view() const {
-    return mlod::TreeView{geo, hdr, momP, momC, momD, AD, pts, nrm, span, n, nn};
+    return mlod::TreeView{geo, hdr, recP, recC, momD, AD, pts, nrm, span, n, nn};
   }
 };
 

@@ -10,10 +10,10 @@
 // is linear in the stats, so it is evaluated top-down: each node carries the product m of
 // the blend factors on its path and adds m * (its own term) to one accumulator.  That needs
 // no per-depth accumulator stack (the reference keeps 12 of them per thread); the per-lane
-// traversal state is, per depth level, the first child, a mask of children still to descend,
-// the node's multiplier and its distance term, held in LDS.  A near node loops over its
-// contiguous children once: far children and leaves are summed right there, the parent's
-// (1 - b_c) share is accumulated, and only near internal children are left in the mask.
+// traversal state is, per depth level, the first child and a mask of children still to descend,
+// held in LDS (the FP64 form keeps the node's multiplier and distance term too).  A near node
+// loops over its contiguous children once: far children and leaves are summed right there, the
+// parent's (1 - b_c) share is accumulated, and only near internal children are left in the mask.
 //
 // Arithmetic forms (template FORM):
 //   0 plain FP32   — global-frame moments and the reference's FP32 sphere fit;
@@ -34,8 +34,7 @@ constexpr int PBS = 128;         // lanes per workgroup
 // Levels of the LDS stack of waiting nodes.  A node waits only while it has more than one near
 // child still to expand, and near children are internal nodes; internal nodes have depth
 // 0..kMaxDepth - 1 and their children depth <= kMaxDepth, so a waiting node has depth at most
-// kMaxDepth - 2 (its near children are internal, hence of depth <= kMaxDepth - 1): 11 levels,
-// 13 B each per lane in the FP32 forms (18.3 KB per workgroup of 128 lanes).
+// kMaxDepth - 2 (its near children are internal, hence of depth <= kMaxDepth - 1): 11 levels.
 constexpr int kLevels = kMaxDepth - 1;
 
 #define LAUNCH_CHECK()                                                           \
@@ -55,42 +54,40 @@ __device__ __forceinline__ float weight32(const KP& k, float d2) {
     if (k.type == MLOD_KERNEL_GAUSSIAN) return weight32<MLOD_KERNEL_GAUSSIAN>(k, d2);
     return weight32<MLOD_KERNEL_SINGULAR>(k, d2);
   } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
-    // sum over s of sigma_s^-3 * 2^(a_s d2), in order of s
+    // sum over s of sigma_s^-3 * 2^(a_s d2), in order of s.  Statically indexed, so the coefficients
+    // sit in scalar registers; two terms between wave-uniform exits (a scalar compare and branch;
+    // the empty asm keeps the compiler from hoisting the compares into lane masks), so that two
+    // exponentials are in flight.  Coefficients past ns are zero: a term past the last adds 0 * 1
     float w = k.b[0] * __builtin_amdgcn_exp2f(d2 * k.a[0]);
-    if (k.ns <= 8) {
-      // statically indexed, so the coefficients sit in scalar registers; the wave-uniform exit
-      // is one scalar compare and branch per term (the empty asm keeps the compiler from
-      // hoisting the compares into lane masks), so no term beyond ns is evaluated
-      int ns = k.ns;
+    w = fmaf(k.b[1], __builtin_amdgcn_exp2f(d2 * k.a[1]), w);
+    int ns = k.ns;
 #pragma unroll
-      for (int s = 1; s < 8; ++s) {
-        asm volatile("" : "+s"(ns));
-        if (s >= ns) break;
-        w = fmaf(k.b[s], __builtin_amdgcn_exp2f(d2 * k.a[s]), w);
-      }
-    } else {
-      // more sigmas (the sample models' settings use up to 30): the first eight from scalar
-      // registers, the rest four at a time, each group's coefficients fetched by two 16-byte
-      // scalar loads (the table is 16-byte aligned) rather than one dependent load per term
-#pragma unroll
-      for (int s = 1; s < 8; ++s) w = fmaf(k.b[s], __builtin_amdgcn_exp2f(d2 * k.a[s]), w);
-      int ns = k.ns;
-      for (int s0 = 8; s0 < ns; s0 += 4) {
-        const float4 A4 = *reinterpret_cast<const float4*>(k.a + s0);
-        const float4 B4 = *reinterpret_cast<const float4*>(k.b + s0);
-        w = fmaf(B4.x, __builtin_amdgcn_exp2f(d2 * A4.x), w);
-        asm volatile("" : "+s"(ns));
-        if (s0 + 1 >= ns) break;
-        w = fmaf(B4.y, __builtin_amdgcn_exp2f(d2 * A4.y), w);
-        asm volatile("" : "+s"(ns));
-        if (s0 + 2 >= ns) break;
-        w = fmaf(B4.z, __builtin_amdgcn_exp2f(d2 * A4.z), w);
-        asm volatile("" : "+s"(ns));
-        if (s0 + 3 >= ns) break;
-        w = fmaf(B4.w, __builtin_amdgcn_exp2f(d2 * A4.w), w);
-      }
+    for (int s = 2; s < 8; s += 2) {
+      asm volatile("" : "+s"(ns));
+      if (s >= ns) break;
+      const float e0 = __builtin_amdgcn_exp2f(d2 * k.a[s]), e1 = __builtin_amdgcn_exp2f(d2 * k.a[s + 1]);
+      w = fmaf(k.b[s], e0, w);
+      w = fmaf(k.b[s + 1], e1, w);
     }
-    return w == 0.f ? k.c : w;  // an all-underflowed sum falls back to constant_shift (Kernel.cpp:69-73)
+    // more sigmas (the sample models' settings use up to 30): four at a time, each group's
+    // coefficients fetched by two 16-byte scalar loads (the table is 16-byte aligned)
+    for (int s0 = 8; s0 < ns; s0 += 4) {
+      const float4 A4 = *reinterpret_cast<const float4*>(k.a + s0);
+      const float4 B4 = *reinterpret_cast<const float4*>(k.b + s0);
+      const float e0 = __builtin_amdgcn_exp2f(d2 * A4.x), e1 = __builtin_amdgcn_exp2f(d2 * A4.y);
+      const float e2 = __builtin_amdgcn_exp2f(d2 * A4.z), e3 = __builtin_amdgcn_exp2f(d2 * A4.w);
+      w = fmaf(B4.x, e0, w);
+      w = fmaf(B4.y, e1, w);
+      w = fmaf(B4.z, e2, w);
+      w = fmaf(B4.w, e3, w);
+    }
+    // an all-underflowed sum falls back to constant_shift (Kernel.cpp:69-73); nothing to do for a zero
+    // one (the empty asm keeps the uniform branch from becoming two selects)
+    if (__float_as_uint(k.c) << 1) {
+      asm volatile("");
+      w = w == 0.f ? k.c : w;
+    }
+    return w;
   } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN) {
     return __builtin_amdgcn_exp2f(d2 * k.a[0]) + k.c;
   } else {
@@ -197,7 +194,7 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
     const float a = P.w;
     const float apx = a * P.x, apy = a * P.y, apz = a * P.z;
     const float dx = apx / a - q.x, dy = apy / a - q.y, dz = apz / a - q.z;
-    const float w = f * weight32<KT>(kp, dx * dx + dy * dy + dz * dz);
+    const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     acc.w = fmaf(w, a, acc.w);
     acc.px = fmaf(w, apx, acc.px);
     acc.py = fmaf(w, apy, acc.py);
@@ -208,17 +205,19 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
     acc.pn = fmaf(w, a * (P.x * N.x + P.y * N.y + P.z * N.z), acc.pn);
     acc.pp = fmaf(w, a * (P.x * P.x + P.y * P.y + P.z * P.z), acc.pp);
   } else if constexpr (FORM == 1) {
+    // the fused operations are written out: every kernel that adds a point rounds alike
     const float dx = P.x - q.x, dy = P.y - q.y, dz = P.z - q.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    const float fa = f * weight32<KT>(kp, d2) * P.w;
-    acc.lw += fa;
+    const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
+    const float fw = __fmul_rn(f, weight32<KT>(kp, d2));
+    const float fa = __fmul_rn(fw, P.w);
+    acc.lw = fmaf(fw, P.w, acc.lw);
     acc.lpx = fmaf(fa, dx, acc.lpx);
     acc.lpy = fmaf(fa, dy, acc.lpy);
     acc.lpz = fmaf(fa, dz, acc.lpz);
     acc.lnx = fmaf(fa, N.x, acc.lnx);
     acc.lny = fmaf(fa, N.y, acc.lny);
     acc.lnz = fmaf(fa, N.z, acc.lnz);
-    acc.lpn = fmaf(fa, dx * N.x + dy * N.y + dz * N.z, acc.lpn);
+    acc.lpn = fmaf(fa, fmaf(dz, N.z, fmaf(dx, N.x, __fmul_rn(dy, N.y))), acc.lpn);
     acc.lpp = fmaf(fa, d2, acc.lpp);
   } else {
     const double a = P.w, x = P.x, y = P.y, z = P.z;
@@ -254,9 +253,9 @@ template <int FORM>
 __device__ __forceinline__ NodeMom<FORM> load_mom(const TreeView& tv, uint32_t c) {
   NodeMom<FORM> r;
   if constexpr (FORM == 0) {
-    r.m0 = ld_rec(tv.momP, 2 * c), r.m1 = ld_rec(tv.momP, 2 * c + 1);
+    r.m0 = tv.recP[4 * (size_t)c + 2], r.m1 = tv.recP[4 * (size_t)c + 3];
   } else if constexpr (FORM == 1) {
-    r.m0 = ld_rec(tv.momC, 2 * c), r.m1 = ld_rec(tv.momC, 2 * c + 1);
+    r.m0 = tv.recC[4 * (size_t)c + 2], r.m1 = tv.recC[4 * (size_t)c + 3];
   } else {
     r.m0 = tv.momD[2 * (size_t)c], r.m1 = tv.momD[2 * (size_t)c + 1];
     r.A = tv.AD[c];
@@ -271,7 +270,7 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
   if constexpr (FORM == 0) {
     const float4 m0 = mm.m0, m1 = mm.m1;
     const float dx = m0.x / Af - q.x, dy = m0.y / Af - q.y, dz = m0.z / Af - q.z;
-    const float w = f * weight32<KT>(kp, dx * dx + dy * dy + dz * dz);
+    const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     acc.w = fmaf(w, Af, acc.w);
     acc.px = fmaf(w, m0.x, acc.px);
     acc.py = fmaf(w, m0.y, acc.py);
@@ -284,18 +283,18 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
   } else if constexpr (FORM == 1) {
     const float4 m0 = mm.m0, m1 = mm.m1;
     const float dx = m0.x - q.x, dy = m0.y - q.y, dz = m0.z - q.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    const float fw = f * weight32<KT>(kp, d2);
-    const float fa = fw * Af;
-    acc.lw += fa;
+    const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
+    const float fw = __fmul_rn(f, weight32<KT>(kp, d2));
+    const float fa = __fmul_rn(fw, Af);
+    acc.lw = fmaf(fw, Af, acc.lw);
     acc.lpx = fmaf(fa, dx, acc.lpx);
     acc.lpy = fmaf(fa, dy, acc.lpy);
     acc.lpz = fmaf(fa, dz, acc.lpz);
     acc.lnx = fmaf(fw, m1.x, acc.lnx);
     acc.lny = fmaf(fw, m1.y, acc.lny);
     acc.lnz = fmaf(fw, m1.z, acc.lnz);
-    acc.lpn = fmaf(fw, m0.w + (dx * m1.x + dy * m1.y + dz * m1.z), acc.lpn);
-    acc.lpp = fmaf(fw, m1.w + Af * d2, acc.lpp);
+    acc.lpn = fmaf(fw, __fadd_rn(m0.w, fmaf(dz, m1.z, fmaf(dx, m1.x, __fmul_rn(dy, m1.y)))), acc.lpn);
+    acc.lpp = fmaf(fw, fmaf(Af, d2, m1.w), acc.lpp);
   } else {
     const double4 m0 = mm.m0, m1 = mm.m1;
     const double A = mm.A;
@@ -345,9 +344,10 @@ __device__ __forceinline__ T dist3(V3<T> q, float4 g) {
 // compensated sums, takes the hardware reciprocal and square root (1 ulp).
 template <int FORM>
 __device__ __forceinline__ typename FormT<FORM>::T tdist(V3<typename FormT<FORM>::T> q, float4 g) {
-  if constexpr (FORM == 1) {
+  if constexpr (FORM != 2) {  // (the fused operations written out: every kernel rounds alike)
     const float dx = q.x - g.x, dy = q.y - g.y, dz = q.z - g.z;
-    return __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
+    const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
+    return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : fsqrt(d2);
   } else {
     return dist3(q, g);
   }
@@ -370,7 +370,7 @@ struct LevelState {
   T (*dist)[PBS];          // its distance term |d - cutoff r| (negative: no blending below it)
 };
 
-// Flattened traversal.  The lane's current node (expanded: near, or above minDepth) has its
+// Flattened traversal (the FP64 form's; traverse_staged is the FP32 forms').  The lane's current node (expanded: near, or above minDepth) has its
 // children tested one per loop iteration; when they are done the node's own (1 - b_c) share
 // is added and its first near child becomes the current node.  Either way an iteration handles
 // exactly one node X: it loads X, computes its distance and its blend factor against its
@@ -538,27 +538,242 @@ struct Walker {
   }
 };
 
-// The whole walk of one query step on one lane.
+// The whole walk of one query step on one lane (FP64 form).
+template <int FORM, int SEM, int KT, bool CNT, class KP>
+__device__ __forceinline__ void traverse_loads(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
+                                               V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T cutoff,
+                                               uint32_t minDepth, LevelState<typename FormT<FORM>::T> st, int tid,
+                                               Counters& ct) {
+  Walker<FORM, SEM, KT, CNT, KP> w;
+  w.begin(acc, kp, tv, q, cutoff, minDepth, ct);
+  while (w.active) w.iter(acc, kp, tv, q, cutoff, minDepth, st, tid, ct);
+}
+
+// ----------------------------------------------------------------------------- staged walk (FP32 forms)
+// The same walk, one node per lane and iteration, with the node's 64-byte record (cell, header,
+// moments: recP / recC) brought in by the four lanes of a quad together.  A lane that gathers its own
+// record takes four 16-byte loads, and each of those costs the L1 cache one access per distinct
+// segment of a quad: 41 accesses per load instruction of 64 lanes, 164 an iteration, one access every
+// cycle of the launch (8M points and queries, FP32C).  Here load j brings the record of lane j of
+// every quad, its four lanes fetching the 16-byte pieces of one segment: 16 accesses, 64 an
+// iteration.  The loads go straight to LDS (load j to row j, 64 lanes x 16 B), from where each lane
+// reads its own record back; a row is one 16-byte bank group longer than its data, which spreads those
+// reads over all banks.  With the L1 out of the way the walk is bound by vector instructions (VALU
+// 100 % busy, 131 an iteration against 152 before: no multiplier, reciprocals of A kept in the
+// records, one stack access an iteration), and the smaller stacks let five waves run per SIMD against
+// four.  8M points, 8M queries, six sigmas, FP32C: 20.6 -> 16.5 ms a step; 1M points and queries,
+// rational kernel, plain FP32: 11.7 -> 10.0; 100k queries x 10 steps on 1M points: 5.5 -> 4.8.
+// (Four waves per SIMD, with the stacks one word a level longer, left the step at 20.6 ms.)
+constexpr uint32_t kStageRow = 1024 + 16;
+constexpr uint32_t kStageBytes = 4 * kStageRow;  // per wavefront
+
+template <int J>
+__device__ __forceinline__ uint32_t quad_lane(uint32_t v) {  // lane J of this lane's quad
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, J * 0x55, 0xf, 0xf, true);
+}
+typedef const __attribute__((address_space(1))) void* GlobalPtr;
+typedef __attribute__((address_space(3))) void* LdsPtr;
+
+// BIG: 2^26 nodes or more, whose byte offsets need more than 32 bits
+template <int J, bool BIG>
+__device__ __forceinline__ void stage_row(const char* rec, uint32_t idx, uint32_t lane, unsigned char* stage) {
+  const uint32_t piece = (lane & 3u) * 16u;
+  const char* src = BIG ? rec + piece + (uint64_t)quad_lane<J>(idx) * 64u : rec + (quad_lane<J>(idx << 6) + piece);
+  __builtin_amdgcn_global_load_lds((GlobalPtr)src, (LdsPtr)(stage + J * kStageRow), 16, 0, 0);
+}
+// Starts the loads of record `idx` of every lane (all 64 lanes take part).
+template <bool BIG>
+__device__ __forceinline__ void stage_issue(const float4* rec, uint32_t idx, uint32_t lane, unsigned char* stage) {
+  const char* r = reinterpret_cast<const char*>(rec);
+  stage_row<0, BIG>(r, idx, lane, stage);
+  stage_row<1, BIG>(r, idx, lane, stage);
+  stage_row<2, BIG>(r, idx, lane, stage);
+  stage_row<3, BIG>(r, idx, lane, stage);
+}
+
+// A node with near children still to expand, per level and lane: its first child, and those children.
+struct StagedStack {
+  uint32_t (*first)[PBS];
+  uint8_t (*mask)[PBS];
+};
+
+// Half a distance term that makes every blend factor 1 (a node above minDepth: no blending below it):
+// kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit.
+constexpr float kNoBlend = 1e30f;
+
+// Cell and header of record idx.
+typedef float Quad __attribute__((ext_vector_type(4)));
+template <bool BIG>
+__device__ __forceinline__ void load_head(const float4* rec, uint32_t idx, Quad& g, Quad& h) {
+  const char* r = reinterpret_cast<const char*>(rec);
+  const char* src = BIG ? r + (uint64_t)idx * 64u : r + (idx << 6);
+  g = *reinterpret_cast<const Quad*>(src);
+  h = *reinterpret_cast<const Quad*>(src + 16);
+  asm volatile("" : "+v"(g), "+v"(h));  // both loads are issued before either is waited for
+}
+__device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
+
+// What the walk relies on.  A near child's blend factor is exactly 1 (its distance is within its
+// cutoff, so t = dP / (dP + 0), at most one rounding off 1, and the hardware cosine at half a
+// revolution, and one float to either side of it, is exactly -1): the product of the factors on
+// the path to any expanded node is 1 and is not kept.  Terms are added in the order of the walk (a node's
+// children in slot order, then its own (1 - b_c) share, then its first near child), and the
+// compensated form's block flushes come every kFlush iterations of the loop, which all lanes start
+// together, so a lane's sums depend on its own query only.
+template <int FORM, int SEM, int KT, bool CNT, bool BIG, class KP>
+__device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
+                                                V3<float> q, float cutoff, uint32_t minDepth, bool live,
+                                                StagedStack st, unsigned char* stage, int tid, Counters& ct) {
+#pragma clang fp contract(off)  // the fused operations are written out
+  const uint32_t lane = __lane_id();
+  const float4* __restrict__ rec = FORM == 0 ? tv.recP : tv.recC;
+  const uint4 h0 = tv.hdr[0];
+  if (hdr_leaf(h0.y)) {  // a one-leaf tree (uniform)
+    if (live) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h0, q, 1.f, ct);
+    if constexpr (FORM == 1) acc.flush();
+    return;
+  }
+  const int32_t blendKey = (int32_t)(min(minDepth, 15u) << 27);  // headers of internal nodes at or below minDepth
+  const float4 g0 = tv.geo[0];
+  uint32_t active = live ? 1u : 0u;  // (a word: one compare makes the wavefront's mask of it)
+  float dh = kNoBlend;  // half the current node's distance term
+  if (minDepth == 0) {
+    const float d0 = tdist<FORM>(q, g0), rc = g0.w * cutoff;
+    dh = 0.5f * fabsf(d0 - rc);
+    if (d0 > rc) {
+      if (live) {
+        add_node<FORM, KT>(acc, kp, tv, 0, __uint_as_float(h0.z), q, 1.f);
+        if constexpr (CNT) ct.far_ += 1;
+      }
+      active = 0u;
+    }
+  }
+  // the current node: its children [first, xEnd), the next one to test, the near ones found
+  uint32_t node = 0, first = h0.x, x = first, xEnd = active ? first + hdr_count(h0.y) : first, mask = 0, pend = 0;
+  int lvl = 0;
+  float Ai = __uint_as_float(h0.z), shareSum = 0.f;
+  float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)hdr_count(h0.y)) : rec[1].w;
+  const unsigned char* mine = stage + (lane & 3u) * kStageRow + (lane >> 2) * 64u;
+  while (any_lane(active != 0u)) {
+#pragma unroll 1
+    for (uint32_t b = 0; b < kFlush && any_lane(active != 0u); ++b) {
+      if constexpr (CNT) ct.iters += active ? 1u : 0u;
+      const bool testing = x < xEnd;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last record has been read
+      stage_issue<BIG>(rec, testing ? x : node, lane, stage);
+      bool contrib = false;
+      float f = 0.f;
+      if (active && !testing) {
+        // the node is finished: its own share is added, and the next near node becomes current: the
+        // first waiting child of the deepest node that has some
+        f = shareSum;
+        contrib = f != 0.f;
+        if constexpr (CNT) ct.nearN += contrib ? 1u : 0u;
+        if (mask) {
+          st.first[lvl][tid] = first;
+          st.mask[lvl][tid] = (uint8_t)mask;
+          pend |= 1u << lvl;
+        }
+        if (pend) {
+          const uint32_t L = 31u - (uint32_t)__builtin_clz(pend);
+          const uint32_t bits = st.mask[L][tid], from = st.first[L][tid];
+          const uint32_t rest = bits & (bits - 1u);
+          st.mask[L][tid] = (uint8_t)rest;
+          if (!rest) pend ^= 1u << L;
+          lvl = (int)L + 1;
+          node = from + (uint32_t)__builtin_ctz(bits);
+          Quad gx, hx;
+          load_head<BIG>(rec, node, gx, hx);
+          const uint32_t code = __float_as_uint(hx.y);
+          dh = 0.5f * fabsf(tdist<FORM>(q, make_float4(gx.x, gx.y, gx.z, gx.w)) - gx.w * cutoff);
+          if (blendKey) {
+            asm volatile("");  // (a uniform branch, not a select)
+            dh = (int32_t)code >= blendKey ? dh : kNoBlend;
+          }
+          first = x = __float_as_uint(hx.x);
+          xEnd = first + (code & 15u);  // an internal node has at most 8 children
+          Ai = hx.z;
+          scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)(code & 15u)) : hx.w;
+        } else {
+          active = 0u;
+          node = 0u;
+        }
+        mask = 0u;
+        shareSum = 0.f;
+      }
+      // the record: every load is back before it is read, and read before the next iteration's loads
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const float4 g = *reinterpret_cast<const float4*>(mine);
+      const uint4 h = *reinterpret_cast<const uint4*>(mine + 16);
+      NodeMom<FORM> mm;
+      mm.m0 = *reinterpret_cast<const float4*>(mine + 32);
+      mm.m1 = *reinterpret_cast<const float4*>(mine + 48);
+      const float At = __uint_as_float(h.z);
+      bool multi = false;
+      if (testing) {
+        // X's blend factor against its parent (CPUUtils.cpp:489-497); far: beyond its cutoff
+        const float over = tdist<FORM>(q, g) - g.w * cutoff;
+        const float dc = fmaxf(over, 0.f);
+        f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
+        const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : At / Ai);
+        shareSum = fmaf(share, 1.f - f, shareSum);
+        const bool leaf = (int32_t)h.y < 0;
+        const bool single = h.y >= (kLeafBit | kSingleBit);
+        const bool far = (int32_t)h.y >= blendKey && over > 0.f;
+        mask |= (leaf || far ? 0u : 1u) << (x - first);
+        multi = leaf && !single;
+        if constexpr (CNT) {
+          ct.tested += 1;
+          ct.far_ += far ? 1u : 0u;
+          ct.leafPts += single ? 1u : 0u;
+        }
+        ++x;
+        contrib = far || single;
+      }
+      if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
+      if (any_lane(multi)) {  // a leaf of several points (at the last level, or by the build's option)
+        if (multi) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);
+      }
+    }
+    if constexpr (FORM == 1) acc.flush();
+  }
+  if constexpr (FORM == 1) acc.flush();
+}
+
+// The LDS of one workgroup's walks: the stacks of waiting nodes (5 B a level and lane in the FP32
+// forms) and the wavefronts' staging rows (15.4 KB: ten workgroups a CU, five waves per SIMD), or the
+// FP64 form's stacks.
+template <int FORM>
+struct WalkLds {
+  uint32_t first[kLevels][PBS];
+  uint8_t mask[kLevels][PBS];
+  alignas(16) unsigned char stage[PBS / 64][kStageBytes];
+};
+template <>
+struct WalkLds<2> {
+  double mul[kLevels][PBS];
+  double dist[kLevels][PBS];
+  uint32_t first[kLevels][PBS];
+  uint8_t mask[kLevels][PBS];
+};
+
+// One walk of each live lane of the wavefront (every lane calls it).
 template <int FORM, int SEM, int KT, bool CNT, class KP>
 __device__ __forceinline__ void traverse(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
                                          V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T cutoff,
-                                         uint32_t minDepth, LevelState<typename FormT<FORM>::T> st, int tid,
-                                         Counters& ct) {
-  Walker<FORM, SEM, KT, CNT, KP> w;
-  w.begin(acc, kp, tv, q, cutoff, minDepth, ct);
-  // the lanes of a wavefront start together and advance one iteration per loop, so the
-  // compensated form's block flushes fall on the same loop iterations for all of them
-  uint32_t itc = 0;
-  while (w.active) {
-    w.iter(acc, kp, tv, q, cutoff, minDepth, st, tid, ct);
-    if constexpr (FORM == 1) {
-      if (++itc == kFlush) {
-        acc.flush();
-        itc = 0;
-      }
-    }
+                                         uint32_t minDepth, bool live, WalkLds<FORM>& lds, int tid, Counters& ct) {
+  if constexpr (FORM == 2) {
+    if (live)
+      traverse_loads<FORM, SEM, KT, CNT>(acc, kp, tv, q, cutoff, minDepth,
+                                         LevelState<double>{lds.first, lds.mask, lds.mul, lds.dist}, tid, ct);
+  } else {
+    const StagedStack st{lds.first, lds.mask};
+    unsigned char* stage = lds.stage[__builtin_amdgcn_readfirstlane(tid >> 6)];
+    if (tv.nn < (1u << 26))
+      traverse_staged<FORM, SEM, KT, CNT, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
+    else
+      traverse_staged<FORM, SEM, KT, CNT, true>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
   }
-  if constexpr (FORM == 1) acc.flush();
 }
 
 // ----------------------------------------------------------------------------- wave-shared walk
@@ -602,9 +817,9 @@ template <int FORM>
 __device__ __forceinline__ NodeMom<FORM> load_mom_uni(const TreeView& tv, uint32_t c) {
   NodeMom<FORM> r;
   if constexpr (FORM == 0) {
-    r.m0 = ld_uni(tv.momP, 2 * c), r.m1 = ld_uni(tv.momP, 2 * c + 1);
+    r.m0 = ld_uni(tv.recP, 4 * c + 2), r.m1 = ld_uni(tv.recP, 4 * c + 3);
   } else if constexpr (FORM == 1) {
-    r.m0 = ld_uni(tv.momC, 2 * c), r.m1 = ld_uni(tv.momC, 2 * c + 1);
+    r.m0 = ld_uni(tv.recC, 4 * c + 2), r.m1 = ld_uni(tv.recC, 4 * c + 3);
   } else {
     r.m0 = ld_uni(tv.momD, 2 * c), r.m1 = ld_uni(tv.momD, 2 * c + 1);
     r.A = ld_uni(tv.AD, c);
@@ -901,17 +1116,13 @@ __global__ __launch_bounds__(PBS) void k_project(TreeView tv, KParams kp, float4
                                                  uint32_t nIter, float stepMax, float cutoff, uint32_t minDepth,
                                                  unsigned long long* __restrict__ counters) {
   using T = typename FormT<FORM>::T;
-  __shared__ uint32_t sFirst[kLevels][PBS];
-  __shared__ uint8_t sMask[kLevels][PBS];
-  __shared__ T sMul[kLevels][PBS];
-  __shared__ T sDist[kLevels][PBS];
+  __shared__ WalkLds<FORM> lds;
   const int tid = threadIdx.x;
   const uint32_t i = xcd_block() * PBS + tid;
   const bool live = i < m && !(limit < m && perm[i] >= limit);
   Counters ct{0, 0, 0, 0, 0};
-  if (live) {
-    const LevelState<T> st{sFirst, sMask, sMul, sDist};
-    const float4 q4 = q[i];
+  if (__any(live)) {  // uniform over a wavefront: its lanes load node records together
+    const float4 q4 = live ? q[i] : make_float4(0.f, 0.f, 0.f, 0.f);
     V3<double> qd{q4.x, q4.y, q4.z};
     float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
     for (uint32_t it = 0; it < nIter; ++it) {
@@ -923,11 +1134,13 @@ __global__ __launch_bounds__(PBS) void k_project(TreeView tv, KParams kp, float4
         qt = V3<T>{qd.x, qd.y, qd.z};
       else
         qt = V3<T>{qf.x, qf.y, qf.z};
-      traverse<FORM, SEM, KT, CNT>(acc, kp, tv, qt, (T)cutoff, minDepth, st, tid, ct);
+      traverse<FORM, SEM, KT, CNT>(acc, kp, tv, qt, (T)cutoff, minDepth, live, lds, tid, ct);
       fit_step<FORM, SEM>(acc, qd, qf, stepMax, nout);
     }
-    q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
-    qn[i] = nout;
+    if (live) {
+      q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
+      qn[i] = nout;
+    }
   }
   if constexpr (CNT) {
     // lane slots: 64 x the longest loop of the wavefront (lanes wait for it)
@@ -1064,10 +1277,7 @@ __global__ __launch_bounds__(PBS) void k_project_batch(const ReqDesc* __restrict
                                                        double4* __restrict__ qdp, BatchOut bo, uint32_t prio) {
   static_assert(PBS == kBatchWG, "one workgroup per pool block");
   using T = typename FormT<FORM>::T;
-  __shared__ uint32_t sFirst[kLevels][PBS];
-  __shared__ uint8_t sMask[kLevels][PBS];
-  __shared__ T sMul[kLevels][PBS];
-  __shared__ T sDist[kLevels][PBS];
+  __shared__ WalkLds<FORM> lds;
   if (prio) __builtin_amdgcn_s_setprio(3);
   const int tid = threadIdx.x;
   const uint32_t lb = xcd_block();
@@ -1075,21 +1285,23 @@ __global__ __launch_bounds__(PBS) void k_project_batch(const ReqDesc* __restrict
   const uint32_t r = __builtin_amdgcn_readfirstlane(b.x), pb = __builtin_amdgcn_readfirstlane(b.y);
   const ReqDesc& R = reqs[r];
   const uint32_t i = pb * PBS + tid, outOff = R.outOff;
-  if (i < R.pad0 + R.count) {
+  const bool live = i < R.pad0 + R.count;
+  V3<double> qd{0, 0, 0};
+  float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (__any(live)) {  // uniform over a wavefront: its lanes load node records together
     const TreeView tv = R.tv;
     const KParams& kp = R.kp;
     const float cutoff = R.cutoff, stepMax = R.stepMax;
     const uint32_t minDepth = R.minDepth, nIter = R.nIter;
-    const LevelState<T> st{sFirst, sMask, sMul, sDist};
-    V3<double> qd;
-    if constexpr (FORM == 2) {
-      const double4 d4 = qdp[i];
-      qd = V3<double>{d4.x, d4.y, d4.z};
-    } else {
-      const float4 q4 = q[i];
-      qd = V3<double>{q4.x, q4.y, q4.z};
+    if (live) {
+      if constexpr (FORM == 2) {
+        const double4 d4 = qdp[i];
+        qd = V3<double>{d4.x, d4.y, d4.z};
+      } else {
+        const float4 q4 = q[i];
+        qd = V3<double>{q4.x, q4.y, q4.z};
+      }
     }
-    float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
     Counters ct{0, 0, 0, 0, 0};
     for (uint32_t it = 0; it < nIter; ++it) {
       typename FormT<FORM>::Acc acc;
@@ -1100,9 +1312,11 @@ __global__ __launch_bounds__(PBS) void k_project_batch(const ReqDesc* __restrict
         qt = V3<T>{qd.x, qd.y, qd.z};
       else
         qt = V3<T>{qf.x, qf.y, qf.z};
-      traverse<FORM, SEM, KT, false>(acc, kp, tv, qt, (T)cutoff, minDepth, st, tid, ct);
+      traverse<FORM, SEM, KT, false>(acc, kp, tv, qt, (T)cutoff, minDepth, live, lds, tid, ct);
       fit_step<FORM, SEM>(acc, qd, qf, stepMax, nout);
     }
+  }
+  if (live) {
     const float4 p4 = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
     q[i] = p4;
     qn[i] = nout;
