@@ -23,7 +23,7 @@ ARCH = os.environ.get("MLOD_ARCH", "gfx950")
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-Wno-unused-result"]
 SOURCES = ["build.hip", "project.hip", "queries.hip", "neighbors.hip", "serve.hip", "adaptive.hip", "dc.hip", "noalloc.hip",
-           "api.cpp"]
+           "api.cpp", "pool.cpp"]
 # The octree build reproduces the reference's float arithmetic (cell boxes, radii, areas,
 # plain moments) bit for bit, and the neighbour search the kd-tree's float distances, so no
 # multiply-add may be fused there.

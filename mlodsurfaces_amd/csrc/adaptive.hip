@@ -223,7 +223,7 @@ struct KeyVec {
   uint64_t* p = nullptr;
   size_t n = 0, cap = 0;
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) dev_free(p);
     p = nullptr;
     n = cap = 0;
   }
@@ -232,11 +232,11 @@ struct KeyVec {
     if (m <= cap) return MLOD_OK;
     const size_t nc = std::max(m, cap + cap / 2);
     uint64_t* q = nullptr;
-    if (hipMalloc((void**)&q, nc * sizeof(uint64_t)) != hipSuccess)
+    if (dev_malloc(&q, nc * sizeof(uint64_t)) != hipSuccess)
       return fail(MLOD_ERR_OOM, "adaptive octree: hipMalloc failed for " + std::to_string(nc) + " cells");
     if (keep) MLOD_HIP(hipMemcpyAsync(q, p, keep * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
     MLOD_HIP(hipStreamSynchronize(s));
-    if (p) (void)hipFree(p);
+    if (p) dev_free(p);
     p = q;
     cap = nc;
     return MLOD_OK;
@@ -284,10 +284,10 @@ int ensure_sort_tmp(mlod_generator* g, size_t n, hipStream_t s) {
   need = std::max(need, need2);
   if (need <= g->sortBytes) return MLOD_OK;
   MLOD_HIP(hipStreamSynchronize(s));
-  if (g->sortTmp) (void)hipFree(g->sortTmp);
+  if (g->sortTmp) dev_free(g->sortTmp);
   g->sortTmp = nullptr;
   g->sortBytes = 0;
-  if (hipMalloc(&g->sortTmp, need + 256) != hipSuccess) return fail(MLOD_ERR_OOM, "adaptive octree: sort buffer");
+  if (dev_malloc(&g->sortTmp, need + 256) != hipSuccess) return fail(MLOD_ERR_OOM, "adaptive octree: sort buffer");
   g->sortBytes = need;
   return MLOD_OK;
 }
@@ -355,10 +355,10 @@ int find_stable(mlod_generator* g, KeyVec& cur, KeyVec& sub, KeyVec& scratch, hi
     return MLOD_OK;
   }
   if (n > g->stageCap) {
-    if (g->dStage) (void)hipFree(g->dStage);
+    if (g->dStage) dev_free(g->dStage);
     g->dStage = nullptr;
     g->stageCap = 0;
-    if (hipMalloc((void**)&g->dStage, n * 3 * sizeof(float)) != hipSuccess)
+    if (dev_malloc(&g->dStage, n * 3 * sizeof(float)) != hipSuccess)
       return fail(MLOD_ERR_OOM, "adaptive octree: centre buffer");
     g->stageCap = n;
   }
@@ -482,10 +482,10 @@ int generate(mlod_generator* g, uint32_t maxDepth, hipStream_t s) {
 int leaf_centres(mlod_generator* g, hipStream_t s) {
   const size_t n = g->leaves.n;
   if (n > g->xyzCap) {
-    if (g->dXyz) (void)hipFree(g->dXyz);
+    if (g->dXyz) dev_free(g->dXyz);
     g->dXyz = nullptr;
     g->xyzCap = 0;
-    if (hipMalloc((void**)&g->dXyz, std::max<size_t>(n, 1) * 3 * sizeof(float)) != hipSuccess)
+    if (dev_malloc(&g->dXyz, std::max<size_t>(n, 1) * 3 * sizeof(float)) != hipSuccess)
       return fail(MLOD_ERR_OOM, "adaptive octree: leaf centre buffer");
     g->xyzCap = n;
   }
@@ -510,9 +510,9 @@ int mlod_generator_create(mlod_tree* t, mlod_generator** out) {
   *out = nullptr;
   mlod_generator* g = new mlod_generator();
   g->tree = t;
-  if (hipMalloc((void**)&g->dCount, sizeof(uint64_t)) != hipSuccess ||
-      hipMalloc((void**)&g->dFlags, sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc((void**)&g->dNonfinite, sizeof(unsigned long long)) != hipSuccess) {
+  if (dev_malloc(&g->dCount, sizeof(uint64_t)) != hipSuccess ||
+      dev_malloc(&g->dFlags, sizeof(uint32_t)) != hipSuccess ||
+      dev_malloc(&g->dNonfinite, sizeof(unsigned long long)) != hipSuccess) {
     mlod_generator_destroy(g);
     return fail(MLOD_ERR_OOM, "generator: hipMalloc failed");
   }
@@ -525,8 +525,7 @@ int mlod_generator_destroy(mlod_generator* g) {
   (void)hipDeviceSynchronize();
   g->leaves.release(), g->total.release(), g->a.release(), g->b.release(), g->c.release();
   void* p[] = {g->sortTmp, g->dCount, g->dFlags, g->dNonfinite, g->dXyz, g->dStage};
-  for (void* q : p)
-    if (q) (void)hipFree(q);
+  dev_free(p, sizeof(p) / sizeof(p[0]));
   delete g;
   return MLOD_OK;
 }
@@ -561,10 +560,10 @@ int mlod_generate_from_points(mlod_generator* g, const float* xyz, uint32_t n, i
   const float* src = xyz;
   if (!device_src) {
     if (n > g->stageCap) {
-      if (g->dStage) (void)hipFree(g->dStage);
+      if (g->dStage) dev_free(g->dStage);
       g->dStage = nullptr;
       g->stageCap = 0;
-      if (hipMalloc((void**)&g->dStage, (size_t)n * 3 * sizeof(float)) != hipSuccess)
+      if (dev_malloc(&g->dStage, (size_t)n * 3 * sizeof(float)) != hipSuccess)
         return fail(MLOD_ERR_OOM, "generator: point buffer");
       g->stageCap = n;
     }
@@ -597,12 +596,12 @@ int mlod_generator_cells(mlod_generator* g, int32_t which, int32_t* out_ids4, vo
   if (!v.n) return MLOD_OK;
   hipStream_t s = (hipStream_t)stream;
   int32_t* d = nullptr;
-  if (hipMalloc((void**)&d, v.n * 4 * sizeof(int32_t)) != hipSuccess) return fail(MLOD_ERR_OOM, "cell download buffer");
+  if (dev_malloc(&d, v.n * 4 * sizeof(int32_t)) != hipSuccess) return fail(MLOD_ERR_OOM, "cell download buffer");
   k_decode<<<blocks(v.n), BS, 0, s>>>(v.p, (uint32_t)v.n, d);
   hipError_t e = hipGetLastError();
   if (!e) e = hipMemcpyAsync(out_ids4, d, v.n * 4 * sizeof(int32_t), hipMemcpyDeviceToHost, s);
   if (!e) e = hipStreamSynchronize(s);
-  (void)hipFree(d);
+  dev_free(d);
   if (e) return hip_fail(e, "generator cells", __FILE__, __LINE__);
   return MLOD_OK;
 }

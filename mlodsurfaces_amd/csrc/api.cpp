@@ -30,8 +30,7 @@ static void free_tree(mlod_tree* t) {
   if (!t) return;
   queries_free(t);
   void* bufs[] = {t->geo, t->hdr, t->recP, t->recC, t->momD, t->AD, t->pts, t->nrm, t->order, t->box, t->area, t->span};
-  for (void* p : bufs)
-    if (p) (void)hipFree(p);
+  dev_free(bufs, sizeof(bufs) / sizeof(bufs[0]));
   delete t;
 }
 
@@ -108,8 +107,8 @@ int mlod_tree_create(const float* xyz, const float* nrm, uint32_t n, const mlod_
   if (!xyz || !nrm) return fail(MLOD_ERR_INVALID, "points or normals are NULL");
   float *dx = nullptr, *dn = nullptr;
   const size_t b = (size_t)n * 3 * sizeof(float);
-  if (hipMalloc((void**)&dx, b) != hipSuccess || hipMalloc((void**)&dn, b) != hipSuccess) {
-    (void)hipFree(dx), (void)hipFree(dn);
+  if (dev_malloc(&dx, b) != hipSuccess || dev_malloc(&dn, b) != hipSuccess) {
+    dev_free(dx), dev_free(dn);
     return fail(MLOD_ERR_OOM, "input staging: hipMalloc failed");
   }
   hipStream_t s = (hipStream_t)stream;
@@ -117,7 +116,7 @@ int mlod_tree_create(const float* xyz, const float* nrm, uint32_t n, const mlod_
   if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, b, hipMemcpyHostToDevice, s);
   int r = e == hipSuccess ? mlod_tree_create_device(dx, dn, n, opts, stream, out) : hip_fail(e, "input upload", __FILE__, __LINE__);
   (void)hipStreamSynchronize(s);
-  (void)hipFree(dx), (void)hipFree(dn);
+  dev_free(dx), dev_free(dn);
   return r;
 }
 
@@ -284,10 +283,9 @@ int mlod_count_visits(mlod_tree* t, uint32_t n, uint64_t* out6, void* stream) {
   const size_t cbytes = 6 * sizeof(unsigned long long);
   float4 *bq = nullptr, *bn = nullptr;
   unsigned long long* dc = nullptr;
-  if (hipMalloc((void**)&bq, (size_t)m * sizeof(float4) + 16) != hipSuccess ||
-      hipMalloc((void**)&bn, (size_t)m * sizeof(float4) + 16) != hipSuccess ||
-      hipMalloc((void**)&dc, cbytes) != hipSuccess) {
-    (void)hipFree(bq), (void)hipFree(bn), (void)hipFree(dc);
+  if (dev_malloc(&bq, (size_t)m * sizeof(float4) + 16) != hipSuccess ||
+      dev_malloc(&bn, (size_t)m * sizeof(float4) + 16) != hipSuccess || dev_malloc(&dc, cbytes) != hipSuccess) {
+    dev_free(bq), dev_free(bn), dev_free(dc);
     return fail(MLOD_ERR_OOM, "counter pass buffers");
   }
   hipError_t e = hipMemcpyAsync(bq, t->qs.q, (size_t)m * sizeof(float4), hipMemcpyDeviceToDevice, s);
@@ -302,7 +300,7 @@ int mlod_count_visits(mlod_tree* t, uint32_t n, uint64_t* out6, void* stream) {
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) r = hip_fail(e, "counter pass", __FILE__, __LINE__);
   }
-  (void)hipFree(bq), (void)hipFree(bn), (void)hipFree(dc);
+  dev_free(bq), dev_free(bn), dev_free(dc);
   const uint64_t laneSlots = 64ull * h[5];
   for (int k = 0; k < 5; ++k) out6[k] = h[k];
   out6[5] = laneSlots;

@@ -594,7 +594,7 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
 template <class T>
 int dalloc(T** p, size_t count, uint64_t* bytes) {
   const size_t b = std::max<size_t>(count, 1) * sizeof(T);
-  hipError_t e = hipMalloc((void**)p, b);
+  hipError_t e = dev_malloc(p, b);
   if (e != hipSuccess) return fail(MLOD_ERR_OOM, "hipMalloc of " + std::to_string(b) + " bytes failed");
   if (bytes) *bytes += b;
   return MLOD_OK;
@@ -603,7 +603,7 @@ int dalloc(T** p, size_t count, uint64_t* bytes) {
 struct Scratch {
   std::vector<void*> ptrs;
   ~Scratch() {
-    for (void* p : ptrs) (void)hipFree(p);
+    dev_free(ptrs.data(), ptrs.size());
   }
   template <class T>
   int alloc(T** p, size_t count) {

@@ -485,7 +485,7 @@ struct DVec {
   T* p = nullptr;
   size_t n = 0, cap = 0;
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) dev_free(p);
     p = nullptr;
     n = cap = 0;
   }
@@ -493,11 +493,11 @@ struct DVec {
     if (m <= cap) return MLOD_OK;
     const size_t nc = std::max(m, cap + cap / 2);
     T* q = nullptr;
-    if (hipMalloc((void**)&q, std::max<size_t>(nc, 1) * sizeof(T)) != hipSuccess)
+    if (dev_malloc(&q, std::max<size_t>(nc, 1) * sizeof(T)) != hipSuccess)
       return fail(MLOD_ERR_OOM, "dual contouring: hipMalloc failed for " + std::to_string(nc) + " elements");
     if (keep) MLOD_HIP(hipMemcpyAsync(q, p, keep * sizeof(T), hipMemcpyDeviceToDevice, s));
     MLOD_HIP(hipStreamSynchronize(s));
-    if (p) (void)hipFree(p);
+    if (p) dev_free(p);
     p = q;
     cap = nc;
     return MLOD_OK;
@@ -533,10 +533,10 @@ namespace {
 int ensure_tmp(mlod_dc* dc, size_t need) {
   if (need <= dc->tmpBytes) return MLOD_OK;
   (void)hipDeviceSynchronize();
-  if (dc->tmp) (void)hipFree(dc->tmp);
+  if (dc->tmp) dev_free(dc->tmp);
   dc->tmp = nullptr;
   dc->tmpBytes = 0;
-  if (hipMalloc(&dc->tmp, need + 256) != hipSuccess) return fail(MLOD_ERR_OOM, "dual contouring: temporary storage");
+  if (dev_malloc(&dc->tmp, need + 256) != hipSuccess) return fail(MLOD_ERR_OOM, "dual contouring: temporary storage");
   dc->tmpBytes = need;
   return MLOD_OK;
 }
@@ -636,7 +636,7 @@ int build(mlod_dc* dc, const int32_t* ids4, uint32_t n, uint32_t maxDepth, bool 
   MLOD_HIP(hipMemsetAsync(dc->dFlags, 0, sizeof(uint32_t), s));
   if (int r = dc->keys.reserve(2 * (size_t)n + 1, 0, s)) return r;
   int32_t* dIds = nullptr;
-  if (hipMalloc((void**)&dIds, std::max<size_t>(n, 1) * 4 * sizeof(int32_t)) != hipSuccess)
+  if (dev_malloc(&dIds, std::max<size_t>(n, 1) * 4 * sizeof(int32_t)) != hipSuccess)
     return fail(MLOD_ERR_OOM, "dual contouring: cells");
   hipError_t e = hipMemcpyAsync(dIds, ids4, (size_t)n * 4 * sizeof(int32_t), hipMemcpyHostToDevice, s);
   if (!e && n) {
@@ -644,7 +644,7 @@ int build(mlod_dc* dc, const int32_t* ids4, uint32_t n, uint32_t maxDepth, bool 
     e = hipGetLastError();
   }
   if (!e) e = hipStreamSynchronize(s);
-  (void)hipFree(dIds);
+  dev_free(dIds);
   if (e) return hip_fail(e, "dual contouring: cells", __FILE__, __LINE__);
   if (int r = check_flags(dc, s)) return r;
   // depth-0 ancestors appended (upsample.cpp:264)
@@ -842,8 +842,8 @@ extern "C" {
 int mlod_dc_create(mlod_dc** out) {
   if (!out) return fail(MLOD_ERR_INVALID, "out is NULL");
   mlod_dc* dc = new mlod_dc();
-  if (hipMalloc((void**)&dc->dCount, 64) != hipSuccess || hipMalloc((void**)&dc->dCount64, 64) != hipSuccess ||
-      hipMalloc((void**)&dc->dFlags, 64) != hipSuccess || hipMalloc((void**)&dc->dBounds, 32 * sizeof(uint32_t)) != hipSuccess) {
+  if (dev_malloc(&dc->dCount, 64) != hipSuccess || dev_malloc(&dc->dCount64, 64) != hipSuccess ||
+      dev_malloc(&dc->dFlags, 64) != hipSuccess || dev_malloc(&dc->dBounds, 32 * sizeof(uint32_t)) != hipSuccess) {
     mlod_dc_destroy(dc);
     return fail(MLOD_ERR_OOM, "dual contouring: counters");
   }
@@ -860,8 +860,7 @@ int mlod_dc_destroy(mlod_dc* dc) {
   dc->cf.release(), dc->cpos.release(), dc->verts.release(), dc->vframe.release();
   dc->rv.release(), dc->rn.release(), dc->rt.release();
   void* p[] = {dc->tmp, dc->dCount, dc->dCount64, dc->dFlags, dc->dBounds};
-  for (void* q : p)
-    if (q) (void)hipFree(q);
+  dev_free(p, sizeof(p) / sizeof(p[0]));
   delete dc;
   return MLOD_OK;
 }
@@ -1018,14 +1017,13 @@ struct MeshBufs {
   ~MeshBufs() {
     (void)hipDeviceSynchronize();
     void* p[] = {key, skey, val, sval, a, b, c, f, tmp, tmp2};
-    for (void* q : p)
-      if (q) (void)hipFree(q);
+    dev_free(p, sizeof(p) / sizeof(p[0]));
   }
 };
 
 template <class T>
 hipError_t dalloc(T** p, size_t n) {
-  return hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T));
+  return dev_malloc(p, std::max<size_t>(n, 1) * sizeof(T));
 }
 
 int check_tris(const uint32_t* tris, uint32_t nt, uint32_t nv) {
@@ -1046,7 +1044,7 @@ int mesh_sort(MeshBufs& B, const uint32_t* dTri, uint32_t nt, int edges, hipStre
   MLOD_HIP(hipGetLastError());
   size_t need = 0;
   MLOD_HIP(rocprim::radix_sort_pairs(nullptr, need, B.key, B.skey, B.val, B.sval, ne, 0, 64, s));
-  MLOD_HIP(hipMalloc(&B.tmp, need + 256));
+  MLOD_HIP(dev_malloc(&B.tmp, need + 256));
   MLOD_HIP(rocprim::radix_sort_pairs(B.tmp, need, B.key, B.skey, B.val, B.sval, ne, 0, 64, s));
   return MLOD_OK;
 }
@@ -1088,7 +1086,7 @@ int mesh_subdivide_dev(const float* dP, uint32_t nv, const uint32_t* dTri, uint3
   size_t n1 = 0, n2 = 0;
   MLOD_HIP(rocprim::inclusive_scan(nullptr, n1, B.a, B.b, ne, rocprim::maximum<uint32_t>(), s));
   MLOD_HIP(rocprim::exclusive_scan(nullptr, n2, B.f, B.c, 0u, ne, rocprim::plus<uint32_t>(), s));
-  MLOD_HIP(hipMalloc(&B.tmp2, std::max(n1, n2) + 256));
+  MLOD_HIP(dev_malloc(&B.tmp2, std::max(n1, n2) + 256));
   size_t bytes = std::max(n1, n2);
   MLOD_HIP(rocprim::inclusive_scan(B.tmp2, bytes, B.a, B.b, ne, rocprim::maximum<uint32_t>(), s));
   bytes = std::max(n1, n2);

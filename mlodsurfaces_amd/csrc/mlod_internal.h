@@ -179,6 +179,16 @@ __device__ __forceinline__ uint32_t xcd_block() {
 }
 #endif
 
+// pool.cpp: device memory from a bounded cache of freed blocks.  dev_free waits for the device, as
+// hipFree does; several blocks given back together wait once.
+hipError_t dev_malloc_bytes(void** p, size_t bytes);
+void dev_free(void* const* ps, size_t n);
+template <class T>
+inline hipError_t dev_malloc(T** p, size_t bytes) {
+  return dev_malloc_bytes(reinterpret_cast<void**>(p), bytes);
+}
+inline void dev_free(void* p) { dev_free(&p, 1); }
+
 // build.hip
 int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t s);
 int dump_tree(const mlod_tree* t, int32_t* depth, float* bb6, float* center3, float* radius, int32_t* father,

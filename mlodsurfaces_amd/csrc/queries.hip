@@ -109,10 +109,8 @@ __global__ void k_reorganize(const uint32_t* __restrict__ invalid, uint32_t n, u
 
 void queries_free(mlod_tree* t) {
   QueryState& qs = t->qs;
-  if (qs.q) (void)hipFree(qs.q);
-  if (qs.qn) (void)hipFree(qs.qn);
-  if (qs.perm) (void)hipFree(qs.perm);
-  if (qs.stage) (void)hipFree(qs.stage);
+  void* bufs[] = {qs.q, qs.qn, qs.perm, qs.stage};
+  dev_free(bufs, 4);
   qs = QueryState{};
 }
 
@@ -120,10 +118,10 @@ int queries_set(mlod_tree* t, const float* xyz, uint32_t m, bool device_src, hip
   QueryState& qs = t->qs;
   if (m > qs.cap) {
     queries_free(t);
-    if (hipMalloc((void**)&qs.q, (size_t)m * sizeof(float4)) != hipSuccess ||
-        hipMalloc((void**)&qs.qn, (size_t)m * sizeof(float4)) != hipSuccess ||
-        hipMalloc((void**)&qs.perm, (size_t)m * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc((void**)&qs.stage, (size_t)m * 3 * sizeof(float)) != hipSuccess) {
+    if (dev_malloc(&qs.q, (size_t)m * sizeof(float4)) != hipSuccess ||
+        dev_malloc(&qs.qn, (size_t)m * sizeof(float4)) != hipSuccess ||
+        dev_malloc(&qs.perm, (size_t)m * sizeof(uint32_t)) != hipSuccess ||
+        dev_malloc(&qs.stage, (size_t)m * 3 * sizeof(float)) != hipSuccess) {
       queries_free(t);
       return fail(MLOD_ERR_OOM, "query buffers: hipMalloc failed for " + std::to_string(m) + " queries");
     }
@@ -140,15 +138,16 @@ int queries_set(mlod_tree* t, const float* xyz, uint32_t m, bool device_src, hip
   void* sortTmp = nullptr;
   const size_t sortBytes = queries_sort_bytes(m);
   if (sortBytes == 0) return fail(MLOD_ERR_HIP, "query sort: temporary storage size query failed");
-  if (hipMalloc((void**)&code, (size_t)m * 4) != hipSuccess || hipMalloc((void**)&code2, (size_t)m * 4) != hipSuccess ||
-      hipMalloc((void**)&idx, (size_t)m * 4) != hipSuccess || hipMalloc(&sortTmp, sortBytes) != hipSuccess) {
-    (void)hipFree(code), (void)hipFree(code2), (void)hipFree(idx), (void)hipFree(sortTmp);
+  if (dev_malloc(&code, (size_t)m * 4) != hipSuccess || dev_malloc(&code2, (size_t)m * 4) != hipSuccess ||
+      dev_malloc(&idx, (size_t)m * 4) != hipSuccess || dev_malloc(&sortTmp, sortBytes) != hipSuccess) {
+    dev_free(code), dev_free(code2), dev_free(idx), dev_free(sortTmp);
     return fail(MLOD_ERR_OOM, "query sort buffers: hipMalloc failed");
   }
   const SortBufs sb{code, code2, idx, sortTmp, sortBytes};
   int r = queries_order(t, src, m, qs.q, qs.qn, qs.perm, sb, s);
   hipError_t e = r == MLOD_OK ? hipStreamSynchronize(s) : hipSuccess;
-  (void)hipFree(code), (void)hipFree(code2), (void)hipFree(idx), (void)hipFree(sortTmp);
+  void* sortBufs[] = {code, code2, idx, sortTmp};
+  dev_free(sortBufs, 4);
   if (r != MLOD_OK) return r;
   if (e != hipSuccess) return hip_fail(e, "query upload", __FILE__, __LINE__);
   return MLOD_OK;
@@ -221,12 +220,12 @@ int queries_fit_kinds(mlod_tree* t, uint32_t n, uint8_t* out, hipStream_t s) {
   if (n > qs.m) return fail(MLOD_ERR_INVALID, "n exceeds the number of uploaded queries");
   if (n == 0) return MLOD_OK;
   uint8_t* d = nullptr;
-  if (hipMalloc((void**)&d, n) != hipSuccess) return fail(MLOD_ERR_OOM, "fit kind buffer");
+  if (dev_malloc(&d, n) != hipSuccess) return fail(MLOD_ERR_OOM, "fit kind buffer");
   k_scatter_kind<<<(qs.m + BS - 1) / BS, BS, 0, s>>>(qs.qn, qs.perm, qs.m, n, d);
   hipError_t e = hipGetLastError();
   if (!e) e = hipMemcpyAsync(out, d, n, hipMemcpyDeviceToHost, s);
   if (!e) e = hipStreamSynchronize(s);
-  (void)hipFree(d);
+  dev_free(d);
   if (e) return hip_fail(e, "fit kinds", __FILE__, __LINE__);
   return MLOD_OK;
 }
@@ -239,8 +238,8 @@ int queries_reorganize(mlod_tree* t, const uint32_t* invalid, uint32_t n, uint32
     if (invalid[i] >= qs.m) return fail(MLOD_ERR_INVALID, "invalid point index out of range");
   if (n == 0) return MLOD_OK;
   uint32_t *dInv = nullptr, *dList = nullptr;
-  if (hipMalloc((void**)&dInv, (size_t)qs.m * 4) != hipSuccess || hipMalloc((void**)&dList, (size_t)n * 4) != hipSuccess) {
-    (void)hipFree(dInv);
+  if (dev_malloc(&dInv, (size_t)qs.m * 4) != hipSuccess || dev_malloc(&dList, (size_t)n * 4) != hipSuccess) {
+    dev_free(dInv);
     return fail(MLOD_ERR_OOM, "reorganize buffers");
   }
   hipError_t e = hipMemcpyAsync(dList, invalid, (size_t)n * 4, hipMemcpyHostToDevice, s);
@@ -253,8 +252,8 @@ int queries_reorganize(mlod_tree* t, const uint32_t* invalid, uint32_t n, uint32
     e = hipGetLastError();
   }
   if (!e) e = hipStreamSynchronize(s);
-  (void)hipFree(dInv);
-  (void)hipFree(dList);
+  dev_free(dInv);
+  dev_free(dList);
   if (e) return hip_fail(e, "reorganize", __FILE__, __LINE__);
   return MLOD_OK;
 }
