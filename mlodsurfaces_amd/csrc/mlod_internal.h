@@ -28,6 +28,7 @@
 #include <string>
 
 #include "../../include/mlod.h"
+#include "curve.h"
 
 namespace mlod {
 
@@ -84,7 +85,7 @@ struct ReqDesc {
   uint32_t count;   // queries
   uint32_t pad0;    // first pool slot of the run (a multiple of kBatchWG)
   uint32_t outOff;  // last steps: first result row of the run in the launch's host staging; else kNoOut
-  float org[3];     // tree box origin and Morton scale
+  float org[3];     // tree box origin and curve scale
   float scale[3];
 };
 constexpr uint32_t kNoOut = 0xffffffffu;
@@ -167,7 +168,7 @@ int hip_fail(hipError_t e, const char* what, const char* file, int line);
   } while (0)
 
 // Workgroups are dispatched round-robin over the 8 XCDs of the chip, each with its own L2.
-// Queries are Morton-sorted, so consecutive workgroups touch the same octree nodes; this maps
+// Queries are sorted along a space-filling curve, so consecutive workgroups touch the same octree nodes; this maps
 // the hardware workgroup index to a logical one such that each XCD walks one contiguous share
 // of the query range (a bijection on [0, gridDim.x)), keeping each L2's working set disjoint.
 #if defined(__HIPCC__)
@@ -218,7 +219,7 @@ int launch_neighbors(mlod_tree* t, uint32_t n, uint32_t n_iter, hipStream_t s);
 int project_uploaded(mlod_tree* t, uint32_t n, uint32_t n_iter, float step_max, hipStream_t s);
 
 // queries.hip
-// Buffers of the query sort: Morton codes (two arrays of m), caller indices (m) and rocPRIM's
+// Buffers of the query sort: curve keys (two arrays of m), caller indices (m) and rocPRIM's
 // temporary storage (tmpBytes, at least queries_sort_bytes(m)).
 struct SortBufs {
   uint32_t* code;
@@ -228,7 +229,7 @@ struct SortBufs {
   size_t tmpBytes;
 };
 size_t queries_sort_bytes(uint32_t m);  // 0 if the size query fails
-// Morton order of m device points in the tree's box: q / qn (m float4 each) receive the sorted
+// Curve order of m device points in the tree's box: q / qn (m float4 each) receive the sorted
 // points and zero normals, perm (m) the caller index of each sorted slot.  Launches only (no
 // allocation, no synchronisation).
 int queries_order(const mlod_tree* t, const float* d_xyz, uint32_t m, float4* q, float4* qn, uint32_t* perm,

@@ -426,7 +426,7 @@ void k_knn(TreeView tv, HalfBox hb, KParams kp,
   qn[i] = nout;
 }
 
-// Ball APSS, one wavefront at a time.  The 64 lanes' queries are Morton neighbours, so their
+// Ball APSS, one wavefront at a time.  The 64 lanes' queries are neighbours on the curve, so their
 // balls overlap almost entirely: the wavefront walks the octree once over the union of its
 // balls (node boxes against the lanes' query box grown by r), takes the points of every
 // reached subtree that is small enough as a contiguous range, loads each range 64 points at a

@@ -2,8 +2,8 @@
 // callers that cannot allocate device memory (code under HIP graph capture, tight serving loops).
 //
 // mlod_project_points keeps the tree's uploaded queries aside and projects the given points in
-// buffers of its own, allocated per call: the Morton-sorted points and their normals, the sort
-// permutation, the Morton codes and caller indices, and rocPRIM's sort storage.  Here those
+// buffers of its own, allocated per call: the curve-sorted points and their normals, the sort
+// permutation, the curve keys and caller indices, and rocPRIM's sort storage.  Here those
 // buffers are carved from one file-scope device array, `scratch`, of kScratchBytes, which holds
 // up to MLOD_NOALLOC_MAX_QUERIES points.  The array exists once per GPU for the life of the
 // process; its address on each device is resolved with hipGetSymbolAddress on the first call

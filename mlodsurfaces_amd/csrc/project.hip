@@ -1,6 +1,6 @@
 // project.hip — MLoD and global APSS projection kernels (gfx950).
 //
-// One lane per query (queries Morton-sorted by queries.hip, so a wavefront's 64 lanes walk
+// One lane per query (queries sorted along a curve by queries.hip, so a wavefront's 64 lanes walk
 // neighbouring parts of the tree).  The MLoD sum of the reference,
 //   value(leaf)  = sum over its points of w(p_i) stats_i                (Fastapss.cu:189-200)
 //   value(far)   = w(pbar) stats                                        (Fastapss.cu:214-237)
@@ -1108,7 +1108,7 @@ __device__ __forceinline__ void fit_step(const typename FormT<FORM>::Acc& acc, V
 // ----------------------------------------------------------------------------- kernels
 // MLoD projection of the sorted queries q[0..m) in place (projectCuda, Fastapss.cu:398-437):
 // n_iter steps per query, one lane per query; queries whose caller index perm[i] >= limit are
-// skipped.  A wavefront's 64 lanes hold 64 consecutive (Morton-ordered) queries, so they start
+// skipped.  A wavefront's 64 lanes hold 64 consecutive (curve-ordered) queries, so they start
 // their walks together and load the same nodes at the same iterations for much of them.
 template <int FORM, int SEM, int KT, bool CNT>
 __global__ __launch_bounds__(PBS) void k_project(TreeView tv, KParams kp, float4* __restrict__ q, float4* __restrict__ qn,

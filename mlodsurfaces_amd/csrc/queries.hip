@@ -3,7 +3,7 @@
 //
 // The reference sorts each query batch along a Morton curve on the host before upload
 // (Pn::order, sources/apss/Pn.cpp:388-445) so that neighbouring GPU threads traverse the
-// same part of the octree.  Here the library does it on the device: a 30-bit Morton code of
+// same part of the octree.  Here the library does it on the device: a 30-bit Hilbert key of
 // each query in the tree box, a radix sort of (code, caller index), and a gather.  The
 // queries then stay in that order, projected in place across calls; downloads scatter back
 // to the caller's order through `perm`.
@@ -20,16 +20,7 @@ namespace {
 
 constexpr int BS = 256;
 
-__device__ __forceinline__ uint32_t spread10(uint32_t v) {
-  v &= 0x3ffu;
-  v = (v | (v << 16)) & 0x030000ffu;
-  v = (v | (v << 8)) & 0x0300f00fu;
-  v = (v | (v << 4)) & 0x030c30c3u;
-  v = (v | (v << 2)) & 0x09249249u;
-  return v;
-}
-
-__global__ __launch_bounds__(BS) void k_morton(const float* __restrict__ xyz, uint32_t m, float bx, float by, float bz,
+__global__ __launch_bounds__(BS) void k_curve(const float* __restrict__ xyz, uint32_t m, float bx, float by, float bz,
                                                float sx, float sy, float sz, uint32_t* __restrict__ code,
                                                uint32_t* __restrict__ idx) {
   const uint32_t i = blockIdx.x * BS + threadIdx.x;
@@ -43,7 +34,7 @@ __global__ __launch_bounds__(BS) void k_morton(const float* __restrict__ xyz, ui
     u = fminf(fmaxf(u, 0.f), 1023.f);  // NaN -> 0
     c[a] = (uint32_t)u;
   }
-  code[i] = spread10(c[0]) | (spread10(c[1]) << 1) | (spread10(c[2]) << 2);
+  code[i] = curve_key(c[0], c[1], c[2]);
   idx[i] = i;
 }
 
@@ -85,8 +76,8 @@ __global__ __launch_bounds__(BS) void k_invperm(const uint32_t* __restrict__ per
 
 // APSS::reorganizePoints (GPUUtils.cu:413-450): for i = 0, 1, ..., n - 1 in order, the caller's
 // queries invalid[i] and endValid - 1 - i exchange positions; normals stay with their index.
-// Positions are exchanged by exchanging the two slots' owners (perm), which keeps the Morton
-// order of the slots, and the two slots' normals are exchanged back.  One lane runs the list in
+// Positions are exchanged by exchanging the two slots' owners (perm), which keeps the
+// curve's order of the slots, and the two slots' normals are exchanged back.  One lane runs the list in
 // order, so overlapping pairs resolve as in a sequential loop.  Indices were checked on the host.
 __global__ void k_reorganize(const uint32_t* __restrict__ invalid, uint32_t n, uint32_t endValid,
                              uint32_t* __restrict__ perm, uint32_t* __restrict__ inv, float4* __restrict__ qn) {
@@ -169,7 +160,7 @@ int queries_order(const mlod_tree* t, const float* d_xyz, uint32_t m, float4* q,
     sc[a] = ext > 0.f ? 1024.f / ext : 0.f;
   }
   const uint32_t nb = (m + BS - 1) / BS;
-  k_morton<<<nb, BS, 0, s>>>(d_xyz, m, t->bb[0], t->bb[1], t->bb[2], sc[0], sc[1], sc[2], sb.code, sb.idx);
+  k_curve<<<nb, BS, 0, s>>>(d_xyz, m, t->bb[0], t->bb[1], t->bb[2], sc[0], sc[1], sc[2], sb.code, sb.idx);
   MLOD_HIP(hipGetLastError());
   size_t bytes = sb.tmpBytes;
   MLOD_HIP(rocprim::radix_sort_pairs(sb.tmp, bytes, sb.code, sb.code2, sb.idx, perm, m, 0, 30, s));

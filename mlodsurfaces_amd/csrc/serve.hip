@@ -11,7 +11,7 @@
 //   arrival order.  Bulk work gets a launch at least every kBulkMaxWaitMs, so interactive
 //   requests cannot starve it.
 // * Residency.  Chunks taken by a step launch are staged into a device query pool (pinned host
-//   staging -> device; Morton key in the tree's box; radix sort; gather into pool blocks of
+//   staging -> device; curve key in the tree's box; radix sort; gather into pool blocks of
 //   kBatchWG slots) and stay there as a run until their last step; consecutive chunks of one
 //   request taken together form one run, sorted and walked together.
 // * Steps.  Each of `inflight` streams keeps one step launch on the device; when it completes,
@@ -66,7 +66,7 @@ namespace {
 
 using clk = std::chrono::steady_clock;
 constexpr int BS = 256;
-constexpr uint32_t kMaxRuns = 1024;         // runs per launch: the run index fits 10 bits above the Morton code
+constexpr uint32_t kMaxRuns = 1024;         // runs per launch: the run index fits 10 bits above the curve key
 constexpr double kNominalPtsPerMs = 2.0e4;  // deadline slack: 1 ms per 20k projected points
 constexpr double kInteractivePts = 2.0e6;   // interactive class: at most 2M projected points (200k queries x 10 steps)
 constexpr uint32_t kInteractiveSteps = 16;  // steps per launch for interactive runs (all, for n_iter <= 16)
@@ -74,16 +74,7 @@ constexpr uint32_t kBulkSteps = 2;          // steps per launch for bulk runs
 constexpr uint32_t kPoolLaunches = 4;       // pool capacity, in launches' worth of blocks per stream
 constexpr double kBulkMaxWaitMs = 20.0;     // bulk work gets a launch at least this often
 
-__device__ __forceinline__ uint32_t spread10(uint32_t v) {
-  v &= 0x3ffu;
-  v = (v | (v << 16)) & 0x030000ffu;
-  v = (v | (v << 8)) & 0x0300f00fu;
-  v = (v | (v << 4)) & 0x030c30c3u;
-  v = (v | (v << 2)) & 0x09249249u;
-  return v;
-}
-
-// key = run index << 30 | Morton code of the query in its tree's box, over the staged queries of
+// key = run index << 30 | curve key of the query in its tree's box, over the staged queries of
 // the launch's new runs (reqs[0..nReq), staged back to back from their slot0)
 __global__ __launch_bounds__(BS) void k_batch_keys(const float* __restrict__ in, uint32_t slots,
                                                    const ReqDesc* __restrict__ reqs, uint32_t nReq,
@@ -106,7 +97,7 @@ __global__ __launch_bounds__(BS) void k_batch_keys(const float* __restrict__ in,
     u = fminf(fmaxf(u, 0.f), 1023.f);
     c[a] = (uint32_t)u;
   }
-  key[i] = ((uint64_t)lo << 30) | (spread10(c[0]) | (spread10(c[1]) << 1) | (spread10(c[2]) << 2));
+  key[i] = ((uint64_t)lo << 30) | curve_key(c[0], c[1], c[2]);
   idx[i] = i;
 }
 
