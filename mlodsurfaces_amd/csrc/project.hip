@@ -104,6 +104,37 @@ __device__ __forceinline__ float weight32(const KP& k, float d2) {
   }
 }
 
+// weight32 of U squared distances at once: the terms of one sigma for all of them before the next
+// sigma's, so that U exponentials are in flight and the uniform exits are shared.
+template <int KT, int U, class KP>
+__device__ __forceinline__ void weights32(const KP& k, const float (&d2)[U], float (&w)[U]) {
+  if constexpr (KT == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = k.b[0] * __builtin_amdgcn_exp2f(d2[u] * k.a[0]);
+    int ns = k.ns;
+#pragma unroll
+    for (int s = 1; s < 8; ++s) {
+      asm volatile("" : "+s"(ns));
+      if (s >= ns) break;
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = fmaf(k.b[s], __builtin_amdgcn_exp2f(d2[u] * k.a[s]), w[u]);
+    }
+    for (int s = 8; s < ns; ++s) {
+      const float A = k.a[s], B = k.b[s];
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = fmaf(B, __builtin_amdgcn_exp2f(d2[u] * A), w[u]);
+    }
+    if (__float_as_uint(k.c) << 1) {
+      asm volatile("");
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = w[u] == 0.f ? k.c : w[u];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = weight32<KT>(k, d2[u]);
+  }
+}
+
 template <int KT>
 __device__ __forceinline__ double weight64(const KParams& k, double d2) {
   if constexpr (KT < 0) {
@@ -1209,14 +1240,148 @@ __global__ __launch_bounds__(PBS) void k_project_wave(TreeView tv, KParams kp, f
   }
 }
 
-// Global APSS over all points (GlobalAPSS.cu:113-192 / APSSStats, CPUUtils.cpp:515-528):
-// point tiles staged through LDS, every lane of the workgroup sums the tile for its query.
+// ----------------------------------------------------------------------------- global APSS
+// One projection step from the nine sums over all neighbours, in the global frame in FP64:
+// {sum w, sum w p, sum w n, sum w p.n, sum w |p|^2}.  The compensated form moves them to the query's
+// frame (in FP64 that costs 1e-16 |q|^2 against the kernel's width squared).
+template <int FORM, int SEM>
+__device__ __forceinline__ void fit_sums(const double* S, V3<double>& qd, float stepMax, float4& nout) {
+  const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
+  if constexpr (FORM == 1) {
+    const V3<double> q{qf.x, qf.y, qf.z}, sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
+    V3<double> p, n;
+    float kind;
+    fit<double, double, SEM, true>(S[0], V3<double>{sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0]}, sn,
+                                   S[7] - dot3(q, sn), S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0], V3<double>{0, 0, 0},
+                                   (double)stepMax, p, n, kind);
+    qd = V3<double>{q.x + p.x, q.y + p.y, q.z + p.z};
+    nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+  } else {
+    AccP64 a{S[0], S[1], S[2], S[3], S[4], S[5], S[6], S[7], S[8]};
+    fit_step<2, SEM>(a, qd, qf, stepMax, nout);
+  }
+}
+
+typedef double Acc4 __attribute__((ext_vector_type(4)));
+
+// Global APSS over all points (GlobalAPSS.cu:113-192 / APSSStats, CPUUtils.cpp:515-528), compensated and
+// FP64 forms: the sums are a contraction, weights (queries x points) times moments (points x 9), and run on the matrix cores.
+// A workgroup of W wavefronts takes 16 queries; in one step a wavefront takes 4 points, each lane the
+// weight of one (query lane % 16, point lane / 16) pair, and one FP64 16x16x4 matrix instruction adds
+// the 64 weights times the 4 points' nine moments (columns 9..15 hold copies that nobody reads).  So a
+// pair costs its distance and weight and none of the nine sums, which the matrix cores add in FP64:
+// the weights keep their form's precision, the sums gain.  Points are staged through LDS a tile at a time,
+// their moments formed once per tile.
+// Step g of a tile belongs to slice g % 16; a wavefront holds 16 / W slices apart, and the slices are
+// added in order at the end, so the result does not depend on W.
+// Bound by the weights' vector instructions.  30k points, four sigmas, FP32C: 20k queries 6.0 -> 0.76 ms,
+// 500 queries 6.0 -> 0.19 (one lane per query left the chip two thirds empty, and each pair paid nine
+// compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries: 20.1 -> 1.2.
 // The fit uses the 1e-12 plane threshold of GlobalAPSS.cu:143 (the REF_CPU fit).
-template <int FORM, int KT>
-__global__ __launch_bounds__(PBS) void k_global(TreeView tv, KParams kp, float4* __restrict__ q, float4* __restrict__ qn,
+constexpr int kGlobalQ = 16;
+constexpr int kSlices = 16;
+template <int FORM, int KT, int W>
+__global__ __launch_bounds__(W * 64) void k_global(TreeView tv, KParams kp, float4* __restrict__ q, float4* __restrict__ qn,
+                                                   const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit,
+                                                   uint32_t nIter, float stepMax) {
+  using T = typename FormT<FORM>::T;
+  constexpr uint32_t TILE = W == 4 ? 256 : 512;
+  constexpr int NA = kSlices / W;         // slices of a wavefront
+  constexpr int U = 4;                    // steps of a round
+  constexpr uint32_t ROUND = U * W * 4;   // points of a round (a multiple of the slices' 64)
+  __shared__ float4 sP[TILE];
+  __shared__ double sF[TILE][9];  // then the slices' sums: [16 slices][16 queries][9]
+  __shared__ double sS[kGlobalQ][9], sQ[kGlobalQ][3];
+  static_assert(sizeof(sF) >= sizeof(double) * kSlices * kGlobalQ * 9, "the slices' sums fit the moments' tile");
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = lane & 15u, kk = lane >> 4, col = min(row, 8u);
+  const uint32_t i = blockIdx.x * kGlobalQ + tid;
+  const bool active = tid < kGlobalQ && i < m && !(limit < m && perm[i] >= limit);
+  V3<double> qd{0, 0, 0};  // (of the first 16 threads)
+  float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (active) {
+    const float4 q4 = q[i];
+    qd = V3<double>{q4.x, q4.y, q4.z};
+  }
+  for (uint32_t it = 0; it < nIter; ++it) {
+    if (tid < kGlobalQ) {
+      sQ[tid][0] = FORM == 2 ? qd.x : (double)(float)qd.x;
+      sQ[tid][1] = FORM == 2 ? qd.y : (double)(float)qd.y;
+      sQ[tid][2] = FORM == 2 ? qd.z : (double)(float)qd.z;
+    }
+    __syncthreads();
+    const T qx = (T)sQ[row][0], qy = (T)sQ[row][1], qz = (T)sQ[row][2];
+    Acc4 acc[NA];
+#pragma unroll
+    for (int u = 0; u < NA; ++u) acc[u] = Acc4{0, 0, 0, 0};
+    for (uint32_t base = 0; base < tv.n; base += TILE) {
+      const uint32_t cnt = min(TILE, tv.n - base), end = (cnt + ROUND - 1u) / ROUND * ROUND;
+      __syncthreads();
+      for (uint32_t t = tid; t < end; t += W * 64) {
+        const bool in = t < cnt;  // past the end: the tile's first point with no moments
+        const float4 P = tv.pts[base + (in ? t : 0u)], N = tv.nrm[base + (in ? t : 0u)];
+        const double a = in ? (double)P.w : 0.0, x = P.x, y = P.y, z = P.z;
+        sP[t] = P;
+        sF[t][0] = a;
+        sF[t][1] = a * x, sF[t][2] = a * y, sF[t][3] = a * z;
+        sF[t][4] = a * N.x, sF[t][5] = a * N.y, sF[t][6] = a * N.z;
+        sF[t][7] = a * ((x * N.x + y * N.y) + z * N.z);
+        sF[t][8] = a * ((x * x + y * y) + z * z);
+      }
+      __syncthreads();
+      for (uint32_t t0 = 4u * wave + kk; t0 < end; t0 += ROUND) {
+        T d2[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float4 P = sP[t0 + u * 4 * W];
+          const T dx = (T)P.x - qx, dy = (T)P.y - qy, dz = (T)P.z - qz;
+          if constexpr (FORM == 2)
+            d2[u] = dx * dx + dy * dy + dz * dz;
+          else
+            d2[u] = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+        }
+        T w[U];
+        if constexpr (FORM == 2) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) w[u] = weight64<KT>(kp, d2[u]);
+        } else {
+          weights32<KT, U>(kp, d2, w);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          acc[u % NA] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)w[u], sF[t0 + u * 4 * W][col], acc[u % NA], 0, 0, 0);
+      }
+    }
+    // the slices' sums: register r of a lane holds query 4 r + lane / 16, moment lane % 16
+    __syncthreads();
+    double* red = &sF[0][0];
+    if (row < 9u) {
+#pragma unroll
+      for (int u = 0; u < NA; ++u)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+          red[((u * W + wave) * kGlobalQ + 4u * r + kk) * 9u + row] = acc[u][r];
+    }
+    __syncthreads();
+    for (uint32_t t = tid; t < kGlobalQ * 9u; t += W * 64) {
+      double x = 0.0;
+      for (int sl = 0; sl < kSlices; ++sl) x += red[sl * kGlobalQ * 9 + t];
+      sS[t / 9u][t % 9u] = x;
+    }
+    __syncthreads();
+    if (tid < kGlobalQ) fit_sums<FORM, MLOD_SEM_REF_CPU>(sS[tid], qd, stepMax, nout);
+  }
+  if (active) {
+    q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
+    qn[i] = nout;
+  }
+}
+
+// The plain FP32 form of global APSS: the reference's own sums, in FP32 and in point order, one lane per
+// query over point tiles in LDS.
+template <int KT>
+__global__ __launch_bounds__(PBS) void k_global_plain(TreeView tv, KParams kp, float4* __restrict__ q, float4* __restrict__ qn,
                                                 const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit,
                                                 uint32_t nIter, float stepMax) {
-  using T = typename FormT<FORM>::T;
   __shared__ float4 sP[PBS], sN[PBS];
   const int tid = threadIdx.x;
   const uint32_t i = blockIdx.x * PBS + tid;
@@ -1225,14 +1390,9 @@ __global__ __launch_bounds__(PBS) void k_global(TreeView tv, KParams kp, float4*
   V3<double> qd{q4.x, q4.y, q4.z};
   float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
   for (uint32_t it = 0; it < nIter; ++it) {
-    typename FormT<FORM>::Acc acc;
+    AccP32 acc;
     acc.init();
     const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
-    V3<T> qt;
-    if constexpr (FORM == 2)
-      qt = V3<T>{qd.x, qd.y, qd.z};
-    else
-      qt = V3<T>{qf.x, qf.y, qf.z};
     for (uint32_t base = 0; base < tv.n; base += PBS) {
       __syncthreads();
       if (base + tid < tv.n) {
@@ -1246,15 +1406,11 @@ __global__ __launch_bounds__(PBS) void k_global(TreeView tv, KParams kp, float4*
         lv.pts = sP;
         lv.nrm = sN;
         for (uint32_t j = 0; j < cnt; ++j) {
-          add_point<FORM, KT>(acc, kp, lv, j, qt, T(1));
-          if constexpr (FORM == 1) {
-            if ((j & (kFlush - 1)) == kFlush - 1) acc.flush();
-          }
+          add_point<0, KT>(acc, kp, lv, j, qf, 1.f);
         }
-        if constexpr (FORM == 1) acc.flush();
       }
     }
-    fit_step<FORM, MLOD_SEM_REF_CPU>(acc, qd, qf, stepMax, nout);
+    fit_step<0, MLOD_SEM_REF_CPU>(acc, qd, qf, stepMax, nout);
   }
   if (active) {
     q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
@@ -1362,8 +1518,19 @@ int launch_one(const mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t n
 template <int FORM, int KT>
 void launch_global(const mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter, float stepMax, hipStream_t s) {
   const uint32_t m = t->qs.m;
-  k_global<FORM, KT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter,
-                                                         stepMax);
+  if constexpr (FORM == 0) {
+    k_global_plain<KT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter,
+                                                            stepMax);
+  } else {
+    // Four wavefronts a workgroup load the chip's 1024 SIMDs twice over from 512 workgroups on; below
+    // that the points are split over sixteen (30k points, us with 4 / 16 wavefronts: 500 queries 276 /
+    // 189, 4k 289 / 203, 8k 385 / 389, 12k 496 / 554, 20k 761 / 884).
+    const uint32_t grid = (m + kGlobalQ - 1) / kGlobalQ;
+    if (grid >= 512)
+      k_global<FORM, KT, 4><<<grid, 4 * 64, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax);
+    else
+      k_global<FORM, KT, 16><<<grid, 16 * 64, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax);
+  }
 }
 
 template <int FORM, int SEM>
