@@ -27,6 +27,7 @@
 #include <cmath>
 
 #include "mlod_internal.h"
+#include "weights.h"
 
 namespace mlod {
 namespace {
@@ -102,41 +103,6 @@ struct SumC {  // compensated, query frame
 struct SumD {
   double w, px, py, pz, nx, ny, nz, pn, pp;
 };
-
-template <int KT>
-__device__ __forceinline__ float weight32(const KParams& k, float d2) {
-  if constexpr (KT == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
-    float w = k.b[0] * __builtin_amdgcn_exp2f(d2 * k.a[0]);
-    for (int s = 1; s < k.ns; ++s) w = fmaf(k.b[s], __builtin_amdgcn_exp2f(d2 * k.a[s]), w);
-    return w == 0.f ? k.c : w;
-  } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN) {
-    return __builtin_amdgcn_exp2f(d2 * k.a[0]) + k.c;
-  } else {
-    const float base = k.cp / (d2 + k.c);
-    if (k.eint > 0) {
-      float r = 1.f, b = base;
-      for (int e = k.eint; e; e >>= 1) {
-        if (e & 1) r *= b;
-        b *= b;
-      }
-      return r;
-    }
-    return __builtin_amdgcn_exp2f(k.e * __builtin_amdgcn_logf(base));
-  }
-}
-
-template <int KT>
-__device__ __forceinline__ double weight64(const KParams& k, double d2) {
-  if constexpr (KT == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
-    double w = 0.0;
-    for (int s = 0; s < k.ns; ++s) w += exp(d2 * k.ad[s]) * k.bd[s];
-    return w == 0.0 ? (double)k.c : w;
-  } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN) {
-    return exp(d2 * k.ad[0]) + (double)k.c;
-  } else {
-    return pow((double)k.cp, (double)k.e) / pow(d2 + (double)k.c, (double)k.e);
-  }
-}
 
 template <int FORM>
 struct Sums;
@@ -426,14 +392,13 @@ void k_knn(TreeView tv, HalfBox hb, KParams kp,
   qn[i] = nout;
 }
 
-// Ball APSS, one wavefront at a time.  The 64 lanes' queries are neighbours on the curve, so their
+// Ball APSS, one wavefront at a time.  A wavefront's queries are neighbours on the curve, so their
 // balls overlap almost entirely: the wavefront walks the octree once over the union of its
-// balls (node boxes against the lanes' query box grown by r), takes the points of every
-// reached subtree that is small enough as a contiguous range, loads each range 64 points at a
-// time with one coalesced load per lane, and broadcasts the points lane to lane; every lane
-// sums the points inside its own ball.  Ranges come in increasing point order, so each lane
-// sums exactly the points inside its ball, in increasing point order (the order of a walk over
-// its own ball alone), whatever the other lanes' queries.
+// balls (node boxes against its queries' box grown by r), takes the points of every
+// reached subtree that is small enough as a contiguous range, and loads each range 64 points at a
+// time with one coalesced load per lane; every query sums the points inside its own ball.  Ranges
+// come in increasing point order, so a query sums exactly the points inside its ball, in increasing
+// point order (the order of a walk over its own ball alone), whatever the wavefront's other queries.
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
@@ -461,6 +426,8 @@ __device__ __forceinline__ float box_box_d2(const float* __restrict__ box, uint3
 
 constexpr uint32_t kWaveScanPoints = 256;  // subtrees up to this size are taken as one range
 
+// The plain FP32 form: the reference's own sums, in FP32, 64 queries a wavefront, each point broadcast
+// lane to lane.
 template <int FORM, int KT>
 __global__ __launch_bounds__(NBS) void k_ball_wave(TreeView tv, const float* __restrict__ box, KParams kp,
                                                    float4* __restrict__ q, float4* __restrict__ qn,
@@ -552,6 +519,188 @@ __global__ __launch_bounds__(NBS) void k_ball_wave(TreeView tv, const float* __r
   }
 }
 
+// One step from FP64 sums over the neighbours in the global frame (CPUUtils.cpp:719-735): the
+// compensated form moves them to the query's frame.
+template <int FORM>
+__device__ __forceinline__ void fit_sums(const double* S, V3<double>& qd, V3<float> qf, float4& nout) {
+  V3<double> p, n;
+  float kind;
+  const V3<double> sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
+  if constexpr (FORM == 1) {
+    const V3<double> q{qf.x, qf.y, qf.z};
+    fit_aliased<double>(S[0], V3<double>{sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0]}, sn, S[7] - dot3(q, sn),
+                        S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0], V3<double>{0, 0, 0}, p, n, kind);
+    qd = V3<double>{q.x + p.x, q.y + p.y, q.z + p.z};
+  } else {
+    fit_aliased<double>(S[0], sp, sn, S[7], S[8], qd, p, n, kind);
+    qd = p;
+  }
+  nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+}
+
+// Orders a wavefront's own LDS writes and reads (its LDS operations complete in order).
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+typedef double Acc4 __attribute__((ext_vector_type(4)));
+
+// The compensated and FP64 forms: a wavefront walks the union of 16 queries' balls, the sums on the matrix
+// cores.  A range's points go to LDS 64 at a time with their nine moments {1, p, n, p.n, |p|^2} in
+// FP64; then, four points a step and four steps at once, each lane weighs one (query lane % 16, point
+// lane / 16) pair a step, a pair outside its ball with weight 0, and an FP64 16x16x4 matrix
+// instruction adds the 64 weights times the points' moments.  A pair so costs its distance, test and
+// weight and none of the nine sums.  The ranges and the steps within them are the tree's, whatever the
+// queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its wavefront's other
+// queries.  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
+// ones.  r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k 1.3;
+// FP64, 100k queries 1.6.  Wavefronts of 64 queries (unions of four times the surface, four times fewer
+// wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
+constexpr uint32_t kBallQ = 16;            // queries a wavefront
+constexpr uint32_t kScanPointsBall = 512;  // subtrees up to this size are taken as one range (256: 1.65 ms, 1024: 1.57)
+
+template <int FORM, int KT>
+__global__ __launch_bounds__(NBS) void k_ball_sums(TreeView tv, const float* __restrict__ box, KParams kp,
+                                                   float4* __restrict__ q, float4* __restrict__ qn,
+                                                   const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit,
+                                                   uint32_t nIter, float r2f) {
+  constexpr int kWaves = NBS / 64, U = 4;  // steps at once
+  __shared__ uint32_t sFirst[kLevels][kWaves];
+  __shared__ uint32_t sMask[kLevels][kWaves];
+  __shared__ float4 sPts[kWaves][64];
+  __shared__ double sMom[kWaves][64][9];  // then the wavefront's sums, 16 queries x 9
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t row = (uint32_t)lane & 15u, kk = (uint32_t)lane >> 4, col = min(row, 8u);
+  const uint32_t i0 = (xcd_block() * kWaves + (uint32_t)wv) * kBallQ;  // the wavefront's first slot
+  const uint32_t i = i0 + (uint32_t)lane;
+  if (i0 >= m) return;  // whole wavefront past the end
+  const bool mine = lane < (int)kBallQ && i < m && !(limit < m && perm[i] >= limit);
+  // lanes without a query of their own follow the wavefront's first query (never stored)
+  const float4 q4 = q[mine ? i : i0];
+  V3<double> qd{q4.x, q4.y, q4.z};
+  float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
+  bool done = !mine;
+  const float r = sqrtf(r2f) * kSlack;
+  float4* pts = sPts[wv];
+  double (*mom)[9] = sMom[wv];
+  for (uint32_t it = 0; it < nIter; ++it) {
+    const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
+    // the union of the live lanes' balls, bounded by their query box grown by r
+    const float big = 3.0e38f;
+    const V3<float> qlo{wave_min(done ? big : qf.x) - r, wave_min(done ? big : qf.y) - r, wave_min(done ? big : qf.z) - r};
+    const V3<float> qhi{wave_max(done ? -big : qf.x) + r, wave_max(done ? -big : qf.y) + r, wave_max(done ? -big : qf.z) + r};
+    if (qlo.x > qhi.x) break;  // every lane finished (uniform)
+    const V3<float> g{__shfl(qf.x, (int)row, 64), __shfl(qf.y, (int)row, 64), __shfl(qf.z, (int)row, 64)};  // the pairs' query
+    V3<double> gd{0, 0, 0};
+    if constexpr (FORM == 2)
+      gd = V3<double>{__shfl(qd.x, (int)row, 64), __shfl(qd.y, (int)row, 64), __shfl(qd.z, (int)row, 64)};
+    Acc4 acc{0, 0, 0, 0};
+    bool some = false;
+    int lvl = -1;
+    uint32_t cur = 0;
+    bool have = true;
+    while (true) {
+      if (have) {
+        const uint4 h = tv.hdr[cur];
+        const uint2 sp = tv.span[cur];
+        if (hdr_leaf(h.y) || sp.y - sp.x <= kScanPointsBall) {
+          const uint32_t a = __builtin_amdgcn_readfirstlane(sp.x), b = __builtin_amdgcn_readfirstlane(sp.y);
+          for (uint32_t base = a; base < b; base += 64) {
+            const uint32_t nb = min(64u, b - base);
+            const bool in = (uint32_t)lane < nb;  // past the end: the first point with no moments
+            const float4 P = tv.pts[base + (in ? (uint32_t)lane : 0u)], N = tv.nrm[base + (in ? (uint32_t)lane : 0u)];
+            const double e = in ? 1.0 : 0.0, x = P.x, y = P.y, z = P.z, nx = N.x, ny = N.y, nz = N.z;
+            pts[lane] = P;
+            mom[lane][0] = e;
+            mom[lane][1] = e * x, mom[lane][2] = e * y, mom[lane][3] = e * z;
+            mom[lane][4] = e * nx, mom[lane][5] = e * ny, mom[lane][6] = e * nz;
+            mom[lane][7] = e * ((x * nx + y * ny) + z * nz);
+            mom[lane][8] = e * ((x * x + y * y) + z * z);
+            wave_order();
+            for (uint32_t t0 = kk; t0 < nb + kk; t0 += 4 * U) {  // uniform
+              float d2[U];
+              bool hit[U], any = false;
+#pragma unroll
+              for (int v = 0; v < U; ++v) {
+                d2[v] = kd_d2(pts[t0 + 4 * v], g);
+                hit[v] = d2[v] <= r2f;
+                any |= hit[v];
+              }
+              if (__builtin_amdgcn_ballot_w64(any) == 0ull) continue;  // uniform
+              double w[U];
+              if constexpr (FORM == 2) {
+#pragma unroll
+                for (int v = 0; v < U; ++v) {
+                  const float4 Pt = pts[t0 + 4 * v];
+                  const double dx = gd.x - (double)Pt.x, dy = gd.y - (double)Pt.y, dz = gd.z - (double)Pt.z;
+                  w[v] = weight64<KT>(kp, dx * dx + dy * dy + dz * dz);
+                }
+              } else {
+                float wf[U];
+                weights32<KT, U>(kp, d2, wf);
+#pragma unroll
+                for (int v = 0; v < U; ++v) w[v] = (double)wf[v];
+              }
+#pragma unroll
+              for (int v = 0; v < U; ++v)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(hit[v] ? w[v] : 0.0, mom[t0 + 4 * v][col], acc, 0, 0, 0);
+              some |= any;
+            }
+            wave_order();
+          }
+        } else {
+          const uint32_t first = __builtin_amdgcn_readfirstlane(h.x), nc = hdr_count(h.y);
+          uint32_t mask = 0;
+          for (uint32_t c = 0; c < nc; ++c)
+            if (box_box_d2(box, first + c, qlo, qhi) <= 0.f) mask |= 1u << c;
+          ++lvl;
+          if (lane == 0) {
+            sFirst[lvl][wv] = first;
+            sMask[lvl][wv] = mask;
+          }
+        }
+        have = false;
+      }
+      if (lvl < 0) break;
+      const uint32_t mask = __builtin_amdgcn_readfirstlane(sMask[lvl][wv]);
+      if (mask == 0) {
+        --lvl;
+        continue;
+      }
+      if (lane == 0) sMask[lvl][wv] = mask & (mask - 1u);
+      cur = __builtin_amdgcn_readfirstlane(sFirst[lvl][wv]) + (uint32_t)__builtin_ctz(mask);
+      have = true;
+    }
+    // register v of a lane holds query 4 v + lane / 16, moment lane % 16
+    const uint64_t b = __builtin_amdgcn_ballot_w64(some);
+    const uint32_t found = (uint32_t)(b | b >> 16 | b >> 32 | b >> 48) & 0xffffu;  // queries with a point in their ball
+    if (row < 9u) {
+#pragma unroll
+      for (uint32_t v = 0; v < 4; ++v) mom[4u * v + kk][row] = acc[v];
+    }
+    wave_order();
+    if (!done) {
+      if (!((found >> lane) & 1u)) {  // empty ball: the starting query, zero normal (CPUUtils.cpp:711-716)
+        qd = V3<double>{q4.x, q4.y, q4.z};
+        nout = make_float4(0.f, 0.f, 0.f, 0.f);
+        done = true;
+      } else {
+        double S[9];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) S[c] = mom[lane][c];
+        fit_sums<FORM>(S, qd, qf, nout);
+      }
+    }
+    wave_order();
+  }
+  if (mine) {
+    q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
+    qn[i] = nout;
+  }
+}
+
 // The root's half extents and the rounding margin of a cell's bounds.  Every bound of a cell is the
 // root's or a split rounded to float, so it is within 2^-24 M of the exact halving of its own
 // level's bounds (M: the largest |coordinate| of the root box); those errors halve from level to
@@ -594,7 +743,10 @@ int launch_form(mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter,
     const double r2 = (double)r * (double)r;
     float r2f = (float)r2;
     if ((double)r2f > r2) r2f = nextafterf(r2f, 0.f);
-    k_ball_wave<FORM, KT><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
+    if constexpr (FORM == 0)
+      k_ball_wave<FORM, KT><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
+    else
+      k_ball_sums<FORM, KT><<<(m + kBallQ * (NBS / 64) - 1) / (kBallQ * (NBS / 64)), NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
   }
   LAUNCH_CHECK();
   return MLOD_OK;
