@@ -235,6 +235,31 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
   }
 }
 
+// add_mom as the (factor, value) pairs of its nine fused operations, in the order of the sums
+// (FP32 forms; the same roundings).
+template <int FORM, int KT, class KP>
+__device__ __forceinline__ void mom_pairs(float2* p, const KP& kp, const NodeMom<FORM>& mm, float Af, V3<float> q, float f) {
+  const float4 m0 = mm.m0, m1 = mm.m1;
+  if constexpr (FORM == 0) {
+    const float dx = m0.x / Af - q.x, dy = m0.y / Af - q.y, dz = m0.z / Af - q.z;
+    const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
+    p[0] = make_float2(w, Af);
+    p[1] = make_float2(w, m0.x), p[2] = make_float2(w, m0.y), p[3] = make_float2(w, m0.z);
+    p[4] = make_float2(w, m1.x), p[5] = make_float2(w, m1.y), p[6] = make_float2(w, m1.z);
+    p[7] = make_float2(w, m0.w), p[8] = make_float2(w, m1.w);
+  } else {
+    const float dx = m0.x - q.x, dy = m0.y - q.y, dz = m0.z - q.z;
+    const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
+    const float fw = __fmul_rn(f, weight32<KT>(kp, d2));
+    const float fa = __fmul_rn(fw, Af);
+    p[0] = make_float2(fw, Af);
+    p[1] = make_float2(fa, dx), p[2] = make_float2(fa, dy), p[3] = make_float2(fa, dz);
+    p[4] = make_float2(fw, m1.x), p[5] = make_float2(fw, m1.y), p[6] = make_float2(fw, m1.z);
+    p[7] = make_float2(fw, __fadd_rn(m0.w, fmaf(dz, m1.z, fmaf(dx, m1.x, __fmul_rn(dy, m1.y)))));
+    p[8] = make_float2(fw, fmaf(Af, d2, m1.w));
+  }
+}
+
 template <int FORM, int KT, class KP>
 __device__ __forceinline__ void add_node(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv, uint32_t c,
                                          float Af, V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
@@ -663,6 +688,253 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
   if constexpr (FORM == 1) acc.flush();
 }
 
+// ----------------------------------------------------------------------------- grouped walk (FP32 forms)
+// The same walk with eight lanes a query, for batches too small to fill the chip with a lane each.
+// There a step lasts as long as its longest walk: some 600 iterations of one dependent load each.
+// Here the children of a node are tested by the group's lanes at once, so a node costs one round
+// trip; what a near child needs to become the current node (its header and distance term) goes to the
+// group's LDS stack when it is found near; and the next node's loads are issued before the sums of the
+// last one are added.  The sums are the lane walk's to the bit: the children's terms go through LDS as
+// (factor, value) pairs and are added in slot order by one fused operation each, lane a of the group
+// adding sum a (and the even lanes the ninth), with the compensated form's block flushes after the same
+// terms.
+struct GroupNode {
+  uint32_t fn;    // first child, #children << 27
+  float dh, A;    // half its distance term; its area
+  uint32_t node;
+};
+constexpr uint32_t kGroup = 8;                 // lanes a query
+constexpr uint32_t kGroups = 64 / kGroup;      // queries a wavefront
+struct GroupLds {  // one wavefront
+  GroupNode wait[kLevels][64];                 // near children, per level: lane's slot
+  float2 pair[64][10];                         // a child's terms: nine sums, then (share, 1 - blend)
+  double sum[kGroups][9];
+  uint8_t mask[kLevels][kGroups];              // the level's children still to expand
+};
+
+// The sums of one lane of a group: partial sum and Kahan pair of sum `lane % 8` and, in the even
+// lanes, of the ninth.
+struct GroupSums {
+  float l0, l8;
+  KSum k0, k8;
+  uint32_t cnt;  // the walk's iterations since the last flush (compensated form)
+  __device__ __forceinline__ void init() { l0 = l8 = 0.f, k0.init(), k8.init(), cnt = 0; }
+  template <int FORM>
+  __device__ __forceinline__ void flush() {
+    if constexpr (FORM == 1) {
+      k0.add(l0), k8.add(l8);
+      l0 = l8 = 0.f;
+      cnt = 0;
+    }
+  }
+};
+
+// The partial sums as an accumulator whose nine sums all hold l, and back: a term added to it by
+// add_mom / add_point adds to every sum, of which the lane keeps its own.
+template <int FORM>
+__device__ __forceinline__ typename FormT<FORM>::Acc spread_sum(float l0, float l8) {
+  typename FormT<FORM>::Acc a;
+  if constexpr (FORM == 0) {
+    a.w = a.px = a.py = a.pz = a.nx = a.ny = a.nz = a.pn = l0, a.pp = l8;
+  } else {
+    a.lw = a.lpx = a.lpy = a.lpz = a.lnx = a.lny = a.lnz = a.lpn = l0, a.lpp = l8;
+  }
+  return a;
+}
+template <int FORM>
+__device__ __forceinline__ void pick_sum(const typename FormT<FORM>::Acc& a, uint32_t c, float& l0, float& l8) {
+  float v[9];
+  if constexpr (FORM == 0) {
+    v[0] = a.w, v[1] = a.px, v[2] = a.py, v[3] = a.pz, v[4] = a.nx, v[5] = a.ny, v[6] = a.nz, v[7] = a.pn, v[8] = a.pp;
+  } else {
+    v[0] = a.lw, v[1] = a.lpx, v[2] = a.lpy, v[3] = a.lpz, v[4] = a.lnx, v[5] = a.lny, v[6] = a.lnz, v[7] = a.lpn,
+    v[8] = a.lpp;
+  }
+  const float x = c & 1u ? v[1] : v[0], y = c & 1u ? v[3] : v[2], z = c & 1u ? v[5] : v[4], t = c & 1u ? v[7] : v[6];
+  const float u = c & 2u ? y : x, r = c & 2u ? t : z;
+  l0 = c & 4u ? r : u;
+  l8 = v[8];
+}
+
+struct Record {
+  float4 g;
+  uint4 h;
+  float4 m0, m1;
+};
+template <bool BIG>
+__device__ __forceinline__ Record load_record(const float4* rec, uint32_t idx) {
+  const char* r = reinterpret_cast<const char*>(rec);
+  const char* src = BIG ? r + (uint64_t)idx * 64u : r + (idx << 6);
+  return Record{reinterpret_cast<const float4*>(src)[0], reinterpret_cast<const uint4*>(src)[1],
+                reinterpret_cast<const float4*>(src)[2], reinterpret_cast<const float4*>(src)[3]};
+}
+
+template <int FORM, int SEM, int KT, bool BIG, class KP>
+__device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, const TreeView& tv, V3<float> q, float cutoff,
+                                               uint32_t minDepth, bool live, GroupLds& lds) {
+#pragma clang fp contract(off)  // the fused operations are written out
+  const uint32_t lane = __lane_id(), c = lane & (kGroup - 1u), grp = lane / kGroup, base = lane & ~(kGroup - 1u);
+  const float4* __restrict__ rec = FORM == 0 ? tv.recP : tv.recC;
+  Counters ct{0, 0, 0, 0, 0};
+  const uint4 h0 = tv.hdr[0];
+  const float4 g0 = tv.geo[0];
+  const float A0 = __uint_as_float(h0.z);
+  const auto single_term = [&](auto&& add) {  // a term added outside the group's exchange
+    auto a = spread_sum<FORM>(gs.l0, gs.l8);
+    add(a);
+    pick_sum<FORM>(a, c, gs.l0, gs.l8);
+  };
+  if (hdr_leaf(h0.y)) {  // a one-leaf tree (uniform)
+    if (live) single_term([&](auto& a) { add_leaf<FORM, SEM, KT, false>(a, kp, tv, h0, q, 1.f, ct); });
+    gs.template flush<FORM>();
+    return;
+  }
+  const int32_t blendKey = (int32_t)(min(minDepth, 15u) << 27);
+  uint32_t active = live ? 1u : 0u;
+  float dh = kNoBlend;
+  if (minDepth == 0) {
+    const float d0 = tdist<FORM>(q, g0), rc = g0.w * cutoff;
+    dh = 0.5f * fabsf(d0 - rc);
+    if (d0 > rc) {
+      if (live) single_term([&](auto& a) { add_node<FORM, KT>(a, kp, tv, 0, A0, q, 1.f); });
+      active = 0u;
+    }
+  }
+  // the current node of the group
+  uint32_t node = 0, first = h0.x, nc = active ? hdr_count(h0.y) : 0u, pend = 0, lvl = 0;
+  float Ai = A0;
+  Record next = load_record<BIG>(rec, first + (c < nc ? c : 0u));  // the lane's child
+  NodeMom<FORM> own = load_mom<FORM>(tv, node);
+  while (any_lane(active != 0u)) {
+    const float4 g = next.g;
+    const uint4 h = next.h;
+    NodeMom<FORM> mm;
+    mm.m0 = next.m0;
+    mm.m1 = next.m1;
+    // the node that is summed below
+    const uint32_t ncP = nc;
+    const float AiP = Ai, dhP = dh;
+    const NodeMom<FORM> ownP = own;
+    const bool mineP = c < ncP, activeP = active != 0u;
+    // --- near children, and the next node
+    const float over = tdist<FORM>(q, g) - g.w * cutoff;
+    const bool leaf = (int32_t)h.y < 0, single = h.y >= (kLeafBit | kSingleBit);
+    const bool far = (int32_t)h.y >= blendKey && over > 0.f;
+    const bool near = mineP && !leaf && !far;
+    const float At = __uint_as_float(h.z);
+    uint32_t bits = (uint32_t)(__builtin_amdgcn_ballot_w64(near) >> base) & 0xffu, L = lvl;
+    if (near)
+      lds.wait[lvl][lane] = GroupNode{h.x | (h.y & 15u) << 27, (int32_t)h.y >= blendKey ? 0.5f * fabsf(over) : kNoBlend, At,
+                                      first + c};
+    if (activeP) {
+      if (bits) {
+        if (bits & (bits - 1u)) pend |= 1u << lvl;
+      } else if (pend) {
+        L = 31u - (uint32_t)__builtin_clz(pend);
+        bits = lds.mask[L][grp];
+      } else {
+        active = 0u;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // records read, near children written
+    nc = 0u;
+    if (active) {
+      const uint32_t k = (uint32_t)__builtin_ctz(bits), rest = bits & (bits - 1u);
+      const GroupNode e = lds.wait[L][base + k];
+      lds.mask[L][grp] = (uint8_t)rest;
+      if (!rest) pend &= ~(1u << L);
+      node = e.node;
+      first = e.fn & kCountMask;
+      nc = e.fn >> 27;
+      dh = e.dh;
+      Ai = e.A;
+      lvl = L + 1u;
+    }
+    next = load_record<BIG>(rec, first + (c < nc ? c : 0u));
+    own = load_mom<FORM>(tv, node);
+    // --- the sums of the node that was tested
+    const float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
+    const float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)ncP) : tratio<FORM>(1.f, AiP);
+    const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : At / AiP);
+    const bool contrib = mineP && (far || single), multi = mineP && leaf && !single;
+    {
+      float2 p[10];
+#pragma unroll
+      for (int t = 0; t < 10; ++t) p[t] = make_float2(0.f, 0.f);
+      if (contrib) mom_pairs<FORM, KT>(p, kp, mm, At, q, f);
+      if (mineP) p[9] = make_float2(share, 1.f - f);
+      float4* out = reinterpret_cast<float4*>(lds.pair[lane]);
+#pragma unroll
+      for (int t = 0; t < 5; ++t) out[t] = make_float4(p[2 * t].x, p[2 * t].y, p[2 * t + 1].x, p[2 * t + 1].y);
+    }
+    float shareSum = 0.f;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // the compensated form's flush falls before child `due` (after the last one when that is their number)
+    const uint32_t terms = gs.cnt + ncP, due = terms >= kFlush ? kFlush - gs.cnt : ~0u;
+    static_assert(kFlush == kGroup, "at most one flush among a node's children");
+    if (!any_lane(multi)) {  // uniform
+      // lane c's second chain is the ninth sum in even lanes, the share sum in odd ones
+      const bool odd = c & 1u;
+      float2 x[kGroup], y[kGroup];
+#pragma unroll
+      for (uint32_t j = 0; j < kGroup; ++j) {  // (children past the last hold zeros)
+        x[j] = lds.pair[base + j][c];
+        y[j] = lds.pair[base + j][8u + (c & 1u)];
+      }
+      float l0 = gs.l0, l1 = odd ? 0.f : gs.l8, b0 = 0.f, b1 = 0.f;  // b: the block that is complete, if one is
+#pragma unroll
+      for (uint32_t j = 0; j <= kGroup; ++j) {
+        if constexpr (FORM == 1) {
+          if (j > 0) {
+            const bool full = j == due;
+            b0 = full ? l0 : b0;
+            l0 = full ? 0.f : l0;
+            b1 = full ? l1 : b1;
+            l1 = full && !odd ? 0.f : l1;
+          }
+        }
+        if (j < kGroup) {
+          l0 = fmaf(x[j].x, x[j].y, l0);
+          l1 = fmaf(y[j].x, y[j].y, l1);
+        }
+      }
+      shareSum = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(l1), 0xf5, 0xf, 0xf, true));  // lane | 1 of the quad
+      gs.l0 = l0;
+      gs.l8 = odd ? gs.l8 : l1;
+      if constexpr (FORM == 1) {
+        if (due != ~0u) gs.k0.add(b0), gs.k8.add(b1);
+      }
+    } else {  // a leaf of several points among the children (at the last level, or by the build's option)
+#pragma unroll 1
+      for (uint32_t j = 0; j < kGroup; ++j) {
+        if constexpr (FORM == 1) {
+          if (j > 0 && j == due) gs.template flush<FORM>();
+        }
+        const float2 x = lds.pair[base + j][c];
+        const float4 y = *reinterpret_cast<const float4*>(lds.pair[base + j] + 8);
+        gs.l0 = fmaf(x.x, x.y, gs.l0);
+        gs.l8 = fmaf(y.x, y.y, gs.l8);
+        shareSum = fmaf(y.z, y.w, shareSum);
+        const uint4 hj = make_uint4((uint32_t)__shfl((int)h.x, (int)(base + j), 64), (uint32_t)__shfl((int)h.y, (int)(base + j), 64), 0u, 0u);
+        const float fj = __shfl(f, (int)(base + j), 64);
+        const bool mj = __shfl((int)multi, (int)(base + j), 64) != 0;
+        if (mj) single_term([&](auto& t) { add_leaf<FORM, SEM, KT, false>(t, kp, tv, hj, q, fj, ct); });
+      }
+      if constexpr (FORM == 1) {
+        if (due == kGroup) gs.template flush<FORM>();
+      }
+    }
+    if constexpr (FORM == 1) gs.cnt = terms >= kFlush ? terms - kFlush : terms;
+    if (activeP) {
+      if (shareSum != 0.f) single_term([&](auto& x) { add_mom<FORM, KT>(x, kp, ownP, AiP, q, shareSum); });
+      if constexpr (FORM == 1) {
+        if (++gs.cnt == kFlush) gs.template flush<FORM>();
+      }
+    }
+  }
+  gs.template flush<FORM>();
+}
+
 // The LDS of one workgroup's walks: the stacks of waiting nodes (5 B a level and lane in the FP32
 // forms) and the wavefronts' staging rows (15.4 KB: ten workgroups a CU, five waves per SIMD), or the
 // FP64 form's stacks.
@@ -998,33 +1270,41 @@ __device__ __forceinline__ void fit(T sw, V3<T> sp, V3<T> sn, T spn, T spp, V3<T
   outN = nr;
 }
 
-// One projection step of query q (double carried between steps).
+// One projection step of query q (double carried between steps) from the nine sums: the global frame's
+// for the plain forms, the query frame's for the compensated one.
+template <int FORM, int SEM>
+__device__ __forceinline__ void fit_total(const double* S, V3<double>& qd, V3<float> qf, float stepMax, float4& nout) {
+  float kind;
+  if constexpr (FORM == 0) {
+    V3<float> p, n;
+    fit<float, float, SEM>((float)S[0], V3<float>{(float)S[1], (float)S[2], (float)S[3]},
+                           V3<float>{(float)S[4], (float)S[5], (float)S[6]}, (float)S[7], (float)S[8], qf, stepMax, p, n, kind);
+    qd = V3<double>{p.x, p.y, p.z};
+    nout = make_float4(n.x, n.y, n.z, kind);
+  } else {
+    V3<double> p, n;
+    if constexpr (FORM == 1) {  // the query is the origin
+      fit<double, double, SEM, true>(S[0], V3<double>{S[1], S[2], S[3]}, V3<double>{S[4], S[5], S[6]}, S[7], S[8],
+                                     V3<double>{0, 0, 0}, (double)stepMax, p, n, kind);
+      qd = V3<double>{(double)qf.x + p.x, (double)qf.y + p.y, (double)qf.z + p.z};
+    } else {
+      fit<double, double, SEM>(S[0], V3<double>{S[1], S[2], S[3]}, V3<double>{S[4], S[5], S[6]}, S[7], S[8], qd,
+                               (double)stepMax, p, n, kind);
+      qd = p;
+    }
+    nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+  }
+}
 template <int FORM, int SEM>
 __device__ __forceinline__ void fit_step(const typename FormT<FORM>::Acc& acc, V3<double>& qd, V3<float> qf, float stepMax,
                                          float4& nout) {
-  if constexpr (FORM == 0) {
-    V3<float> p, n;
-    float kind;
-    fit<float, float, SEM>(acc.w, V3<float>{acc.px, acc.py, acc.pz}, V3<float>{acc.nx, acc.ny, acc.nz}, acc.pn, acc.pp, qf,
-                           stepMax, p, n, kind);
-    qd = V3<double>{p.x, p.y, p.z};
-    nout = make_float4(n.x, n.y, n.z, kind);
-  } else if constexpr (FORM == 1) {
-    // query frame: the query is the origin
-    V3<double> p, n;
-    float kind;
-    fit<double, double, SEM, true>(acc.w.val(), V3<double>{acc.px.val(), acc.py.val(), acc.pz.val()},
-                             V3<double>{acc.nx.val(), acc.ny.val(), acc.nz.val()}, acc.pn.val(), acc.pp.val(),
-                             V3<double>{0, 0, 0}, (double)stepMax, p, n, kind);
-    qd = V3<double>{(double)qf.x + p.x, (double)qf.y + p.y, (double)qf.z + p.z};
-    nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+  if constexpr (FORM == 1) {
+    const double S[9] = {acc.w.val(),  acc.px.val(), acc.py.val(), acc.pz.val(), acc.nx.val(),
+                         acc.ny.val(), acc.nz.val(), acc.pn.val(), acc.pp.val()};
+    fit_total<1, SEM>(S, qd, qf, stepMax, nout);
   } else {
-    V3<double> p, n;
-    float kind;
-    fit<double, double, SEM>(acc.w, V3<double>{acc.px, acc.py, acc.pz}, V3<double>{acc.nx, acc.ny, acc.nz}, acc.pn, acc.pp,
-                             qd, (double)stepMax, p, n, kind);
-    qd = p;
-    nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+    const double S[9] = {acc.w, acc.px, acc.py, acc.pz, acc.nx, acc.ny, acc.nz, acc.pn, acc.pp};
+    fit_total<FORM, SEM>(S, qd, qf, stepMax, nout);
   }
 }
 
@@ -1077,6 +1357,45 @@ __global__ __launch_bounds__(PBS) void k_project(TreeView tv, KParams kp, float4
       atomicAdd(&counters[4], (unsigned long long)ct.iters);
     }
     if (__lane_id() == 0) atomicAdd(&counters[5], (unsigned long long)wmax);
+  }
+}
+
+// k_project with the grouped walk: a wavefront projects 8 queries, one wavefront a workgroup.  Bound by
+// the latency of its own instructions (about 400 a node): 1k queries, three steps, 60k points: 1.77 -> 0.49
+// ms.  With the records staged through LDS as in the lane walk it took 0.57: the compiler then holds the
+// exchange back until the staging loads are in.
+template <int FORM, int SEM, int KT>
+__global__ __launch_bounds__(64) void k_project_group(TreeView tv, KParams kp, float4* __restrict__ q,
+                                                      float4* __restrict__ qn, const uint32_t* __restrict__ perm,
+                                                      uint32_t m, uint32_t limit, uint32_t nIter, float stepMax,
+                                                      float cutoff, uint32_t minDepth) {
+  __shared__ GroupLds lds;
+  const uint32_t lane = threadIdx.x, c = lane & (kGroup - 1u), grp = lane / kGroup;
+  const uint32_t i = xcd_block() * kGroups + grp;
+  const bool live = i < m && !(limit < m && perm[i] >= limit);
+  if (!any_lane(live)) return;
+  const float4 q4 = live ? q[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  V3<double> qd{q4.x, q4.y, q4.z};
+  float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (uint32_t it = 0; it < nIter; ++it) {
+    GroupSums gs;
+    gs.init();
+    const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
+    if (tv.nn < (1u << 26))
+      traverse_group<FORM, SEM, KT, false>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
+    else
+      traverse_group<FORM, SEM, KT, true>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
+    lds.sum[grp][c] = FORM == 0 ? (double)gs.l0 : gs.k0.val();
+    if (c == 0) lds.sum[grp][8] = FORM == 0 ? (double)gs.l8 : gs.k8.val();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    double S[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) S[t] = lds.sum[grp][t];
+    fit_total<FORM, SEM>(S, qd, qf, stepMax, nout);
+  }
+  if (live && c == 0) {
+    q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
+    qn[i] = nout;
   }
 }
 
@@ -1141,16 +1460,11 @@ __device__ __forceinline__ void fit_sums(const double* S, V3<double>& qd, float 
   const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
   if constexpr (FORM == 1) {
     const V3<double> q{qf.x, qf.y, qf.z}, sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
-    V3<double> p, n;
-    float kind;
-    fit<double, double, SEM, true>(S[0], V3<double>{sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0]}, sn,
-                                   S[7] - dot3(q, sn), S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0], V3<double>{0, 0, 0},
-                                   (double)stepMax, p, n, kind);
-    qd = V3<double>{q.x + p.x, q.y + p.y, q.z + p.z};
-    nout = make_float4((float)n.x, (float)n.y, (float)n.z, kind);
+    const double R[9] = {S[0], sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0], sn.x, sn.y, sn.z, S[7] - dot3(q, sn),
+                         S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0]};
+    fit_total<1, SEM>(R, qd, qf, stepMax, nout);
   } else {
-    AccP64 a{S[0], S[1], S[2], S[3], S[4], S[5], S[6], S[7], S[8]};
-    fit_step<2, SEM>(a, qd, qf, stepMax, nout);
+    fit_total<FORM, SEM>(S, qd, qf, stepMax, nout);
   }
 }
 
@@ -1392,6 +1706,13 @@ void launch_batch_all(const ReqDesc* r, const uint2* blocks, uint32_t nblk, floa
   k_project_batch<FORM, SEM, -1><<<nblk, PBS, 0, s>>>(r, blocks, q, qn, qd, bo, prio);
 }
 
+// Batches of at most this many queries take the grouped walk: it issues three times the instructions of
+// the lane walk and is done in a third of its time while the chip has room for them.  Three steps on 1M
+// points, four sigmas, FP32C, us with a lane / a group: 4k queries 1283 / 427, 16k 1315 / 530, 32k
+// 1318 / 884, 48k 1428 / 1186, 64k 1452 / 1473; plain FP32, rational, cutoff 3: 32k 3533 / 2045, 64k
+// 3789 / 3514.
+constexpr uint32_t kGroupMax = 49152;
+
 template <int FORM, int SEM, int KT, bool CNT>
 int launch_one(const mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter, float stepMax,
                unsigned long long* counters, hipStream_t s) {
@@ -1400,6 +1721,9 @@ int launch_one(const mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t n
   if (t->traversal == MLOD_TRAVERSAL_WAVE)
     k_project_wave<FORM, SEM, KT, CNT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(
         t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth, counters);
+  else if (FORM != 2 && !CNT && m <= kGroupMax)
+    k_project_group<FORM == 2 ? 1 : FORM, SEM, KT><<<(m + kGroups - 1) / kGroups, 64, 0, s>>>(
+        t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth);
   else
     k_project<FORM, SEM, KT, CNT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m,
                                                                        limit, nIter, stepMax, t->cutoff, t->min_depth,

@@ -1,6 +1,7 @@
-"""The FP32 forms' walk with node records staged through LDS: ragged query counts (lanes without a query
-beside lanes that have one), multi-point leaves, trees of one leaf and of one level, min depths on both sides
-of the tree's depth, and a tree of 2^26 nodes or more (64-bit record offsets)."""
+"""The FP32 forms' walks, one lane a query with node records staged through LDS and, for small batches, eight lanes a
+query: the same bits from both, ragged query counts (lanes without a query beside lanes that have one), multi-point
+leaves, trees of one leaf and of one level, min depths on both sides of the tree's depth, and a tree of 2^26 nodes
+or more (64-bit record offsets)."""
 import numpy as np
 import pytest
 
@@ -54,6 +55,31 @@ def test_leaf_and_level_edges(cloud, max_depth, leaf, min_depth, semantics):
         assert out["fp32c"].shape == out["fp64"].shape
 
 
+KERNELS = {"mg": dict(type=2, sigmas=[0.03, 0.06, 0.12]), "mg11": dict(type=2, sigmas=[0.02 * 1.3 ** i for i in range(11)]),
+           "rat": dict(type=1, exponent=4.0, constant_shift=1e-3), "gauss": dict(type=0, sigma=0.1)}
+
+
+@pytest.mark.parametrize("kernel", sorted(KERNELS))
+@pytest.mark.parametrize("precision", ["fp32", "fp32c"])
+@pytest.mark.parametrize("semantics", ["ref_gpu", "ref_cpu"])
+@pytest.mark.parametrize("max_depth,leaf,min_depth,cutoff", [(12, 1, 0, 2.0), (5, 1, 0, 1.4), (12, 9, 1, 3.0), (3, 1, 2, 2.0)])
+def test_lane_and_group_walks_give_the_same_bits(cloud, kernel, precision, semantics, max_depth, leaf, min_depth, cutoff):
+    """60000 queries take a lane each, 999 of them a group of eight; some lie beyond every cutoff."""
+    p, n, _, _ = cloud
+    t = A.APSSOctree().build(p, n, maxDepth=max_depth, maxNumberOfPointsPerLeaf=leaf)
+    q = ds.jitter_queries(np.tile(p, (3, 1)), 0.03, seed=24)
+    q[::100] *= 4.0
+    ap = A.Fastapss(t, A.Kernel(**KERNELS[kernel]))
+    ap.setScalingProtectionSphere(cutoff)
+    ap.setMinDepth(min_depth)
+    ap.set_precision(precision)
+    ap.set_semantics(semantics)
+    ref = ap.project_points(q, 2)
+    got = ap.project_points(q[:999], 2)
+    for g, r in zip(got, ref):
+        assert np.array_equal(g.view(np.int32), r[:999].view(np.int32))
+
+
 def test_records_beyond_32_bit_offsets():
     """18M pairs of near points: a chain of nodes for each pair, so the tree has more than 2^26 nodes."""
     rng = np.random.default_rng(31)
@@ -71,3 +97,5 @@ def test_records_beyond_32_bit_offsets():
     diag = 2 * t.radius()
     assert np.abs(out["fp32c"] - out["fp64"]).max() <= 1e-6 * diag
     assert np.abs(out["fp32"] - out["fp64"]).max() <= 1e-5 * diag
+    many = np.tile(q, (26, 1))  # a lane a query
+    assert np.array_equal(_plugin(t, sig, "fp32c").project_points(many, 1)[0][:2000], out["fp32c"])
