@@ -23,6 +23,7 @@
 //   6. node moments bottom-up, one depth per launch: plain FP32 sums in the reference's
 //      order (leaf points in input order, children in slot order, CPUUtils.cpp:358-398),
 //      the same in FP64, and node-centred moments for the precision form.
+#include <cfloat>
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -577,9 +578,12 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
   float4* rc = recC + 4 * (uint64_t)k;
   rp[0] = g;
   // the walk's header: a leaf's depth gives way to a flag for a leaf of one point, the father to the
-  // reciprocal of A (rounded as a division for the plain form, the hardware's for the other)
+  // reciprocal of A (correctly rounded for the plain form, held finite for a subnormal A, since quotients
+  // by A are formed from it; the hardware's for the other)
   const uint32_t code = !hdr_leaf(h.y) ? h.y : kLeafBit | (cnt == 1 ? kSingleBit : 0u) | cnt;
-  reinterpret_cast<uint4*>(rp)[1] = make_uint4(first, code, h.z, __float_as_uint((float)(1.0 / (double)sf.a)));
+  const double rA = 1.0 / (double)sf.a;
+  reinterpret_cast<uint4*>(rp)[1] =
+      make_uint4(first, code, h.z, __float_as_uint(sf.a > 0.f && rA > (double)FLT_MAX ? FLT_MAX : (float)rA));
   rp[2] = make_float4(sf.px, sf.py, sf.pz, sf.pn);
   rp[3] = make_float4(sf.nx, sf.ny, sf.nz, sf.pp);
   rc[0] = g;

@@ -116,7 +116,7 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
   if constexpr (FORM == 0) {
     const float a = P.w;
     const float apx = a * P.x, apy = a * P.y, apz = a * P.z;
-    const float dx = apx / a - q.x, dy = apy / a - q.y, dz = apz / a - q.z;
+    const float dx = quot(apx, a) - q.x, dy = quot(apy, a) - q.y, dz = quot(apz, a) - q.z;
     const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     acc.w = fmaf(w, a, acc.w);
     acc.px = fmaf(w, apx, acc.px);
@@ -162,6 +162,7 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
 // Moments of one node as loaded from HBM (node-centred FP32 for the compensated form,
 // global-frame FP32 for the plain form, FP64 for the FP64 form).
 template <int FORM> struct NodeMom { float4 m0, m1; };
+template <> struct NodeMom<0> { float4 m0, m1; float rA; };  // rA = 1 / A, correctly rounded
 template <> struct NodeMom<2> { double4 m0, m1; double A; };
 
 // Record `idx` of `bytes` bytes from `base`, with the byte offset formed in 32 bits (the tree
@@ -177,6 +178,7 @@ __device__ __forceinline__ NodeMom<FORM> load_mom(const TreeView& tv, uint32_t c
   NodeMom<FORM> r;
   if constexpr (FORM == 0) {
     r.m0 = tv.recP[4 * (size_t)c + 2], r.m1 = tv.recP[4 * (size_t)c + 3];
+    r.rA = tv.recP[4 * (size_t)c + 1].w;
   } else if constexpr (FORM == 1) {
     r.m0 = tv.recC[4 * (size_t)c + 2], r.m1 = tv.recC[4 * (size_t)c + 3];
   } else {
@@ -192,7 +194,8 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
                                         V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
   if constexpr (FORM == 0) {
     const float4 m0 = mm.m0, m1 = mm.m1;
-    const float dx = m0.x / Af - q.x, dy = m0.y / Af - q.y, dz = m0.z / Af - q.z;
+    const float dx = quot_rcp(m0.x, Af, mm.rA) - q.x, dy = quot_rcp(m0.y, Af, mm.rA) - q.y,
+                dz = quot_rcp(m0.z, Af, mm.rA) - q.z;
     const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     acc.w = fmaf(w, Af, acc.w);
     acc.px = fmaf(w, m0.x, acc.px);
@@ -241,7 +244,8 @@ template <int FORM, int KT, class KP>
 __device__ __forceinline__ void mom_pairs(float2* p, const KP& kp, const NodeMom<FORM>& mm, float Af, V3<float> q, float f) {
   const float4 m0 = mm.m0, m1 = mm.m1;
   if constexpr (FORM == 0) {
-    const float dx = m0.x / Af - q.x, dy = m0.y / Af - q.y, dz = m0.z / Af - q.z;
+    const float dx = quot_rcp(m0.x, Af, mm.rA) - q.x, dy = quot_rcp(m0.y, Af, mm.rA) - q.y,
+                dz = quot_rcp(m0.z, Af, mm.rA) - q.z;
     const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     p[0] = make_float2(w, Af);
     p[1] = make_float2(w, m0.x), p[2] = make_float2(w, m0.y), p[3] = make_float2(w, m0.z);
@@ -287,15 +291,15 @@ __device__ __forceinline__ T dist3(V3<T> q, float4 g) {
   return fsqrt(dx * dx + dy * dy + dz * dz);
 }
 
-// Traversal arithmetic per form.  The plain forms keep IEEE division and square root (the
-// reference's arithmetic); the compensated form, whose error budget is set by its FP64 fit and
+// Traversal arithmetic per form.  The plain forms keep correctly rounded division and square root
+// (the reference's arithmetic); the compensated form, whose error budget is set by its FP64 fit and
 // compensated sums, takes the hardware reciprocal and square root (1 ulp).
 template <int FORM>
 __device__ __forceinline__ typename FormT<FORM>::T tdist(V3<typename FormT<FORM>::T> q, float4 g) {
   if constexpr (FORM != 2) {  // (the fused operations written out: every kernel rounds alike)
     const float dx = q.x - g.x, dy = q.y - g.y, dz = q.z - g.z;
     const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
-    return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : fsqrt(d2);
+    return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : root(d2);
   } else {
     return dist3(q, g);
   }
@@ -304,6 +308,8 @@ template <int FORM, class T>
 __device__ __forceinline__ T tratio(T a, T b) {  // a / b
   if constexpr (FORM == 1)
     return a * __builtin_amdgcn_rcpf(b);
+  else if constexpr (FORM == 0)
+    return quot(a, b);
   else
     return a / b;
 }
@@ -510,7 +516,8 @@ __device__ __forceinline__ void traverse_loads(typename FormT<FORM>::Acc& acc, c
 // 100 % busy, 131 an iteration against 152 before: no multiplier, reciprocals of A kept in the
 // records, one stack access an iteration), and the smaller stacks let five waves run per SIMD against
 // four.  8M points, 8M queries, six sigmas, FP32C: 20.6 -> 16.5 ms a step; 1M points and queries,
-// rational kernel, plain FP32: 11.7 -> 10.0; 100k queries x 10 steps on 1M points: 5.5 -> 4.8.
+// rational kernel, plain FP32: 11.7 -> 10.0 (8.1 with the quotients and roots of
+// weights.h); 100k queries x 10 steps on 1M points: 5.5 -> 4.8.
 // (Four waves per SIMD, with the stacks one word a level longer, left the step at 20.6 ms.)
 constexpr uint32_t kStageRow = 1024 + 16;
 constexpr uint32_t kStageBytes = 4 * kStageRow;  // per wavefront
@@ -656,6 +663,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       NodeMom<FORM> mm;
       mm.m0 = *reinterpret_cast<const float4*>(mine + 32);
       mm.m1 = *reinterpret_cast<const float4*>(mine + 48);
+      if constexpr (FORM == 0) mm.rA = __uint_as_float(h.w);
       const float At = __uint_as_float(h.z);
       bool multi = false;
       if (testing) {
@@ -663,7 +671,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
         const float over = tdist<FORM>(q, g) - g.w * cutoff;
         const float dc = fmaxf(over, 0.f);
         f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
-        const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : At / Ai);
+        const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : quot_rcp(At, Ai, scale));
         shareSum = fmaf(share, 1.f - f, shareSum);
         const bool leaf = (int32_t)h.y < 0;
         const bool single = h.y >= (kLeafBit | kSingleBit);
@@ -811,6 +819,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     NodeMom<FORM> mm;
     mm.m0 = next.m0;
     mm.m1 = next.m1;
+    if constexpr (FORM == 0) mm.rA = __uint_as_float(h.w);
     // the node that is summed below
     const uint32_t ncP = nc;
     const float AiP = Ai, dhP = dh;
@@ -854,8 +863,13 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     own = load_mom<FORM>(tv, node);
     // --- the sums of the node that was tested
     const float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
-    const float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)ncP) : tratio<FORM>(1.f, AiP);
-    const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : At / AiP);
+    float share;
+    if constexpr (SEM == MLOD_SEM_REF_CPU)
+      share = tratio<FORM>(1.f, (float)ncP);
+    else if constexpr (FORM == 1)
+      share = At * tratio<FORM>(1.f, AiP);
+    else
+      share = quot_rcp(At, AiP, ownP.rA);
     const bool contrib = mineP && (far || single), multi = mineP && leaf && !single;
     {
       float2 p[10];
@@ -1013,6 +1027,7 @@ __device__ __forceinline__ NodeMom<FORM> load_mom_uni(const TreeView& tv, uint32
   NodeMom<FORM> r;
   if constexpr (FORM == 0) {
     r.m0 = ld_uni(tv.recP, 4 * c + 2), r.m1 = ld_uni(tv.recP, 4 * c + 3);
+    r.rA = ld_uni(tv.recP, 4 * c + 1).w;
   } else if constexpr (FORM == 1) {
     r.m0 = ld_uni(tv.recC, 4 * c + 2), r.m1 = ld_uni(tv.recC, 4 * c + 3);
   } else {

@@ -99,3 +99,16 @@ def test_records_beyond_32_bit_offsets():
     assert np.abs(out["fp32"] - out["fp64"]).max() <= 1e-5 * diag
     many = np.tile(q, (26, 1))  # a lane a query
     assert np.array_equal(_plugin(t, sig, "fp32c").project_points(many, 1)[0][:2000], out["fp32c"])
+
+
+@pytest.mark.parametrize("k", [-16, 16])
+@pytest.mark.parametrize("m", [999, 60000])
+def test_plain_form_scales_exactly(cloud, k, m):
+    """A cloud scaled by a power of two goes through the same roundings: its walk's quotients by the nodes' areas,
+    blend ratios and square roots are right at every exponent, so the results scale to the bit."""
+    p, n, sig, _ = cloud
+    s = np.float32(2.0) ** k
+    q = ds.jitter_queries(np.tile(p, (3, 1)), 0.02, seed=25)[:m]
+    got = [_plugin(A.APSSOctree().build(p * f, n), [float(np.float32(x) * f) for x in sig], "fp32").project_points(q * f, 2)
+           for f in (np.float32(1.0), s)]
+    assert np.array_equal(got[0][0] * s, got[1][0]) and np.array_equal(got[0][1], got[1][1])
