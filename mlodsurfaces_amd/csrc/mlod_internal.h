@@ -68,8 +68,9 @@ struct alignas(16) KParams {
   float c;           // constant_shift
   float cp;          // max(c, 1e-4)
   float e;           // exponent
-  double ad[MLOD_MAX_SIGMAS];  // FP64: -1 / (2 s^2)
-  double bd[MLOD_MAX_SIGMAS];  // FP64: 1 / s^3
+  double ad[MLOD_MAX_SIGMAS + 1];  // FP64: -log2(e) / (2 s^2)  (read two at a time)
+  double bd[MLOD_MAX_SIGMAS + 1];  // FP64: 1 / s^3
+  double cpe;        // FP64: cp^e
 };
 
 // One run of a serving step launch (a resident range of one request's queries): its tree,

@@ -556,8 +556,8 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its wavefront's other
 // queries.  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
 // ones.  r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k 1.3;
-// FP64, 100k queries 1.6.  Wavefronts of 64 queries (unions of four times the surface, four times fewer
-// wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
+// FP64, 100k queries 1.6 (1.3 with weights.h's exponential).  Wavefronts of 64 queries (unions of four
+// times the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
 constexpr uint32_t kBallQ = 16;            // queries a wavefront
 constexpr uint32_t kScanPointsBall = 512;  // subtrees up to this size are taken as one range (256: 1.65 ms, 1024: 1.57)
 

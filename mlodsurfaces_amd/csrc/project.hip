@@ -11,7 +11,7 @@
 // the blend factors on its path and adds m * (its own term) to one accumulator.  That needs
 // no per-depth accumulator stack (the reference keeps 12 of them per thread); the per-lane
 // traversal state is, per depth level, the first child and a mask of children still to descend,
-// held in LDS (the FP64 form keeps the node's multiplier and distance term too).  A near node
+// held in LDS.  A near node
 // loops over its contiguous children once: far children and leaves are summed right there, the
 // parent's (1 - b_c) share is accumulated, and only near internal children are left in the mask.
 //
@@ -47,7 +47,22 @@ constexpr int kLevels = kMaxDepth - 1;
 // Level blending (1 - cos(pi x)) / 2 (CPUUtils.cpp:400-408, Fastapss.cu:84-95).  The FP32
 // form uses the hardware cosine, which takes revolutions: cos(pi x) = cos_rev(x / 2).
 __device__ __forceinline__ float blend(float x) { return 0.5f - 0.5f * __builtin_amdgcn_cosf(0.5f * x); }
-__device__ __forceinline__ double blend(double x) { return (1.0 - cos(3.14159265 * x)) * 0.5; }
+// In FP64 (x in [0, 1], 3.14159265 x as the reference has it): (1 + sin(u)) / 2 with u = 3.14159265 x - pi/2, the
+// Taylor series of the sine to the 21st power (remainder 1.3e-18 at |u| = pi/2).  Exactly 1 at x = 1.
+__device__ __forceinline__ double blend(double x) {
+  const double u = fma(x, 3.14159265, -1.5707963267948966), z = u * u;
+  double p = 1.9572941063391263e-20;
+  p = fma(p, z, -8.22063524662433e-18);
+  p = fma(p, z, 2.8114572543455206e-15);
+  p = fma(p, z, -7.647163731819816e-13);
+  p = fma(p, z, 1.6059043836821613e-10);
+  p = fma(p, z, -2.505210838544172e-08);
+  p = fma(p, z, 2.7557319223985893e-06);
+  p = fma(p, z, -0.0001984126984126984);
+  p = fma(p, z, 0.008333333333333333);
+  p = fma(p, z, -0.16666666666666666);
+  return fma(0.5, fma(u * z, p, u), 0.5);
+}
 
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_sqrtf(x); }
 __device__ __forceinline__ double fsqrt(double x) { return sqrt(x); }
@@ -145,7 +160,8 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
   } else {
     const double a = P.w, x = P.x, y = P.y, z = P.z;
     const double apx = a * x, apy = a * y, apz = a * z;
-    const double dx = apx / a - q.x, dy = apy / a - q.y, dz = apz / a - q.z;
+    const double ra = near_rcp(a);
+    const double dx = quot_rcp(apx, a, ra) - q.x, dy = quot_rcp(apy, a, ra) - q.y, dz = quot_rcp(apz, a, ra) - q.z;
     const double w = f * weight64<KT>(kp, dx * dx + dy * dy + dz * dz);
     acc.w += w * a;
     acc.px += w * apx;
@@ -224,7 +240,8 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
   } else {
     const double4 m0 = mm.m0, m1 = mm.m1;
     const double A = mm.A;
-    const double dx = m0.x / A - q.x, dy = m0.y / A - q.y, dz = m0.z / A - q.z;
+    const double rA = near_rcp(A);
+    const double dx = quot_rcp(m0.x, A, rA) - q.x, dy = quot_rcp(m0.y, A, rA) - q.y, dz = quot_rcp(m0.z, A, rA) - q.z;
     const double w = f * weight64<KT>(kp, dx * dx + dy * dy + dz * dz);
     acc.w += w * A;
     acc.px += w * m0.x;
@@ -285,12 +302,6 @@ __device__ __forceinline__ void add_leaf(typename FormT<FORM>::Acc& acc, const K
   }
 }
 
-template <class T>
-__device__ __forceinline__ T dist3(V3<T> q, float4 g) {
-  const T dx = q.x - (T)g.x, dy = q.y - (T)g.y, dz = q.z - (T)g.z;
-  return fsqrt(dx * dx + dy * dy + dz * dz);
-}
-
 // Traversal arithmetic per form.  The plain forms keep correctly rounded division and square root
 // (the reference's arithmetic); the compensated form, whose error budget is set by its FP64 fit and
 // compensated sums, takes the hardware reciprocal and square root (1 ulp).
@@ -301,206 +312,131 @@ __device__ __forceinline__ typename FormT<FORM>::T tdist(V3<typename FormT<FORM>
     const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
     return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : root(d2);
   } else {
-    return dist3(q, g);
+    const double dx = q.x - (double)g.x, dy = q.y - (double)g.y, dz = q.z - (double)g.z;
+    return root(dx * dx + dy * dy + dz * dz);
   }
 }
 template <int FORM, class T>
 __device__ __forceinline__ T tratio(T a, T b) {  // a / b
   if constexpr (FORM == 1)
     return a * __builtin_amdgcn_rcpf(b);
-  else if constexpr (FORM == 0)
-    return quot(a, b);
   else
-    return a / b;
+    return quot(a, b);
 }
 
-// A node whose near children wait, per level and lane: what its next near child needs to start
-// (the node's first child, multiplier and distance term), so a lane resumes it without reloading it.
-template <class T>
-struct LevelState {
-  uint32_t (*first)[PBS];  // the node's first child
-  uint8_t (*mask)[PBS];    // its near children still to expand
-  T (*mul)[PBS];           // its multiplier
-  T (*dist)[PBS];          // its distance term |d - cutoff r| (negative: no blending below it)
+// A node with near children still to expand, per level and lane: its first child, and those children.
+struct WalkStack {
+  uint32_t (*first)[PBS];
+  uint8_t (*mask)[PBS];
 };
 
-// Flattened traversal (the FP64 form's; traverse_staged is the FP32 forms').  The lane's current node (expanded: near, or above minDepth) has its
-// children tested one per loop iteration; when they are done the node's own (1 - b_c) share
-// is added and its first near child becomes the current node.  Either way an iteration handles
-// exactly one node X: it loads X, computes its distance and its blend factor against its
-// parent, then either classifies X as a child (far / leaf / near) or makes it the current node,
-// and ends in one shared node contribution.  Lanes of a wavefront therefore advance by one node
-// per iteration whatever their position in their own tree walk, instead of waiting for the
-// widest child loop of the wavefront at every level.
+// Flattened traversal (the FP64 form's; traverse_staged is the FP32 forms').  The lane's current node
+// (expanded: near, or above minDepth) has its children tested one per loop iteration; when they are done
+// the node's own (1 - b_c) share is added and the next near node becomes the current one.  Either way an
+// iteration handles exactly one node X: it loads X's cell and header and the moments of the node it
+// contributes (X itself when testing, the finished node when moving on), computes X's distance, then
+// either classifies X as a child (far / leaf / near) or makes it the current node, and ends in one shared
+// node contribution.  Lanes of a wavefront therefore advance by one node per iteration whatever their
+// position in their own tree walk, instead of waiting for the widest child loop of the wavefront at every
+// level.  A near child's blend factor is exactly 1 (its t is dp / (dp + 0)), so the product of the factors
+// on the path to any expanded node is 1 and is not kept.
 //
-// Each iteration loads X's geometry and header, and the moments of the node it contributes (X
-// itself when testing, the finished node when moving on).  A finished node with more than one
-// near child leaves {first child, remaining near children, multiplier, distance term} in LDS for
-// its depth (13 B per level and lane, a per-lane bit set marks the levels in use); when a lane's
-// path runs out, the deepest such node's next near child is taken from there directly.
+// A finished node with near children leaves {first child, near children} in LDS for its depth (5 B per
+// level and lane, a per-lane bit set marks the levels in use), and the first waiting child of the deepest
+// such node is next.
 //
-// The walk is resumable: begin() sets it up for one query step, iter() advances it by one
-// iteration, and `active` drops when the step's sum is complete, so a kernel can interleave
-// the walks of successive queries on one lane.
+// Bound by FP64 vector instructions (276 an iteration against 370: weights.h has the exponential, quotients and
+// roots, blend() the cosine, and no multiplier), with the L1 72 % busy beside them.  1M points, 400k queries, two steps, six sigmas:
+// 8.0 -> 4.75 ms; 1k queries 2.1 -> 1.3; a rational kernel, 400k queries, 7.4 -> 3.8.
+constexpr double kNoBlend64 = 1e300;  // a distance term that makes every blend factor exactly 1 (above minDepth)
 template <int FORM, int SEM, int KT, bool CNT, class KP>
-struct Walker {
-  using T = typename FormT<FORM>::T;
-  using Acc = typename FormT<FORM>::Acc;
-  uint32_t node, first, nc, k, mask, pend;
-  int lvl;
-  bool blendNode, active;
-  T m, distP, shareSum, shareScale;
-  float Ai;
-
-  __device__ __forceinline__ void begin(Acc& acc, const KP& kp, const TreeView& tv, V3<T> q, T cutoff,
-                                        uint32_t minDepth, Counters& ct) {
-    active = false;
-    const uint4 h0 = tv.hdr[0];
-    if (hdr_leaf(h0.y)) {
-      add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h0, q, T(1), ct);
-      return;
-    }
-    const float4 g0 = tv.geo[0];
-    const T d0 = tdist<FORM>(q, g0);
-    if (minDepth == 0 && d0 > (T)g0.w * cutoff) {
-      add_node<FORM, KT>(acc, kp, tv, 0, __uint_as_float(h0.z), q, T(1));
+__device__ __forceinline__ void traverse_loads(AccP64& acc, const KP& kp, const TreeView& tv, V3<double> q, double cutoff,
+                                               uint32_t minDepth, WalkStack st, int tid, Counters& ct) {
+  static_assert(FORM == 2, "the FP32 forms' walk is staged");
+  const uint4 h0 = tv.hdr[0];
+  if (hdr_leaf(h0.y)) {
+    add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h0, q, 1.0, ct);
+    return;
+  }
+  const float4 g0 = tv.geo[0];
+  double dp = kNoBlend64;  // the current node's distance term
+  if (minDepth == 0) {
+    const double over = tdist<FORM>(q, g0) - (double)g0.w * cutoff;
+    if (over > 0.0) {
+      add_node<FORM, KT>(acc, kp, tv, 0, __uint_as_float(h0.z), q, 1.0);
       if constexpr (CNT) ct.far_ += 1;
       return;
     }
-    // current node = root
-    node = 0, first = h0.x, nc = hdr_count(h0.y), k = 0, mask = 0, pend = 0;
-    lvl = 0;
-    blendNode = minDepth == 0;
-    m = T(1);
-    distP = blendNode ? fabs(d0 - (T)g0.w * cutoff) : T(-1);
-    shareSum = T(0);
-    Ai = __uint_as_float(h0.z);
-    shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(T(1), (T)nc) : tratio<FORM>(T(1), (T)Ai);
-    active = true;
+    dp = fabs(over);
   }
-
-  __device__ __forceinline__ void iter(Acc& acc, const KP& kp, const TreeView& tv, V3<T> q, T cutoff,
-                                       uint32_t minDepth, LevelState<T> st, int tid, Counters& ct) {
+  const int32_t blendKey = (int32_t)(min(minDepth, 15u) << 27);  // headers of internal nodes at or below minDepth
+  // the current node: its children [x, xEnd) still to test, the near ones found
+  uint32_t node = 0, first = h0.x, x = first, xEnd = first + hdr_count(h0.y), mask = 0, pend = 0;
+  int lvl = 0;
+  double A = __uint_as_float(h0.z), shareSum = 0.0;
+  double scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.0, (double)hdr_count(h0.y)) : near_rcp(A);
+  for (bool active = true; active;) {
     if constexpr (CNT) ct.iters += 1;
-    // --- pick X: the next child of the current node, or the next near node to expand (of the
-    // finished node, or of the deepest node whose near children wait)
-    const bool testing = k < nc;
-    uint32_t x = 0;
-    T mp = T(0), dp = T(-1);
-    bool ownContrib = false;
-    const uint32_t ownNode = node;
-    const float ownA = Ai;
-    T ownF = T(0);
-    if (testing) {
-      x = first + k;
-      mp = m;
-      dp = blendNode ? distP : T(-1);
-    } else {
-      ownContrib = blendNode && shareSum != T(0);
-      ownF = m * shareSum;
-      if constexpr (CNT) ct.nearN += (blendNode && shareSum != T(0)) ? 1u : 0u;
+    const bool testing = x < xEnd;
+    const uint32_t tgt = testing ? x : node;
+    uint32_t nx = x;
+    if (!testing) {
       if (mask) {
-        // the finished node's first near child is next; the rest wait at this level
-        const uint32_t rest = mask & (mask - 1u);
-        mp = m;
-        dp = blendNode ? distP : T(-1);
-        if (rest) {
-          st.first[lvl][tid] = first;
-          st.mask[lvl][tid] = (uint8_t)rest;
-          st.mul[lvl][tid] = mp;
-          st.dist[lvl][tid] = dp;
-          pend |= 1u << lvl;
-        }
-        x = first + (uint32_t)__builtin_ctz(mask);
-        lvl = lvl + 1;
-      } else if (pend) {
-        // the deepest waiting node's next near child
-        const int L = 31 - __builtin_clz(pend);
-        const uint32_t wm = st.mask[L][tid];
-        const uint32_t rest = wm & (wm - 1u);
-        x = st.first[L][tid] + (uint32_t)__builtin_ctz(wm);
-        mp = st.mul[L][tid];
-        dp = st.dist[L][tid];
-        if (rest)
-          st.mask[L][tid] = (uint8_t)rest;
-        else
-          pend &= ~(1u << L);
-        lvl = L + 1;
+        st.first[lvl][tid] = first;
+        st.mask[lvl][tid] = (uint8_t)mask;
+        pend |= 1u << lvl;
+      }
+      active = pend != 0u;
+      if (active) {
+        const uint32_t L = 31u - (uint32_t)__builtin_clz(pend);
+        const uint32_t bits = st.mask[L][tid], rest = bits & (bits - 1u);
+        nx = st.first[L][tid] + (uint32_t)__builtin_ctz(bits);
+        st.mask[L][tid] = (uint8_t)rest;
+        if (!rest) pend ^= 1u << L;
+        lvl = (int)L + 1;
       } else {
-        active = false;
+        nx = 0u;
       }
     }
-    // --- loads: X's geometry and header, and the moments that may be added
-    const uint32_t tgt = testing ? x : ownNode;
+    const float4* rec = tv.recP + 4 * (uint64_t)nx;
     const NodeMom<FORM> mm = load_mom<FORM>(tv, tgt);
-    float4 gx = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint4 hx = make_uint4(0u, 0u, 0u, 0u);
-    if (active) {
-      gx = ld_rec(tv.geo, x);
-      hx = ld_rec(tv.hdr, x);
-    }
-    // --- X's blend factor against its parent (CPUUtils.cpp:489-497)
-    bool contrib = ownContrib;
-    float At = ownA;
-    T f = ownF;
-    if (active) {
-      const T dxq = tdist<FORM>(q, gx);
-      const T rc = (T)gx.w * cutoff;
-      T beta = T(1);
-      if (dp >= T(0)) {
-        const T dc = fmax(dxq - rc, T(0));
-        beta = blend(tratio<FORM>(dp, dp + dc));
+    const float4 g = rec[0];
+    const uint4 h = reinterpret_cast<const uint4*>(rec)[1];
+    const double over = tdist<FORM>(q, g) - (double)g.w * cutoff;
+    const double Ax = __uint_as_float(h.z);
+    bool contrib;
+    double f;
+    if (testing) {
+      // X's blend factor against its parent (CPUUtils.cpp:489-497); far: beyond its cutoff
+      f = blend(tratio<FORM>(dp, dp + fmax(over, 0.0)));
+      shareSum += (1.0 - f) * (SEM == MLOD_SEM_REF_CPU ? scale : quot_rcp(Ax, A, scale));
+      const bool leaf = (int32_t)h.y < 0, single = h.y >= (kLeafBit | kSingleBit);
+      const bool far = (int32_t)h.y >= blendKey && over > 0.0;
+      mask |= (leaf || far ? 0u : 1u) << (x - first);
+      if (leaf && !single) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);  // multi-point leaf
+      if constexpr (CNT) {
+        ct.tested += 1;
+        ct.far_ += far ? 1u : 0u;
+        ct.leafPts += single ? 1u : 0u;
       }
-      const T mx = mp * beta;
-      const float Ax = __uint_as_float(hx.z);
-      if (testing) {
-        ++k;
-        if (blendNode) {
-          const T share = SEM == MLOD_SEM_REF_CPU ? shareScale
-                                                  : (FORM == 1 ? (T)Ax * shareScale : (T)Ax / (T)Ai);
-          shareSum += (T(1) - beta) * share;
-        }
-        if constexpr (CNT) ct.tested += 1;
-        const bool leaf = hdr_leaf(hx.y);
-        const bool single = leaf && hdr_count(hx.y) == 1u;
-        const bool far = !leaf && hdr_depth(hx.y) >= minDepth && dxq > rc;
-        if (leaf && !single) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, hx, q, mx, ct);  // multi-point leaf
-        if (!leaf && !far) mask |= 1u << (k - 1u);
-        if constexpr (CNT) {
-          ct.far_ += far ? 1u : 0u;
-          ct.leafPts += single ? 1u : 0u;
-        }
-        contrib = far || single;
-        At = Ax;
-        f = mx;
-      } else {
-        // X becomes the current node, its children to test
-        node = x;
-        first = hx.x;
-        nc = hdr_count(hx.y);
-        k = 0u;
-        mask = 0u;
-        blendNode = hdr_depth(hx.y) >= minDepth;
-        distP = fabs(dxq - rc);
-        m = mx;
-        shareSum = T(0);
-        Ai = Ax;
-        shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(T(1), (T)nc) : tratio<FORM>(T(1), (T)Ax);
-      }
+      ++x;
+      contrib = far || single;
+    } else {
+      // the finished node's own share; X becomes the current node, its children to test
+      f = shareSum;
+      contrib = f != 0.0;
+      if constexpr (CNT) ct.nearN += contrib ? 1u : 0u;
+      node = nx;
+      first = x = h.x;
+      xEnd = first + (h.y & 15u);  // an internal node has at most 8 children
+      mask = 0u;
+      dp = (int32_t)h.y >= blendKey ? fabs(over) : kNoBlend64;
+      A = Ax;
+      scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.0, (double)(h.y & 15u)) : near_rcp(A);
+      shareSum = 0.0;
     }
-    if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
+    if (contrib) add_mom<FORM, KT>(acc, kp, mm, 0.f, q, f);
   }
-};
-
-// The whole walk of one query step on one lane (FP64 form).
-template <int FORM, int SEM, int KT, bool CNT, class KP>
-__device__ __forceinline__ void traverse_loads(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
-                                               V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T cutoff,
-                                               uint32_t minDepth, LevelState<typename FormT<FORM>::T> st, int tid,
-                                               Counters& ct) {
-  Walker<FORM, SEM, KT, CNT, KP> w;
-  w.begin(acc, kp, tv, q, cutoff, minDepth, ct);
-  while (w.active) w.iter(acc, kp, tv, q, cutoff, minDepth, st, tid, ct);
 }
 
 // ----------------------------------------------------------------------------- staged walk (FP32 forms)
@@ -546,12 +482,6 @@ __device__ __forceinline__ void stage_issue(const float4* rec, uint32_t idx, uin
   stage_row<3, BIG>(r, idx, lane, stage);
 }
 
-// A node with near children still to expand, per level and lane: its first child, and those children.
-struct StagedStack {
-  uint32_t (*first)[PBS];
-  uint8_t (*mask)[PBS];
-};
-
 // Half a distance term that makes every blend factor 1 (a node above minDepth: no blending below it):
 // kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit.
 constexpr float kNoBlend = 1e30f;
@@ -578,7 +508,7 @@ __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballo
 template <int FORM, int SEM, int KT, bool CNT, bool BIG, class KP>
 __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
                                                 V3<float> q, float cutoff, uint32_t minDepth, bool live,
-                                                StagedStack st, unsigned char* stage, int tid, Counters& ct) {
+                                                WalkStack st, unsigned char* stage, int tid, Counters& ct) {
 #pragma clang fp contract(off)  // the fused operations are written out
   const uint32_t lane = __lane_id();
   const float4* __restrict__ rec = FORM == 0 ? tv.recP : tv.recC;
@@ -960,8 +890,6 @@ struct WalkLds {
 };
 template <>
 struct WalkLds<2> {
-  double mul[kLevels][PBS];
-  double dist[kLevels][PBS];
   uint32_t first[kLevels][PBS];
   uint8_t mask[kLevels][PBS];
 };
@@ -972,11 +900,9 @@ __device__ __forceinline__ void traverse(typename FormT<FORM>::Acc& acc, const K
                                          V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T cutoff,
                                          uint32_t minDepth, bool live, WalkLds<FORM>& lds, int tid, Counters& ct) {
   if constexpr (FORM == 2) {
-    if (live)
-      traverse_loads<FORM, SEM, KT, CNT>(acc, kp, tv, q, cutoff, minDepth,
-                                         LevelState<double>{lds.first, lds.mask, lds.mul, lds.dist}, tid, ct);
+    if (live) traverse_loads<FORM, SEM, KT, CNT>(acc, kp, tv, q, cutoff, minDepth, WalkStack{lds.first, lds.mask}, tid, ct);
   } else {
-    const StagedStack st{lds.first, lds.mask};
+    const WalkStack st{lds.first, lds.mask};
     unsigned char* stage = lds.stage[__builtin_amdgcn_readfirstlane(tid >> 6)];
     if (tv.nn < (1u << 26))
       traverse_staged<FORM, SEM, KT, CNT, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
@@ -1497,7 +1423,7 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // added in order at the end, so the result does not depend on W.
 // Bound by the weights' vector instructions.  30k points, four sigmas, FP32C: 20k queries 6.0 -> 0.76 ms,
 // 500 queries 6.0 -> 0.19 (one lane per query left the chip two thirds empty, and each pair paid nine
-// compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries: 20.1 -> 1.2.
+// compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries: 20.1 -> 1.05.
 // The fit uses the 1e-12 plane threshold of GlobalAPSS.cu:143 (the REF_CPU fit).
 constexpr int kGlobalQ = 16;
 constexpr int kSlices = 16;
@@ -1792,6 +1718,7 @@ KParams make_kparams(const mlod_kernel& k) {
   p.cp = k.constant_shift > 0.0001f ? k.constant_shift : 0.0001f;
   p.e = k.exponent;
   const double er = std::nearbyint((double)k.exponent);
+  p.cpe = std::pow((double)p.cp, (double)p.e);
   p.eint = (er == (double)k.exponent && er >= 1.0 && er <= 16.0) ? (int)er : -1;
   const double log2e = 1.4426950408889634;
   if (k.type == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
@@ -1799,13 +1726,13 @@ KParams make_kparams(const mlod_kernel& k) {
       const double sg = k.sigmas[s];
       p.a[s] = (float)(-log2e / (2.0 * sg * sg));
       p.b[s] = (float)(1.0 / (sg * sg * sg));
-      p.ad[s] = -1.0 / (2.0 * sg * sg);
+      p.ad[s] = (double)(-1.44269504088896340736L / (2.0L * sg * sg));
       p.bd[s] = 1.0 / (sg * sg * sg);
     }
   } else if (k.type == MLOD_KERNEL_GAUSSIAN) {
     const double sg = k.sigma;
     p.a[0] = (float)(-log2e / (2.0 * sg * sg));
-    p.ad[0] = -1.0 / (2.0 * sg * sg);
+    p.ad[0] = (double)(-1.44269504088896340736L / (2.0L * sg * sg));
   }
   return p;
 }
