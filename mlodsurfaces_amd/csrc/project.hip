@@ -452,9 +452,14 @@ __device__ __forceinline__ void traverse_loads(AccP64& acc, const KP& kp, const 
 // 100 % busy, 131 an iteration against 152 before: no multiplier, reciprocals of A kept in the
 // records, one stack access an iteration), and the smaller stacks let five waves run per SIMD against
 // four.  8M points, 8M queries, six sigmas, FP32C: 20.6 -> 16.5 ms a step; 1M points and queries,
-// rational kernel, plain FP32: 11.7 -> 10.0 (8.1 with the quotients and roots of
-// weights.h); 100k queries x 10 steps on 1M points: 5.5 -> 4.8.
+// rational kernel, plain FP32: 11.7 -> 10.0 (8.1 with the quotients and roots of weights.h).
 // (Four waves per SIMD, with the stacks one word a level longer, left the step at 20.6 ms.)
+// A launch that fills the chip less is bound by an iteration's round trip.  So a record serves both its
+// visits: a node that becomes current comes through the stage like a child, its moments stay in
+// registers until its own share is added, and the next record's loads are issued as soon as this one has
+// been classified, before its terms are formed.  100k queries x 10 steps on 1M points: 5.5 -> 4.8 ms with
+// the stage, 4.2 so (loading the cell of the node that becomes current apart, and the finished node's
+// moments again, at the iteration's start); a burst of 20 requests served 29.3 -> 26.0.
 constexpr uint32_t kStageRow = 1024 + 16;
 constexpr uint32_t kStageBytes = 4 * kStageRow;  // per wavefront
 
@@ -486,15 +491,9 @@ __device__ __forceinline__ void stage_issue(const float4* rec, uint32_t idx, uin
 // kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit.
 constexpr float kNoBlend = 1e30f;
 
-// Cell and header of record idx.
-typedef float Quad __attribute__((ext_vector_type(4)));
-template <bool BIG>
-__device__ __forceinline__ void load_head(const float4* rec, uint32_t idx, Quad& g, Quad& h) {
-  const char* r = reinterpret_cast<const char*>(rec);
-  const char* src = BIG ? r + (uint64_t)idx * 64u : r + (idx << 6);
-  g = *reinterpret_cast<const Quad*>(src);
-  h = *reinterpret_cast<const Quad*>(src + 16);
-  asm volatile("" : "+v"(g), "+v"(h));  // both loads are issued before either is waited for
+__device__ __forceinline__ void swap_regs(float& a, float& b) { asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
+__device__ __forceinline__ void swap_regs(float4& a, float4& b) {
+  swap_regs(a.x, b.x), swap_regs(a.y, b.y), swap_regs(a.z, b.z), swap_regs(a.w, b.w);
 }
 __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
@@ -533,60 +532,19 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       active = 0u;
     }
   }
-  // the current node: its children [first, xEnd), the next one to test, the near ones found
-  uint32_t node = 0, first = h0.x, x = first, xEnd = active ? first + hdr_count(h0.y) : first, mask = 0, pend = 0;
+  // the current node: its children [first, xEnd), the next one to test, the near ones found; its area and moments
+  uint32_t first = h0.x, x = first, xEnd = active ? first + hdr_count(h0.y) : first, mask = 0, pend = 0;
   int lvl = 0;
   float Ai = __uint_as_float(h0.z), shareSum = 0.f;
   float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)hdr_count(h0.y)) : rec[1].w;
+  NodeMom<FORM> own = load_mom<FORM>(tv, 0);
   const unsigned char* mine = stage + (lane & 3u) * kStageRow + (lane >> 2) * 64u;
+  stage_issue<BIG>(rec, x, lane, stage);
   while (any_lane(active != 0u)) {
 #pragma unroll 1
     for (uint32_t b = 0; b < kFlush && any_lane(active != 0u); ++b) {
       if constexpr (CNT) ct.iters += active ? 1u : 0u;
-      const bool testing = x < xEnd;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last record has been read
-      stage_issue<BIG>(rec, testing ? x : node, lane, stage);
-      bool contrib = false;
-      float f = 0.f;
-      if (active && !testing) {
-        // the node is finished: its own share is added, and the next near node becomes current: the
-        // first waiting child of the deepest node that has some
-        f = shareSum;
-        contrib = f != 0.f;
-        if constexpr (CNT) ct.nearN += contrib ? 1u : 0u;
-        if (mask) {
-          st.first[lvl][tid] = first;
-          st.mask[lvl][tid] = (uint8_t)mask;
-          pend |= 1u << lvl;
-        }
-        if (pend) {
-          const uint32_t L = 31u - (uint32_t)__builtin_clz(pend);
-          const uint32_t bits = st.mask[L][tid], from = st.first[L][tid];
-          const uint32_t rest = bits & (bits - 1u);
-          st.mask[L][tid] = (uint8_t)rest;
-          if (!rest) pend ^= 1u << L;
-          lvl = (int)L + 1;
-          node = from + (uint32_t)__builtin_ctz(bits);
-          Quad gx, hx;
-          load_head<BIG>(rec, node, gx, hx);
-          const uint32_t code = __float_as_uint(hx.y);
-          dh = 0.5f * fabsf(tdist<FORM>(q, make_float4(gx.x, gx.y, gx.z, gx.w)) - gx.w * cutoff);
-          if (blendKey) {
-            asm volatile("");  // (a uniform branch, not a select)
-            dh = (int32_t)code >= blendKey ? dh : kNoBlend;
-          }
-          first = x = __float_as_uint(hx.x);
-          xEnd = first + (code & 15u);  // an internal node has at most 8 children
-          Ai = hx.z;
-          scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)(code & 15u)) : hx.w;
-        } else {
-          active = 0u;
-          node = 0u;
-        }
-        mask = 0u;
-        shareSum = 0.f;
-      }
-      // the record: every load is back before it is read, and read before the next iteration's loads
+      // the record: a child of the current node, or the node that follows it
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       const float4 g = *reinterpret_cast<const float4*>(mine);
       const uint4 h = *reinterpret_cast<const uint4*>(mine + 16);
@@ -594,11 +552,12 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       mm.m0 = *reinterpret_cast<const float4*>(mine + 32);
       mm.m1 = *reinterpret_cast<const float4*>(mine + 48);
       if constexpr (FORM == 0) mm.rA = __uint_as_float(h.w);
-      const float At = __uint_as_float(h.z);
-      bool multi = false;
-      if (testing) {
+      float At = __uint_as_float(h.z);
+      const float over = tdist<FORM>(q, g) - g.w * cutoff;
+      bool contrib = false, multi = false;
+      float f = 0.f;
+      if (x < xEnd) {
         // X's blend factor against its parent (CPUUtils.cpp:489-497); far: beyond its cutoff
-        const float over = tdist<FORM>(q, g) - g.w * cutoff;
         const float dc = fmaxf(over, 0.f);
         f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
         const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : quot_rcp(At, Ai, scale));
@@ -615,7 +574,50 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
         }
         ++x;
         contrib = far || single;
+      } else if (active) {
+        // the current node is finished: its own share is added, and X becomes current
+        f = shareSum;
+        contrib = f != 0.f;
+        if constexpr (CNT) ct.nearN += contrib ? 1u : 0u;
+        swap_regs(mm.m0, own.m0);
+        swap_regs(mm.m1, own.m1);
+        if constexpr (FORM == 0) swap_regs(mm.rA, own.rA);
+        swap_regs(At, Ai);
+        shareSum = 0.f;
+        active = lvl >= 0 ? 1u : 0u;  // (none follows the last node)
+        first = x = h.x;
+        xEnd = active ? first + (h.y & 15u) : first;  // an internal node has at most 8 children
+        dh = 0.5f * fabsf(over);
+        if (blendKey) {
+          asm volatile("");  // (a uniform branch, not a select)
+          dh = (int32_t)h.y >= blendKey ? dh : kNoBlend;
+        }
+        scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)(h.y & 15u)) : __uint_as_float(h.w);
       }
+      uint32_t idx = x;
+      if (active && x == xEnd) {
+        // the children are done: the first waiting child of the deepest node that has some follows
+        if (mask) {
+          st.first[lvl][tid] = first;
+          st.mask[lvl][tid] = (uint8_t)mask;
+          pend |= 1u << lvl;
+          mask = 0u;
+        }
+        lvl = -1;
+        idx = 0u;
+        if (pend) {
+          const uint32_t L = 31u - (uint32_t)__builtin_clz(pend);
+          const uint32_t bits = st.mask[L][tid], from = st.first[L][tid];
+          const uint32_t rest = bits & (bits - 1u);
+          st.mask[L][tid] = (uint8_t)rest;
+          if (!rest) pend ^= 1u << L;
+          lvl = (int)L + 1;
+          idx = from + (uint32_t)__builtin_ctz(bits);
+        }
+      }
+      // the next record's loads go out before this one's terms are formed (it has been read by now)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      stage_issue<BIG>(rec, idx, lane, stage);
       if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
       if (any_lane(multi)) {  // a leaf of several points (at the last level, or by the build's option)
         if (multi) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);
@@ -623,6 +625,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
     }
     if constexpr (FORM == 1) acc.flush();
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the stage may be used again)
   if constexpr (FORM == 1) acc.flush();
 }
 
