@@ -8,11 +8,13 @@
 // outer loop restarts from the depth-0 neighbours of the cells reached and adapts the final
 // depth to the extent of the depth-0 cells used (getRelativeDepth, upsample.cpp:146-161).
 //
-// Here the cell sets stay on the device as sorted, unique 64-bit keys whose unsigned order is
-// the reference's node_comparator (octree.h:147-154: depth, then z, y, x, signed):
+// Here the cell sets stay on the device as unique 64-bit keys whose unsigned order is the
+// reference's node_comparator (octree.h:147-154: depth, then z, y, x, signed):
 //   key = depth << 60 | (z + 2^19) << 40 | (y + 2^19) << 20 | (x + 2^19)
-// Every set operation of the reference (sort + unique, children, neighbour expansion, ancestor
-// maps) is a kernel plus a rocPRIM radix sort / unique; the projection is the library's own
+// The sets between two levels need no order (the queries are sorted along a curve before they are
+// projected, and a query's projection depends on it alone), so the kernel that makes the cells of one
+// (enclosing cells, children with their neighbours, ancestors) keeps the first of each through a hash
+// table; the results are sorted by a rocPRIM radix sort / unique.  The projection is the library's own
 // projection of the tree (its kernel, parameters, semantics, form and neighbourhood mode).  Only
 // the handful of depth-0 cells of the outer loop live on the host.
 #include <cstring>
@@ -49,6 +51,86 @@ __host__ __device__ __forceinline__ bool coord_ok(int v) { return v >= -kBias &&
 // Error flags raised by kernels (bit 0: a coordinate left the key range).
 enum { kFlagRange = 1 };
 
+// ----------------------------------------------------------------------------- sets of cells
+// What the kernels of one set operation leave for the host (one copy brings it).
+struct GenState {
+  uint64_t count;                // cells of the set
+  unsigned long long nonfinite;  // projections that were not finite
+  uint32_t flags;
+};
+
+// An open-addressing table of keys, empty slots kNone, at least twice as many slots as keys are offered
+// (a probe so ends); the keys that enter it first go to `out`, in no particular order.  Most offers are
+// repeats (a cell's 64 slots hold some 10 new ones), which one load settles; sorting them all took up to
+// 20 launches and four waits a set.  generate() on 1M points, ms with each set sorted / hashed: depth 5 5.7 /
+// 4.3, 7 18.6 / 15.1, 8 36.4 / 31.1, 9 88 / 77, 10 294 / 260, 11 1086 / 967 (33M cells).
+struct CellSet {
+  uint64_t* table;
+  uint64_t mask;  // slots - 1, slots a power of two
+  uint64_t* out;
+  GenState* st;
+};
+
+__global__ __launch_bounds__(BS) void k_clear_set(CellSet set) {
+  const uint64_t stride = (uint64_t)gridDim.x * BS;
+  const uint64_t i0 = (uint64_t)blockIdx.x * BS + threadIdx.x;
+  if (i0 == 0) set.st->count = 0;
+  ulonglong2* t = reinterpret_cast<ulonglong2*>(set.table);
+  for (uint64_t i = i0; i <= set.mask / 2; i += stride) t[i] = make_ulonglong2(kNone, kNone);
+}
+
+// True for the one offer of `key` that enters it.
+__device__ __forceinline__ bool set_enter(const CellSet& set, uint64_t key) {
+  uint64_t h = key * 0x9e3779b97f4a7c15ull;
+  h ^= h >> 32;
+  for (;; ++h) {
+    unsigned long long* slot = reinterpret_cast<unsigned long long*>(set.table + (h & set.mask));
+    // most offers find their key with a load (a stale one is settled by the exchange)
+    const uint64_t seen = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (seen == key) return false;
+    if (seen != kNone) continue;
+    const uint64_t was = atomicCAS(slot, (unsigned long long)kNone, (unsigned long long)key);
+    if (was == kNone) return true;
+    if (was == key) return false;
+  }
+}
+
+// Offers R keys a thread (kNone: no offer) and appends those that entered; every thread of the
+// workgroup calls it.  A key that the lane before or the thread's last one has too is left to that one:
+// ancestors come in long runs, and exchanges on one slot take 12 ns each (120k cells of one ancestor: 1.5
+// ms without this).
+template <int R>
+__device__ __forceinline__ void set_add(const CellSet& set, const uint64_t (&key)[R]) {
+  constexpr uint32_t W = BS / 64;
+  __shared__ uint32_t sCount[R * W];
+  __shared__ uint64_t sBase;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint64_t fresh[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint64_t left = __shfl_up(key[r], 1);
+    const bool again = (lane != 0 && key[r] == left) || (r != 0 && key[r] == key[r ? r - 1 : 0]);
+    const bool f = key[r] != kNone && !again && set_enter(set, key[r]);
+    fresh[r] = __ballot(f);
+    if (lane == 0) sCount[r * W + wave] = (uint32_t)__popcll(fresh[r]);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t sum = 0;
+    for (uint32_t k = 0; k < R * W; ++k) {
+      const uint32_t c = sCount[k];
+      sCount[k] = sum;
+      sum += c;
+    }
+    sBase = sum ? atomicAdd(reinterpret_cast<unsigned long long*>(&set.st->count), (unsigned long long)sum) : 0ull;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (fresh[r] >> lane & 1ull)
+      set.out[sBase + sCount[r * W + wave] + (uint32_t)__popcll(fresh[r] & ((1ull << lane) - 1ull))] = key[r];
+}
+
 // aabb_octree::center over [-1, 1]^3 (octree.h:946-955): min + w p and min + w (p + 1) with
 // w = 2 / 2^d, averaged.  Every one of those float operations is exact for |p| < 2^19 and
 // d <= 14, so the centre is exactly (2p + 1) 2^-d - 1, which is what is computed.
@@ -79,12 +161,9 @@ __device__ __forceinline__ bool enclose1(float p, int d, int& out) {
 // find_stable_nodesGPU's cell assignment (upsample.cpp:336-343) for the projected queries in
 // the tree's sorted order: slot j holds the projection of input cell perm[j].  A degenerate
 // normal (|n|^2 < 0.5, glm::length2) or a non-finite projected position gives the root.
-__global__ __launch_bounds__(BS) void k_enclose(const float4* __restrict__ q, const float4* __restrict__ qn,
-                                                const uint32_t* __restrict__ perm, const uint64_t* __restrict__ in,
-                                                uint32_t n, uint64_t* __restrict__ out, uint32_t* __restrict__ flags,
-                                                unsigned long long* __restrict__ nonfinite) {
-  const uint32_t j = blockIdx.x * BS + threadIdx.x;
-  if (j >= n) return;
+__device__ __forceinline__ uint64_t enclosing_key(const float4* __restrict__ q, const float4* __restrict__ qn,
+                                                  const uint32_t* __restrict__ perm, const uint64_t* __restrict__ in,
+                                                  uint32_t j, GenState* __restrict__ st) {
   const int d = key_depth(in[perm[j]]);
   const float4 nm = qn[j];
   const float l2 = __fadd_rn(__fadd_rn(__fmul_rn(nm.x, nm.x), __fmul_rn(nm.y, nm.y)), __fmul_rn(nm.z, nm.z));
@@ -96,22 +175,27 @@ __global__ __launch_bounds__(BS) void k_enclose(const float4* __restrict__ q, co
       if (coord_ok(x) && coord_ok(y) && coord_ok(z))
         key = cell_key(d, x, y, z);
       else
-        atomicOr(flags, (uint32_t)kFlagRange);
+        atomicOr(&st->flags, (uint32_t)kFlagRange);
     } else {
-      atomicAdd(nonfinite, 1ull);
+      atomicAdd(&st->nonfinite, 1ull);
     }
   }
-  out[j] = key;
+  return key;
+}
+__global__ __launch_bounds__(BS) void k_enclose_set(const float4* __restrict__ q, const float4* __restrict__ qn,
+                                                    const uint32_t* __restrict__ perm, const uint64_t* __restrict__ in,
+                                                    uint32_t n, CellSet set) {
+  const uint32_t j = blockIdx.x * BS + threadIdx.x;
+  const uint64_t key[1] = {j < n ? enclosing_key(q, qn, perm, in, j, set.st) : kNone};
+  set_add<1>(set, key);
 }
 
 // add_children (upsample.cpp:348-358) followed by expand(current, depth + 1)
 // (upsample.cpp:409-419): a cell at `depth` contributes the 4 x 4 x 4 block of depth + 1 cells
 // made of its children and their neighbours; a shallower cell (the root and its descendants
 // re-entered after a failed projection) contributes its 8 children only.  64 slots per cell.
-__global__ __launch_bounds__(BS) void k_expand(const uint64_t* __restrict__ sub, uint32_t n, int depth,
-                                               uint64_t* __restrict__ out, uint32_t* __restrict__ flags) {
-  const uint64_t t = (uint64_t)blockIdx.x * BS + threadIdx.x;
-  if (t >= (uint64_t)n * 64) return;
+__device__ __forceinline__ uint64_t expanded_key(const uint64_t* __restrict__ sub, uint64_t t, int depth,
+                                                 GenState* __restrict__ st) {
   const uint32_t i = (uint32_t)(t >> 6), s = (uint32_t)(t & 63);
   const uint64_t k = sub[i];
   const int d = key_depth(k), x = key_x(k), y = key_y(k), z = key_z(k);
@@ -125,39 +209,54 @@ __global__ __launch_bounds__(BS) void k_expand(const uint64_t* __restrict__ sub,
     cy = 2 * y + (int)((s >> 1) & 1);
     cz = 2 * z + (int)(s >> 2);
   } else {
-    out[t] = kNone;
-    return;
+    return kNone;
   }
   if (!coord_ok(cx) || !coord_ok(cy) || !coord_ok(cz)) {
-    atomicOr(flags, (uint32_t)kFlagRange);
-    out[t] = kNone;
-    return;
+    atomicOr(&st->flags, (uint32_t)kFlagRange);
+    return kNone;
   }
-  out[t] = cell_key(d + 1, cx, cy, cz);
+  return cell_key(d + 1, cx, cy, cz);
+}
+constexpr int kExpandRun = 4;  // offers a thread
+__global__ __launch_bounds__(BS) void k_expand_set(const uint64_t* __restrict__ sub, uint32_t n, int depth, CellSet set) {
+  const uint64_t t0 = (uint64_t)blockIdx.x * (BS * kExpandRun) + threadIdx.x;
+  uint64_t key[kExpandRun];
+#pragma unroll
+  for (int r = 0; r < kExpandRun; ++r) {
+    const uint64_t t = t0 + r * BS;
+    key[r] = t < (uint64_t)n * 64 ? expanded_key(sub, t, depth, set.st) : kNone;
+  }
+  set_add<kExpandRun>(set, key);
 }
 
 // ancestor_at_depth (octree.h:561-573): repeated floor halving, i.e. an arithmetic shift.
 // Cells at or above `depth` are kept as they are (onlySetDepthNodes, upsample.cpp:163-173).
+__device__ __forceinline__ uint64_t ancestor_key(uint64_t k, int depth) {
+  const int sh = key_depth(k) - depth;
+  return sh <= 0 ? k : cell_key(depth, key_x(k) >> sh, key_y(k) >> sh, key_z(k) >> sh);
+}
 __global__ __launch_bounds__(BS) void k_ancestor(const uint64_t* __restrict__ in, uint32_t n, int depth,
                                                  uint64_t* __restrict__ out) {
   const uint32_t i = blockIdx.x * BS + threadIdx.x;
-  if (i >= n) return;
-  const uint64_t k = in[i];
-  const int d = key_depth(k);
-  if (d <= depth) {
-    out[i] = k;
-    return;
+  if (i < n) out[i] = ancestor_key(in[i], depth);
+}
+constexpr int kAncestorRun = 8;
+__global__ __launch_bounds__(BS) void k_ancestor_set(const uint64_t* __restrict__ in, uint32_t n, int depth, CellSet set) {
+  const uint32_t i0 = blockIdx.x * (BS * kAncestorRun) + threadIdx.x;
+  uint64_t key[kAncestorRun];
+#pragma unroll
+  for (int r = 0; r < kAncestorRun; ++r) {
+    const uint32_t i = i0 + r * BS;
+    key[r] = i < n ? ancestor_key(in[i], depth) : kNone;
   }
-  const int sh = d - depth;
-  out[i] = cell_key(depth, key_x(k) >> sh, key_y(k) >> sh, key_z(k) >> sh);
+  set_add<kAncestorRun>(set, key);
 }
 
 // generateFromPoints (upsample.cpp:128-144): the max_depth cell enclosing each point of the
 // box (aabb_octree::enclosing, octree.h:957-965): floor(((p - min) / diag) / 2^-d).
 __global__ __launch_bounds__(BS) void k_enclose_points(const float* __restrict__ xyz, uint32_t n, int d, float mnx,
                                                        float mny, float mnz, float dgx, float dgy, float dgz,
-                                                       uint64_t* __restrict__ out, uint32_t* __restrict__ flags,
-                                                       unsigned long long* __restrict__ nonfinite) {
+                                                       uint64_t* __restrict__ out, GenState* __restrict__ st) {
   const uint32_t i = blockIdx.x * BS + threadIdx.x;
   if (i >= n) return;
   const float w = __builtin_ldexpf(1.0f, -d);
@@ -175,12 +274,12 @@ __global__ __launch_bounds__(BS) void k_enclose_points(const float* __restrict__
     }
   }
   if (!fin) {
-    atomicAdd(nonfinite, 1ull);
+    atomicAdd(&st->nonfinite, 1ull);
     out[i] = kNone;
     return;
   }
   if (!coord_ok(c[0]) || !coord_ok(c[1]) || !coord_ok(c[2])) {
-    atomicOr(flags, (uint32_t)kFlagRange);
+    atomicOr(&st->flags, (uint32_t)kFlagRange);
     out[i] = kNone;
     return;
   }
@@ -218,7 +317,8 @@ __global__ __launch_bounds__(BS) void k_decode(const uint64_t* __restrict__ keys
 
 inline uint32_t blocks(uint64_t n) { return (uint32_t)((n + BS - 1) / BS); }
 
-// A growable device array of keys.
+// A growable device array of keys.  (A growth waits for the stream: the small levels share one size.)
+constexpr size_t kKeyVecMin = (size_t)1 << 18;
 struct KeyVec {
   uint64_t* p = nullptr;
   size_t n = 0, cap = 0;
@@ -230,7 +330,7 @@ struct KeyVec {
   // room for m keys, keeping the first `keep`
   int reserve(size_t m, size_t keep, hipStream_t s) {
     if (m <= cap) return MLOD_OK;
-    const size_t nc = std::max(m, cap + cap / 2);
+    const size_t nc = std::max({m, cap + cap / 2, kKeyVecMin});
     uint64_t* q = nullptr;
     if (dev_malloc(&q, nc * sizeof(uint64_t)) != hipSuccess)
       return fail(MLOD_ERR_OOM, "adaptive octree: hipMalloc failed for " + std::to_string(nc) + " cells");
@@ -250,11 +350,10 @@ struct mlod_generator {
   mlod_tree* tree = nullptr;
   mlod::KeyVec leaves, total;   // results, sorted and unique
   mlod::KeyVec a, b, c;         // work sets
+  mlod::KeyVec table;           // slots of the set that is being made
   void* sortTmp = nullptr;
   size_t sortBytes = 0;
-  uint64_t* dCount = nullptr;   // unique count
-  uint32_t* dFlags = nullptr;
-  unsigned long long* dNonfinite = nullptr;
+  mlod::GenState* dState = nullptr;
   float* dXyz = nullptr;        // centres of the leaves (n x 3), valid after mlod_generator_centres
   size_t xyzCap = 0;
   float* dStage = nullptr;      // centres projected by the current level
@@ -292,7 +391,20 @@ int ensure_sort_tmp(mlod_generator* g, size_t n, hipStream_t s) {
   return MLOD_OK;
 }
 
-// remove_duplicates (upsample.cpp:28-32) of the n keys in `in` (clobbered) into `out`; drops the
+// The count, flags and non-finite projections of the operations so far (waits for the stream).
+int read_state(mlod_generator* g, uint64_t* count, hipStream_t s) {
+  GenState st;
+  MLOD_HIP(hipMemcpyAsync(&st, g->dState, sizeof(st), hipMemcpyDeviceToHost, s));
+  MLOD_HIP(hipStreamSynchronize(s));
+  g->nonfinite = st.nonfinite;
+  if (count) *count = st.count;
+  if (st.flags & kFlagRange)
+    return fail(MLOD_ERR_UNSUPPORTED, "adaptive octree: a cell coordinate left [-2^19, 2^19) (the surface reaches far "
+                                      "outside [-1, 1]^3 at this depth)");
+  return MLOD_OK;
+}
+
+// remove_duplicates (upsample.cpp:28-32) of the n keys in `in` (clobbered) into `out`, sorted; drops the
 // empty-slot key.  Returns the unique count through *m (waits for the stream).
 int sort_unique(mlod_generator* g, KeyVec& in, size_t n, KeyVec& out, size_t* m, hipStream_t s) {
   *m = 0;
@@ -306,10 +418,10 @@ int sort_unique(mlod_generator* g, KeyVec& in, size_t n, KeyVec& out, size_t* m,
   size_t bytes = g->sortBytes;
   MLOD_HIP(rocprim::radix_sort_keys(g->sortTmp, bytes, in.p, out.p, n, 0, 64, s));
   bytes = g->sortBytes;
-  MLOD_HIP(rocprim::unique(g->sortTmp, bytes, out.p, in.p, g->dCount, n, rocprim::equal_to<uint64_t>(), s));
+  MLOD_HIP(rocprim::unique(g->sortTmp, bytes, out.p, in.p, &g->dState->count, n, rocprim::equal_to<uint64_t>(), s));
   uint64_t cnt = 0, last = 0;
-  MLOD_HIP(hipMemcpyAsync(&cnt, g->dCount, sizeof(cnt), hipMemcpyDeviceToHost, s));
-  MLOD_HIP(hipStreamSynchronize(s));
+  const int flagged = read_state(g, &cnt, s);  // (the set is handed over all the same)
+  if (flagged && flagged != MLOD_ERR_UNSUPPORTED) return flagged;
   if (cnt) {
     MLOD_HIP(hipMemcpyAsync(&last, in.p + cnt - 1, sizeof(last), hipMemcpyDeviceToHost, s));
     MLOD_HIP(hipStreamSynchronize(s));
@@ -319,20 +431,26 @@ int sort_unique(mlod_generator* g, KeyVec& in, size_t n, KeyVec& out, size_t* m,
   out.n = cnt;
   in.n = 0;
   *m = cnt;
-  return MLOD_OK;
+  return flagged;
 }
 
-int check_flags(mlod_generator* g, hipStream_t s) {
-  uint32_t f = 0;
-  unsigned long long nf = 0;
-  MLOD_HIP(hipMemcpyAsync(&f, g->dFlags, sizeof(f), hipMemcpyDeviceToHost, s));
-  MLOD_HIP(hipMemcpyAsync(&nf, g->dNonfinite, sizeof(nf), hipMemcpyDeviceToHost, s));
-  MLOD_HIP(hipStreamSynchronize(s));
-  g->nonfinite = nf;
-  if (f & kFlagRange)
-    return fail(MLOD_ERR_UNSUPPORTED, "adaptive octree: a cell coordinate left [-2^19, 2^19) (the surface reaches far "
-                                      "outside [-1, 1]^3 at this depth)");
+// An empty set for `offers` keys, its cells to go to `out`.
+int begin_set(mlod_generator* g, size_t offers, KeyVec& out, CellSet* set, hipStream_t s) {
+  if (offers > 0xffffffffu) return fail(MLOD_ERR_UNSUPPORTED, "adaptive octree: more than 2^32 cells in one set");
+  uint64_t slots = 4096;
+  while (slots < 2 * offers) slots *= 2;
+  if (int r = out.reserve(offers, 0, s)) return r;
+  if (int r = g->table.reserve(slots, 0, s)) return r;
+  *set = CellSet{g->table.p, slots - 1, out.p, g->dState};
+  k_clear_set<<<std::min<uint32_t>(blocks(slots / 2), 2048u), BS, 0, s>>>(*set);
+  MLOD_HIP(hipGetLastError());
   return MLOD_OK;
+}
+int end_set(mlod_generator* g, KeyVec& out, hipStream_t s) {
+  uint64_t n = 0;
+  const int r = read_state(g, &n, s);
+  out.n = n;
+  return r;
 }
 
 // The tree's own projection of the n centres in g->dStage: one step, step bound FLT_MAX
@@ -347,8 +465,8 @@ int project_centres(mlod_generator* g, uint32_t n, hipStream_t s) {
   return r;
 }
 
-// find_stable_nodesGPU (upsample.cpp:317-346) on the cells in cur -> sorted unique cells in sub
-int find_stable(mlod_generator* g, KeyVec& cur, KeyVec& sub, KeyVec& scratch, hipStream_t s) {
+// find_stable_nodesGPU (upsample.cpp:317-346) on the cells in cur -> unique cells in sub
+int find_stable(mlod_generator* g, KeyVec& cur, KeyVec& sub, hipStream_t s) {
   const size_t n = cur.n;
   if (!n) {
     sub.n = 0;
@@ -365,29 +483,29 @@ int find_stable(mlod_generator* g, KeyVec& cur, KeyVec& sub, KeyVec& scratch, hi
   k_centres<<<blocks(n), BS, 0, s>>>(cur.p, (uint32_t)n, g->dStage);
   MLOD_HIP(hipGetLastError());
   if (int r = project_centres(g, (uint32_t)n, s)) return r;
-  if (int r = scratch.reserve(n, 0, s)) return r;
   const QueryState& qs = g->tree->qs;
-  k_enclose<<<blocks(n), BS, 0, s>>>(qs.q, qs.qn, qs.perm, cur.p, (uint32_t)n, scratch.p, g->dFlags, g->dNonfinite);
+  CellSet set;
+  if (int r = begin_set(g, n, sub, &set, s)) return r;
+  k_enclose_set<<<blocks(n), BS, 0, s>>>(qs.q, qs.qn, qs.perm, cur.p, (uint32_t)n, set);
   MLOD_HIP(hipGetLastError());
-  size_t m = 0;
-  if (int r = sort_unique(g, scratch, n, sub, &m, s)) return r;
-  return check_flags(g, s);
+  return end_set(g, sub, s);
 }
 
 // compute_leaves (upsample.cpp:274-287): cur in, the cells after the last level in cur
 int compute_leaves(mlod_generator* g, uint32_t maxDepth, hipStream_t s) {
-  KeyVec &cur = g->a, &sub = g->b, &tmp = g->c;
+  KeyVec &cur = g->a, &sub = g->b;
   for (uint32_t depth = 0; depth < maxDepth + 1; ++depth) {
-    if (int r = find_stable(g, cur, sub, tmp, s)) return r;
+    if (int r = find_stable(g, cur, sub, s)) return r;
     const size_t ns = sub.n;
-    if (int r = tmp.reserve(ns * 64, 0, s)) return r;
+    cur.n = 0;
     if (ns) {
-      k_expand<<<blocks(ns * 64), BS, 0, s>>>(sub.p, (uint32_t)ns, (int)depth, tmp.p, g->dFlags);
+      CellSet set;
+      if (int r = begin_set(g, ns * 64, cur, &set, s)) return r;
+      k_expand_set<<<(uint32_t)((ns * 64 + BS * kExpandRun - 1) / (BS * kExpandRun)), BS, 0, s>>>(sub.p, (uint32_t)ns,
+                                                                                                 (int)depth, set);
       MLOD_HIP(hipGetLastError());
+      if (int r = end_set(g, cur, s)) return r;
     }
-    size_t m = 0;
-    if (int r = sort_unique(g, tmp, ns * 64, cur, &m, s)) return r;
-    if (int r = check_flags(g, s)) return r;
     if (g->keepTotal)
       if (int r = KeyVec_append(g->total, cur.p, cur.n, hipMemcpyDeviceToDevice, s)) return r;
   }
@@ -413,8 +531,7 @@ struct HostCell {
 int generate(mlod_generator* g, uint32_t maxDepth, hipStream_t s) {
   g->leaves.n = g->total.n = 0;
   g->projected = g->calls = g->nonfinite = 0;
-  MLOD_HIP(hipMemsetAsync(g->dFlags, 0, sizeof(uint32_t), s));
-  MLOD_HIP(hipMemsetAsync(g->dNonfinite, 0, sizeof(unsigned long long), s));
+  MLOD_HIP(hipMemsetAsync(g->dState, 0, sizeof(GenState), s));
   std::vector<uint64_t> depth0{cell_key(0, 0, 0, 0)}, old0;
   uint32_t maxRel = maxDepth;
   int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {-INT_MAX, -INT_MAX, -INT_MAX};
@@ -429,11 +546,13 @@ int generate(mlod_generator* g, uint32_t maxDepth, hipStream_t s) {
     // depth0_ancestors(current) (upsample.cpp:360-368): a small set, brought to the host
     std::vector<uint64_t> anc;
     if (cur.n) {
-      if (int r = g->b.reserve(cur.n, 0, s)) return r;
-      k_ancestor<<<blocks(cur.n), BS, 0, s>>>(cur.p, (uint32_t)cur.n, 0, g->b.p);
+      CellSet set;
+      if (int r = begin_set(g, cur.n, g->c, &set, s)) return r;
+      k_ancestor_set<<<(uint32_t)((cur.n + BS * kAncestorRun - 1) / (BS * kAncestorRun)), BS, 0, s>>>(
+          cur.p, (uint32_t)cur.n, 0, set);
       MLOD_HIP(hipGetLastError());
-      size_t m = 0;
-      if (int r = sort_unique(g, g->b, cur.n, g->c, &m, s)) return r;
+      if (int r = end_set(g, g->c, s)) return r;
+      const size_t m = g->c.n;
       anc.resize(m);
       if (m) {
         MLOD_HIP(hipMemcpyAsync(anc.data(), g->c.p, m * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
@@ -476,7 +595,7 @@ int generate(mlod_generator* g, uint32_t maxDepth, hipStream_t s) {
     if (int r = only_set_depth(g, g->total, maxRel, s)) return r;
   g->maxRel = maxRel;
   for (int a = 0; a < 3; ++a) g->box[a] = -1.f, g->box[3 + a] = 1.f;
-  return check_flags(g, s);
+  return read_state(g, nullptr, s);
 }
 
 int leaf_centres(mlod_generator* g, hipStream_t s) {
@@ -510,9 +629,7 @@ int mlod_generator_create(mlod_tree* t, mlod_generator** out) {
   *out = nullptr;
   mlod_generator* g = new mlod_generator();
   g->tree = t;
-  if (dev_malloc(&g->dCount, sizeof(uint64_t)) != hipSuccess ||
-      dev_malloc(&g->dFlags, sizeof(uint32_t)) != hipSuccess ||
-      dev_malloc(&g->dNonfinite, sizeof(unsigned long long)) != hipSuccess) {
+  if (dev_malloc(&g->dState, sizeof(GenState)) != hipSuccess) {
     mlod_generator_destroy(g);
     return fail(MLOD_ERR_OOM, "generator: hipMalloc failed");
   }
@@ -523,8 +640,8 @@ int mlod_generator_create(mlod_tree* t, mlod_generator** out) {
 int mlod_generator_destroy(mlod_generator* g) {
   if (!g) return MLOD_OK;
   (void)hipDeviceSynchronize();
-  g->leaves.release(), g->total.release(), g->a.release(), g->b.release(), g->c.release();
-  void* p[] = {g->sortTmp, g->dCount, g->dFlags, g->dNonfinite, g->dXyz, g->dStage};
+  g->leaves.release(), g->total.release(), g->a.release(), g->b.release(), g->c.release(), g->table.release();
+  void* p[] = {g->sortTmp, g->dState, g->dXyz, g->dStage};
   dev_free(p, sizeof(p) / sizeof(p[0]));
   delete g;
   return MLOD_OK;
@@ -555,8 +672,7 @@ int mlod_generate_from_points(mlod_generator* g, const float* xyz, uint32_t n, i
   g->projected = g->calls = 0;
   std::memcpy(g->box, b, sizeof(b));
   if (n == 0) return MLOD_OK;  // upsample.cpp:130
-  MLOD_HIP(hipMemsetAsync(g->dFlags, 0, sizeof(uint32_t), s));
-  MLOD_HIP(hipMemsetAsync(g->dNonfinite, 0, sizeof(unsigned long long), s));
+  MLOD_HIP(hipMemsetAsync(g->dState, 0, sizeof(GenState), s));
   const float* src = xyz;
   if (!device_src) {
     if (n > g->stageCap) {
@@ -572,11 +688,10 @@ int mlod_generate_from_points(mlod_generator* g, const float* xyz, uint32_t n, i
   }
   if (int r = g->c.reserve(n, 0, s)) return r;
   k_enclose_points<<<blocks(n), BS, 0, s>>>(src, n, (int)max_depth, b[0], b[1], b[2], b[3] - b[0], b[4] - b[1],
-                                            b[5] - b[2], g->c.p, g->dFlags, g->dNonfinite);
+                                            b[5] - b[2], g->c.p, g->dState);
   MLOD_HIP(hipGetLastError());
   size_t m = 0;
-  if (int r = sort_unique(g, g->c, n, g->leaves, &m, s)) return r;
-  return check_flags(g, s);
+  return sort_unique(g, g->c, n, g->leaves, &m, s);
 }
 
 int mlod_generator_info(const mlod_generator* g, uint64_t* out6) {
