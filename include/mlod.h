@@ -74,7 +74,8 @@ enum {
 
 /* How the MLoD walk is laid on the GPU (no counterpart in the reference, whose kernel walks one
  * thread per query, Fastapss.cu:160-333).  LANE: each lane walks its own query's tree path
- * (the default, and the faster on every workload measured).  WAVE: one walk per wavefront over
+ * (the default, and the faster on every workload measured; a batch too small to fill the chip is
+ * walked by eight lanes a query, to the same bits).  WAVE: one walk per wavefront over
  * the union of its 64 lanes' paths, node records in scalar registers, each lane taking part in
  * the nodes its own walk visits (near/far decided per lane and combined by ballot).  Both add
  * every lane's terms in the same order: the FP64 form gives the same bits, the FP32 forms the

@@ -1652,9 +1652,9 @@ void launch_batch_all(const ReqDesc* r, const uint2* blocks, uint32_t nblk, floa
 
 // Batches of at most this many queries take the grouped walk: it issues three times the instructions of
 // the lane walk and is done in a third of its time while the chip has room for them.  Three steps on 1M
-// points, four sigmas, FP32C, us with a lane / a group: 4k queries 1283 / 427, 16k 1315 / 530, 32k
-// 1318 / 884, 48k 1428 / 1186, 64k 1452 / 1473; plain FP32, rational, cutoff 3: 32k 3533 / 2045, 64k
-// 3789 / 3514.
+// points, four sigmas, FP32C, us with a lane / a group: 4k queries 1140 / 427, 16k 1178 / 537, 32k
+// 1180 / 905, 48k 1271 / 1212, 64k 1289 / 1464; plain FP32, rational, cutoff 3, torus: 32k 5412 / 3097,
+// 48k 5673 / 4314, 64k 5807 / 5470.
 constexpr uint32_t kGroupMax = 49152;
 
 template <int FORM, int SEM, int KT, bool CNT>
