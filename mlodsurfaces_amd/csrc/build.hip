@@ -398,7 +398,8 @@ __global__ __launch_bounds__(BS) void k_points(const float* __restrict__ xyz, co
                                                const uint32_t* __restrict__ order, uint32_t n,
                                                const uint32_t* __restrict__ pointLeaf, const float4* __restrict__ geo,
                                                const uint4* __restrict__ hdr, float4* __restrict__ pts,
-                                               float4* __restrict__ nrm, float* __restrict__ areaOrig) {
+                                               float4* __restrict__ nrm, float* __restrict__ areaOrig,
+                                               unsigned long long* __restrict__ nonfinite) {
   const uint32_t i = blockIdx.x * BS + threadIdx.x;
   if (i >= n) return;
   const uint32_t src = order[i];
@@ -406,9 +407,13 @@ __global__ __launch_bounds__(BS) void k_points(const float* __restrict__ xyz, co
   const float diag = __fmul_rn(geo[leaf].w, 2.0f);
   const float leafArea = __fmul_rn(diag, diag);
   const float a = (float)((double)leafArea / (double)hdr_count(hdr[leaf].y));  // correctly rounded f32 division
-  pts[i] = make_float4(xyz[3 * (uint64_t)src], xyz[3 * (uint64_t)src + 1], xyz[3 * (uint64_t)src + 2], a);
-  nrm[i] = make_float4(nrmIn[3 * (uint64_t)src], nrmIn[3 * (uint64_t)src + 1], nrmIn[3 * (uint64_t)src + 2], 0.f);
+  const float4 P = make_float4(xyz[3 * (uint64_t)src], xyz[3 * (uint64_t)src + 1], xyz[3 * (uint64_t)src + 2], a);
+  const float4 N = make_float4(nrmIn[3 * (uint64_t)src], nrmIn[3 * (uint64_t)src + 1], nrmIn[3 * (uint64_t)src + 2], 0.f);
+  pts[i] = P;
+  nrm[i] = N;
   areaOrig[src] = a;
+  const float z = 0.f * P.x + 0.f * P.y + 0.f * P.z + 0.f * N.x + 0.f * N.y + 0.f * N.z;  // NaN if one is not finite
+  if (z != 0.f) atomicAdd(nonfinite, 1ull);
 }
 
 // ----------------------------------------------------------------------------- moments
@@ -718,9 +723,9 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
   t->nn = (uint32_t)tot;
   const uint32_t nn = t->nn;
   uint32_t *nodeLast = nullptr, *pointLeaf = nullptr;
-  unsigned long long* dties = nullptr;
+  unsigned long long* dcount = nullptr;  // ties, points that are not finite
   float* areaOrig = nullptr;
-  if ((r = sc.alloc(&nodeLast, nn)) || (r = sc.alloc(&pointLeaf, n)) || (r = sc.alloc(&dties, 1)) ||
+  if ((r = sc.alloc(&nodeLast, nn)) || (r = sc.alloc(&pointLeaf, n)) || (r = sc.alloc(&dcount, 2)) ||
       (r = sc.alloc(&areaOrig, n)))
     return r;
   if ((r = dalloc(&t->geo, nn, &t->bytes)) || (r = dalloc(&t->hdr, nn, &t->bytes)) ||
@@ -730,14 +735,14 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
       (r = dalloc(&t->nrm, n, &t->bytes)) || (r = dalloc(&t->area, n, &t->bytes)) ||
       (r = dalloc(&t->span, nn, &t->bytes)))
     return r;
-  MLOD_HIP(hipMemsetAsync(dties, 0, sizeof(unsigned long long), s));
+  MLOD_HIP(hipMemsetAsync(dcount, 0, 2 * sizeof(unsigned long long), s));
   k_emit<<<nb, BS, 0, s>>>(codes2, t->order, d_xyz, n, maxDepth, W, nb, blockOff, lev, dbox, t->geo, t->hdr, t->box, nodeLast,
-                           pointLeaf, reinterpret_cast<uint32_t*>(t->span), dties);
+                           pointLeaf, reinterpret_cast<uint32_t*>(t->span), dcount);
   LAUNCH_CHECK();
   k_finalize<<<(nn + BS - 1) / BS, BS, 0, s>>>(nn, t->hdr, nodeLast);
   LAUNCH_CHECK();
   // 5. sorted points and areas
-  k_points<<<nb, BS, 0, s>>>(d_xyz, d_nrm, t->order, n, pointLeaf, t->geo, t->hdr, t->pts, t->nrm, t->area);
+  k_points<<<nb, BS, 0, s>>>(d_xyz, d_nrm, t->order, n, pointLeaf, t->geo, t->hdr, t->pts, t->nrm, t->area, dcount + 1);
   LAUNCH_CHECK();
   // 6. moments bottom-up
   for (int d = (int)t->depth; d >= 0; --d) {
@@ -746,10 +751,11 @@ int build_tree(mlod_tree* t, const float* d_xyz, const float* d_nrm, hipStream_t
     k_moments<<<(end - beg + BS - 1) / BS, BS, 0, s>>>(beg, end, t->hdr, t->geo, t->pts, t->nrm, t->recP, t->recC, t->momD, t->AD);
     LAUNCH_CHECK();
   }
-  unsigned long long hties = 0;
-  MLOD_HIP(hipMemcpyAsync(&hties, dties, sizeof(hties), hipMemcpyDeviceToHost, s));
+  unsigned long long hcount[2] = {0, 0};
+  MLOD_HIP(hipMemcpyAsync(hcount, dcount, sizeof(hcount), hipMemcpyDeviceToHost, s));
   MLOD_HIP(hipStreamSynchronize(s));
-  t->ties = hties;
+  t->ties = hcount[0];
+  t->finite = hcount[1] == 0;
   return MLOD_OK;
 }
 

@@ -121,6 +121,7 @@ struct mlod_tree {
   float bb[3] = {0, 0, 0}, BB[3] = {0, 0, 0};
   float radius = 0;
   uint64_t ties = 0;
+  bool finite = true;  // every point's position and normal is
   uint64_t bytes = 0;
   mlod_build_opts opts{12, 1, 0};
   // device buffers

@@ -426,8 +426,8 @@ __device__ __forceinline__ float box_box_d2(const float* __restrict__ box, uint3
 
 constexpr uint32_t kWaveScanPoints = 256;  // subtrees up to this size are taken as one range
 
-// The plain FP32 form: the reference's own sums, in FP32, 64 queries a wavefront, each point broadcast
-// lane to lane.
+// The plain FP32 form, and every form of a cloud with points that are not finite (see k_ball_sums): the form's own
+// sums one after another, 64 queries a wavefront, each point broadcast lane to lane.
 template <int FORM, int KT>
 __global__ __launch_bounds__(NBS) void k_ball_wave(TreeView tv, const float* __restrict__ box, KParams kp,
                                                    float4* __restrict__ q, float4* __restrict__ qn,
@@ -554,7 +554,9 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // instruction adds the 64 weights times the points' moments.  A pair so costs its distance, test and
 // weight and none of the nine sums.  The ranges and the steps within them are the tree's, whatever the
 // queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its wavefront's other
-// queries.  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
+// queries.  That holds for finite moments only (0 * NaN and 0 * infinity are NaN), so a cloud with a point that is
+// not finite goes to k_ball_wave, which leaves out what a ball does not hold (adding such points apart in this
+// kernel took 14 more registers, a wavefront a SIMD, and 7 % of every other cloud's time).  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
 // ones.  r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k 1.3;
 // FP64, 100k queries 1.6 (1.3 with weights.h's exponential).  Wavefronts of 64 queries (unions of four
 // times the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
@@ -743,10 +745,10 @@ int launch_form(mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t nIter,
     const double r2 = (double)r * (double)r;
     float r2f = (float)r2;
     if ((double)r2f > r2) r2f = nextafterf(r2f, 0.f);
-    if constexpr (FORM == 0)
+    if (FORM == 0 || !t->finite)
       k_ball_wave<FORM, KT><<<grid, NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
     else
-      k_ball_sums<FORM, KT><<<(m + kBallQ * (NBS / 64) - 1) / (kBallQ * (NBS / 64)), NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
+      k_ball_sums<FORM == 0 ? 1 : FORM, KT><<<(m + kBallQ * (NBS / 64) - 1) / (kBallQ * (NBS / 64)), NBS, 0, s>>>(t->view(), t->box, kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, r2f);
   }
   LAUNCH_CHECK();
   return MLOD_OK;
