@@ -161,6 +161,7 @@ __device__ __forceinline__ double root(double x) {
 // 2^y: y = k + f with |f| <= 1/2, 2^f by the Taylor series of exp(f log 2) to the 13th power (remainder
 // 4e-18), 0.86 ulp in all, as the library's exp, in 17 instructions against some 40.  y is finite (or NaN); a k out of range underflows in ldexp.
 __device__ __forceinline__ double pow2(double y) {
+#pragma clang fp contract(off)  // y is a product: f of the fused one is its rounding error, which is huge where y is
   const double t = __builtin_rint(y), f = y - t;
   double p = 1.3691488853904128e-12;
   p = fma(p, f, 2.5678435993488206e-11);

@@ -1,0 +1,35 @@
+"""Queries far beyond the cloud (sentinels of 1e19 to FLT_MAX among them), where squared distances leave the float range
+and every Gaussian underflows: the weights are then the kernel's constant shift, and the step goes towards the sphere of
+the whole cloud."""
+import numpy as np
+import pytest
+
+from gpu_util import gpu_project, gpu_tree
+from mlodsurfaces_amd import datasets as ds
+
+pytestmark = pytest.mark.gpu
+
+FM = np.finfo(np.float32).max
+FAR = np.array([[FM, FM, FM], [-FM, 0, 0], [0, FM, 0], [1e20, 0, 1e20], [1e19, 1e19, 0], [0, 1e17, 0], [1e12, 0, 2e12],
+                [100, 200, 50]], np.float32)
+
+
+@pytest.fixture(scope="module")
+def scene(oracle_built):
+    p, n = ds.torus(5000, seed=71)
+    return gpu_tree(p, n), oracle_built.OracleTree(p, n)
+
+
+@pytest.mark.parametrize("mode", ["mlod", "global"])
+@pytest.mark.parametrize("min_depth", [0, 2])
+@pytest.mark.parametrize("sigmas", [1, 2, 3, 5, 9, 10, 11, 30])
+def test_fp64_form(oracle_built, scene, sigmas, min_depth, mode):
+    tree, o = scene
+    k = dict(type=2, sigmas=[0.05 * 1.1 ** i for i in range(sigmas)], constant_shift=1e-3)
+    kw = dict(cutoff=2.0, min_depth=min_depth, semantics="ref_cpu" if mode == "global" else "ref_gpu", mode=mode)
+    got, nrm, _ = gpu_project(tree, FAR, k, precision="fp64", **kw)
+    ref, rn = o.project(FAR, oracle_built.make_kernel(**k), oracle_built.make_params(**kw), precision=1)
+    assert np.linalg.norm(rn, axis=1).min() > 0.99  # the definition gives every one of them a normal
+    scale = np.abs(FAR).max(1, keepdims=True).astype(np.float64)
+    assert (np.abs(got - ref) / scale).max() <= 2.4e-7  # a float32 unit in the last place or two of the largest coordinate
+    assert np.abs(nrm - rn).max() <= 2.4e-7
