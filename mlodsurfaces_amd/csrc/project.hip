@@ -1732,6 +1732,10 @@ KParams make_kparams(const mlod_kernel& k) {
       p.ad[s] = (double)(-1.44269504088896340736L / (2.0L * sg * sg));
       p.bd[s] = 1.0 / (sg * sg * sg);
     }
+    // the weights are formed two or four terms at a time: a term past the last is the first's exponential times 0
+    // (of a coefficient 0 it would be exp2(inf * 0), a NaN, where the squared distance overflows)
+    for (int s = p.ns; s < MLOD_MAX_SIGMAS; ++s) p.a[s] = p.a[0];
+    for (int s = p.ns; s < MLOD_MAX_SIGMAS + 1; ++s) p.ad[s] = p.ad[0];
   } else if (k.type == MLOD_KERNEL_GAUSSIAN) {
     const double sg = k.sigma;
     p.a[0] = (float)(-log2e / (2.0 * sg * sg));

@@ -48,7 +48,7 @@ __device__ __forceinline__ float weight32(const KP& k, float d2) {
     // sum over s of sigma_s^-3 * 2^(a_s d2), in order of s.  Statically indexed, so the coefficients
     // sit in scalar registers; two terms between wave-uniform exits (a scalar compare and branch;
     // the empty asm keeps the compiler from hoisting the compares into lane masks), so that two
-    // exponentials are in flight.  Coefficients past ns are zero: a term past the last adds 0 * 1
+    // exponentials are in flight.  A term past the last adds 0 times the first's exponential (make_kparams)
     float w = k.b[0] * __builtin_amdgcn_exp2f(d2 * k.a[0]);
     w = fmaf(k.b[1], __builtin_amdgcn_exp2f(d2 * k.a[1]), w);
     int ns = k.ns;
@@ -191,7 +191,7 @@ __device__ __forceinline__ double weight64(const KParams& k, double d2) {
   } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN_MULTIPLE) {
     d2 = d2 > 1e200 ? 1e200 : d2;  // (keeps a NaN; the exponents stay finite for every float sigma)
     double w = 0.0;
-    for (int s = 0; s < k.ns; s += 2) {  // two in flight; coefficients past ns are zero
+    for (int s = 0; s < k.ns; s += 2) {  // two in flight; bd is zero past ns
       const double e0 = pow2(d2 * k.ad[s]), e1 = pow2(d2 * k.ad[s + 1]);
       w = fma(e0, k.bd[s], w);
       w = fma(e1, k.bd[s + 1], w);

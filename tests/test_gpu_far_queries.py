@@ -33,3 +33,21 @@ def test_fp64_form(oracle_built, scene, sigmas, min_depth, mode):
     scale = np.abs(FAR).max(1, keepdims=True).astype(np.float64)
     assert (np.abs(got - ref) / scale).max() <= 2.4e-7  # a float32 unit in the last place or two of the largest coordinate
     assert np.abs(nrm - rn).max() <= 2.4e-7
+
+
+@pytest.mark.parametrize("mode,m", [("mlod", 5), ("mlod", 60000), ("knn", 5), ("global", 5)])  # (a batch of 5: eight lanes each)
+@pytest.mark.parametrize("precision", ["fp32", "fp32c"])
+def test_float_forms_take_any_number_of_sigmas(scene, precision, mode, m):
+    """The five farthest: every float squared distance overflows, the weights are the shift whatever the sigmas."""
+    tree, _ = scene
+    q = np.tile(FAR[:5], (m // 5, 1))
+    out = {}
+    for sigmas in (2, 1, 3, 5, 7, 8, 9, 10, 11, 12, 30, 32):
+        k = dict(type=2, sigmas=[0.05 * 1.1 ** i for i in range(sigmas)], constant_shift=1e-3)
+        out[sigmas] = gpu_project(tree, q, k, cutoff=2.0, semantics="ref_gpu" if mode == "mlod" else "ref_cpu",
+                                  precision=precision, mode=mode)[:2]
+    for sigmas, o in out.items():
+        for a, b in zip(o, out[2]):
+            assert np.array_equal(a.view(np.int32), b.view(np.int32)), sigmas
+    if precision == "fp32" and mode != "knn":  # (the other form's offsets overflow too, and knn's distances)
+        assert np.linalg.norm(out[2][1], axis=1).min() > 0.99
