@@ -583,7 +583,7 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
   float4* rc = recC + 4 * (uint64_t)k;
   rp[0] = g;
   // the walk's header: a leaf's depth gives way to a flag for a leaf of one point, the father to the
-  // reciprocal of A (correctly rounded for the plain form, held finite for a subnormal A, since quotients
+  // reciprocal of A, held finite for a subnormal A (correctly rounded for the plain form, since quotients
   // by A are formed from it; the hardware's for the other)
   const uint32_t code = !hdr_leaf(h.y) ? h.y : kLeafBit | (cnt == 1 ? kSingleBit : 0u) | cnt;
   const double rA = 1.0 / (double)sf.a;
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(BS) void k_moments(uint32_t beg, uint32_t end, uint
   rp[2] = make_float4(sf.px, sf.py, sf.pz, sf.pn);
   rp[3] = make_float4(sf.nx, sf.ny, sf.nz, sf.pp);
   rc[0] = g;
-  reinterpret_cast<uint4*>(rc)[1] = make_uint4(first, code, h.z, __float_as_uint(__builtin_amdgcn_rcpf(sf.a)));
+  reinterpret_cast<uint4*>(rc)[1] = make_uint4(first, code, h.z, __float_as_uint(fminf(__builtin_amdgcn_rcpf(sf.a), FLT_MAX)));
   rc[2] = make_float4(pb[0], pb[1], pb[2], Cc);
   rc[3] = make_float4(Nk[0].val(), Nk[1].val(), Nk[2].val(), Vc);
   momD[2 * (uint64_t)k] = make_double4(sd.px, sd.py, sd.pz, sd.pn);

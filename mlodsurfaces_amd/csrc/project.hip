@@ -23,6 +23,7 @@
 //   2 plain FP64   — everything in double.
 // Semantics (template SEM): 0 = REF_GPU (Fastapss.cu), 1 = REF_CPU (CPUUtils.cpp), see
 // mlod.h.  Weight kernels (template KT): Kernel.h:37 numbering.
+#include <cfloat>
 #include <cmath>
 
 #include "mlod_internal.h"
@@ -470,25 +471,26 @@ __device__ __forceinline__ uint32_t quad_lane(uint32_t v) {  // lane J of this l
 typedef const __attribute__((address_space(1))) void* GlobalPtr;
 typedef __attribute__((address_space(3))) void* LdsPtr;
 
-// BIG: 2^26 nodes or more, whose byte offsets need more than 32 bits
-template <int J, bool BIG>
+// WIDE: byte offsets of 64 bits (walk_narrow)
+template <int J, bool WIDE>
 __device__ __forceinline__ void stage_row(const char* rec, uint32_t idx, uint32_t lane, unsigned char* stage) {
   const uint32_t piece = (lane & 3u) * 16u;
-  const char* src = BIG ? rec + piece + (uint64_t)quad_lane<J>(idx) * 64u : rec + (quad_lane<J>(idx << 6) + piece);
+  const char* src = WIDE ? rec + piece + (uint64_t)quad_lane<J>(idx) * 64u : rec + (quad_lane<J>(idx << 6) + piece);
   __builtin_amdgcn_global_load_lds((GlobalPtr)src, (LdsPtr)(stage + J * kStageRow), 16, 0, 0);
 }
 // Starts the loads of record `idx` of every lane (all 64 lanes take part).
-template <bool BIG>
+template <bool WIDE>
 __device__ __forceinline__ void stage_issue(const float4* rec, uint32_t idx, uint32_t lane, unsigned char* stage) {
   const char* r = reinterpret_cast<const char*>(rec);
-  stage_row<0, BIG>(r, idx, lane, stage);
-  stage_row<1, BIG>(r, idx, lane, stage);
-  stage_row<2, BIG>(r, idx, lane, stage);
-  stage_row<3, BIG>(r, idx, lane, stage);
+  stage_row<0, WIDE>(r, idx, lane, stage);
+  stage_row<1, WIDE>(r, idx, lane, stage);
+  stage_row<2, WIDE>(r, idx, lane, stage);
+  stage_row<3, WIDE>(r, idx, lane, stage);
 }
 
 // Half a distance term that makes every blend factor 1 (a node above minDepth: no blending below it):
-// kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit.
+// kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit, and its shares are 0 (areas'
+// reciprocals are held finite).  Not so over an infinite distance: walk_narrow.
 constexpr float kNoBlend = 1e30f;
 
 __device__ __forceinline__ void swap_regs(float& a, float& b) { asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
@@ -497,6 +499,19 @@ __device__ __forceinline__ void swap_regs(float4& a, float4& b) {
 }
 __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
+// Whether a wavefront takes the narrow walk (uniform; the wide one gives the same bits): the tree has fewer than
+// 2^26 nodes, whose byte offsets fit 32 bits, and, in the plain form, no query is so far away that its distances
+// overflow and meets nodes without blending (the compensated form has no fit there: its sum of squared offsets
+// overflows too).
+template <int FORM>
+__device__ __forceinline__ bool walk_narrow(const TreeView& tv, V3<float> q, uint32_t minDepth, bool live) {
+  bool narrow = tv.nn < (1u << 26);
+  if constexpr (FORM == 0) {
+    if (minDepth) narrow = narrow && !any_lane(live && !(fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fabsf(q.z)) < 1e18f));
+  }
+  return narrow;
+}
+
 // What the walk relies on.  A near child's blend factor is exactly 1 (its distance is within its
 // cutoff, so t = dP / (dP + 0), at most one rounding off 1, and the hardware cosine at half a
 // revolution, and one float to either side of it, is exactly -1): the product of the factors on
@@ -504,7 +519,7 @@ __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballo
 // children in slot order, then its own (1 - b_c) share, then its first near child), and the
 // compensated form's block flushes come every kFlush iterations of the loop, which all lanes start
 // together, so a lane's sums depend on its own query only.
-template <int FORM, int SEM, int KT, bool CNT, bool BIG, class KP>
+template <int FORM, int SEM, int KT, bool CNT, bool WIDE, class KP>
 __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
                                                 V3<float> q, float cutoff, uint32_t minDepth, bool live,
                                                 WalkStack st, unsigned char* stage, int tid, Counters& ct) {
@@ -539,7 +554,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
   float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)hdr_count(h0.y)) : rec[1].w;
   NodeMom<FORM> own = load_mom<FORM>(tv, 0);
   const unsigned char* mine = stage + (lane & 3u) * kStageRow + (lane >> 2) * 64u;
-  stage_issue<BIG>(rec, x, lane, stage);
+  stage_issue<WIDE>(rec, x, lane, stage);
   while (any_lane(active != 0u)) {
 #pragma unroll 1
     for (uint32_t b = 0; b < kFlush && any_lane(active != 0u); ++b) {
@@ -560,6 +575,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
         // X's blend factor against its parent (CPUUtils.cpp:489-497); far: beyond its cutoff
         const float dc = fmaxf(over, 0.f);
         f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
+        if constexpr (FORM == 0 && WIDE) f = dh == kNoBlend ? 1.f : f;
         const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : quot_rcp(At, Ai, scale));
         shareSum = fmaf(share, 1.f - f, shareSum);
         const bool leaf = (int32_t)h.y < 0;
@@ -617,7 +633,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       }
       // the next record's loads go out before this one's terms are formed (it has been read by now)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      stage_issue<BIG>(rec, idx, lane, stage);
+      stage_issue<WIDE>(rec, idx, lane, stage);
       if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
       if (any_lane(multi)) {  // a leaf of several points (at the last level, or by the build's option)
         if (multi) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);
@@ -702,15 +718,15 @@ struct Record {
   uint4 h;
   float4 m0, m1;
 };
-template <bool BIG>
+template <bool WIDE>
 __device__ __forceinline__ Record load_record(const float4* rec, uint32_t idx) {
   const char* r = reinterpret_cast<const char*>(rec);
-  const char* src = BIG ? r + (uint64_t)idx * 64u : r + (idx << 6);
+  const char* src = WIDE ? r + (uint64_t)idx * 64u : r + (idx << 6);
   return Record{reinterpret_cast<const float4*>(src)[0], reinterpret_cast<const uint4*>(src)[1],
                 reinterpret_cast<const float4*>(src)[2], reinterpret_cast<const float4*>(src)[3]};
 }
 
-template <int FORM, int SEM, int KT, bool BIG, class KP>
+template <int FORM, int SEM, int KT, bool WIDE, class KP>
 __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, const TreeView& tv, V3<float> q, float cutoff,
                                                uint32_t minDepth, bool live, GroupLds& lds) {
 #pragma clang fp contract(off)  // the fused operations are written out
@@ -744,8 +760,9 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
   // the current node of the group
   uint32_t node = 0, first = h0.x, nc = active ? hdr_count(h0.y) : 0u, pend = 0, lvl = 0;
   float Ai = A0;
-  Record next = load_record<BIG>(rec, first + (c < nc ? c : 0u));  // the lane's child
+  Record next = load_record<WIDE>(rec, first + (c < nc ? c : 0u));  // the lane's child
   NodeMom<FORM> own = load_mom<FORM>(tv, node);
+  float rA = rec[4 * (size_t)node + 1].w;  // the reciprocal of its area
   while (any_lane(active != 0u)) {
     const float4 g = next.g;
     const uint4 h = next.h;
@@ -755,7 +772,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     if constexpr (FORM == 0) mm.rA = __uint_as_float(h.w);
     // the node that is summed below
     const uint32_t ncP = nc;
-    const float AiP = Ai, dhP = dh;
+    const float AiP = Ai, dhP = dh, rAP = rA;
     const NodeMom<FORM> ownP = own;
     const bool mineP = c < ncP, activeP = active != 0u;
     // --- near children, and the next node
@@ -792,17 +809,19 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
       Ai = e.A;
       lvl = L + 1u;
     }
-    next = load_record<BIG>(rec, first + (c < nc ? c : 0u));
+    next = load_record<WIDE>(rec, first + (c < nc ? c : 0u));
     own = load_mom<FORM>(tv, node);
+    rA = rec[4 * (size_t)node + 1].w;
     // --- the sums of the node that was tested
-    const float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
+    float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
+    if constexpr (FORM == 0 && WIDE) f = dhP == kNoBlend ? 1.f : f;
     float share;
     if constexpr (SEM == MLOD_SEM_REF_CPU)
       share = tratio<FORM>(1.f, (float)ncP);
     else if constexpr (FORM == 1)
-      share = At * tratio<FORM>(1.f, AiP);
+      share = At * rAP;
     else
-      share = quot_rcp(At, AiP, ownP.rA);
+      share = quot_rcp(At, AiP, rAP);
     const bool contrib = mineP && (far || single), multi = mineP && leaf && !single;
     {
       float2 p[10];
@@ -907,7 +926,7 @@ __device__ __forceinline__ void traverse(typename FormT<FORM>::Acc& acc, const K
   } else {
     const WalkStack st{lds.first, lds.mask};
     unsigned char* stage = lds.stage[__builtin_amdgcn_readfirstlane(tid >> 6)];
-    if (tv.nn < (1u << 26))
+    if (walk_narrow<FORM>(tv, q, minDepth, live))
       traverse_staged<FORM, SEM, KT, CNT, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
     else
       traverse_staged<FORM, SEM, KT, CNT, true>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
@@ -1325,7 +1344,7 @@ __global__ __launch_bounds__(64) void k_project_group(TreeView tv, KParams kp, f
     GroupSums gs;
     gs.init();
     const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
-    if (tv.nn < (1u << 26))
+    if (walk_narrow<FORM>(tv, qf, minDepth, live))
       traverse_group<FORM, SEM, KT, false>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
     else
       traverse_group<FORM, SEM, KT, true>(gs, kp, tv, qf, cutoff, minDepth, live, lds);

@@ -51,3 +51,23 @@ def test_float_forms_take_any_number_of_sigmas(scene, precision, mode, m):
             assert np.array_equal(a.view(np.int32), b.view(np.int32)), sigmas
     if precision == "fp32" and mode != "knn":  # (the other form's offsets overflow too, and knn's distances)
         assert np.linalg.norm(out[2][1], axis=1).min() > 0.99
+
+
+@pytest.mark.parametrize("semantics", ["ref_gpu", "ref_cpu"])
+@pytest.mark.parametrize("precision", ["fp32", "fp32c"])
+@pytest.mark.parametrize("min_depth", [1, 2, 13])
+@pytest.mark.parametrize("scale", [0, -62])  # at -62 the nodes' areas are subnormal: their reciprocals overflow
+def test_no_blending_above_the_min_depth(scale, min_depth, precision, semantics):
+    """Infinite distances, and areas without a reciprocal, against the wave walk, which keeps such nodes' factors apart."""
+    s = np.float32(2.0) ** scale
+    p, n = ds.torus(5000, seed=71)
+    tree = gpu_tree(p * s, n)
+    q = np.concatenate([FAR, ds.jitter_queries(p[:20], 0.02, seed=72) * s])
+    kw = dict(kernel=dict(type=0, sigma=float(0.05 * s), constant_shift=1e-3), min_depth=min_depth, semantics=semantics,
+              precision=precision)
+    ref = gpu_project(tree, q, traversal="wave", **kw)[:2]
+    for m in (1, 2000):  # eight lanes a query; one
+        got = gpu_project(tree, np.tile(q, (m, 1)), **kw)[:2]
+        # the two walks add the same terms in the same order, but may fuse a multiply-add differently
+        assert np.abs(got[1][:len(q)] - ref[1]).max() <= 1e-4
+        assert (np.abs(got[0][:len(q)].astype(np.float64) - ref[0]) / np.abs(q).max(1, keepdims=True)).max() <= 1e-6
