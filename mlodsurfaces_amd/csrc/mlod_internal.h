@@ -68,6 +68,7 @@ struct alignas(16) KParams {
   float c;           // constant_shift
   float cp;          // max(c, 1e-4)
   float e;           // exponent
+  float c4, cp4;     // c / 4, cp / 4
   double ad[MLOD_MAX_SIGMAS + 1];  // FP64: -log2(e) / (2 s^2)  (read two at a time)
   double bd[MLOD_MAX_SIGMAS + 1];  // FP64: 1 / s^3
   double cpe;        // FP64: cp^e

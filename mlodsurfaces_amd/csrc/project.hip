@@ -1739,6 +1739,8 @@ KParams make_kparams(const mlod_kernel& k) {
   p.c = k.constant_shift;
   p.cp = k.constant_shift > 0.0001f ? k.constant_shift : 0.0001f;
   p.e = k.exponent;
+  p.c4 = 0.25f * p.c;
+  p.cp4 = 0.25f * p.cp;
   const double er = std::nearbyint((double)k.exponent);
   p.cpe = std::pow((double)p.cp, (double)p.e);
   p.eint = (er == (double)k.exponent && er >= 1.0 && er <= 16.0) ? (int)er : -1;

@@ -13,8 +13,8 @@ namespace {
 // 8.1 ms a step, the same bits).  An approximation within an ulp, its residual by one fused operation,
 // which is exact, and one fused correction (Markstein, "Computation of elementary functions on the IBM
 // RISC System/6000 processor", 1990).  The expansions spend the rest on operands at the ends of the
-// exponent range.  Here the divisor is zero or at least 2^-126 (a smaller one's reciprocal overflows),
-// and the quotient is right where it and the residual are normal (above some 2^-100), and within an ulp
+// exponent range.  Here the divisor is zero, from 2^-126 to 2^126 (a smaller one's reciprocal overflows, a larger one's is flushed) or
+// infinite, and the quotient is right where it and the residual are normal (above some 2^-100), and within an ulp
 // below; zeros, infinities and NaN go through the hardware's fix-up.  The square root is right from 2^-100 on,
 // checked for every float there; below it loses up to an ulp, and a subnormal argument (a distance
 // under 1e-19) is returned as it is.
@@ -82,14 +82,13 @@ __device__ __forceinline__ float weight32(const KP& k, float d2) {
   } else if constexpr (KT == MLOD_KERNEL_GAUSSIAN) {
     return __builtin_amdgcn_exp2f(d2 * k.a[0]) + k.c;
   } else {
-    const float den = d2 + k.c;
     float base;
-    if ((__float_as_uint(k.c) & 0x7fffffffu) > 0x0da24260u) {  // |c| > 1e-30: den is no subnormal (uniform)
+    if ((__float_as_uint(k.c) & 0x7fffffffu) > 0x0da24260u) {  // |c| > 1e-30: the divisor is no subnormal (uniform)
       asm volatile("");
-      base = quot(k.cp, den);
+      base = quot(k.cp4, fmaf(d2, 0.25f, k.c4));  // both a quarter: the largest divisor has a normal reciprocal too
     } else {
       asm volatile("");
-      base = k.cp / den;
+      base = k.cp / (d2 + k.c);
     }
     if (k.eint > 0) {
       float r = 1.f, b = base;

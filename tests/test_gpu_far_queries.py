@@ -71,3 +71,22 @@ def test_no_blending_above_the_min_depth(scale, min_depth, precision, semantics)
         # the two walks add the same terms in the same order, but may fuse a multiply-add differently
         assert np.abs(got[1][:len(q)] - ref[1]).max() <= 1e-4
         assert (np.abs(got[0][:len(q)].astype(np.float64) - ref[0]) / np.abs(q).max(1, keepdims=True)).max() <= 1e-6
+
+
+@pytest.mark.parametrize("exponent", [1.0, 4.0, 2.5])
+@pytest.mark.parametrize("precision", ["fp32", "fp32c"])
+def test_rational_weights_near_the_end_of_the_float_range(precision, exponent):
+    """Squared distances between 2^126 and 2^128, whose reciprocals are subnormal: a large cloud (2^58 across) with a
+    shift of its scale, the nearest points of queries 1.1e19 to 1.7e19 away: weights and a fit as in the FP64 form."""
+    s = np.float32(2.0) ** 58
+    p, n = ds.torus(3000, seed=73)
+    p = p * s
+    shift = float(np.float32(8e31))
+    u = np.random.default_rng(74).standard_normal((16, 3))
+    u /= np.linalg.norm(u, axis=1, keepdims=True)
+    q = (u * np.linspace(1.1e19, 1.7e19, 16)[:, None]).astype(np.float32)
+    got, _, _ = gpu_project(gpu_tree(p, n), q, dict(type=1, exponent=exponent, constant_shift=shift), mode="knn", knn=20,
+                            precision="fp64")
+    out, nrm, _ = gpu_project(gpu_tree(p, n), q, dict(type=1, exponent=exponent, constant_shift=shift), mode="knn", knn=20,
+                              precision=precision)
+    assert np.isfinite(got).all() and np.isfinite(out).all() and np.linalg.norm(nrm, axis=1).min() > 0.99
