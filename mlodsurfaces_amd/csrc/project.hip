@@ -123,6 +123,29 @@ struct Counters {
   uint32_t far_, leafPts, tested, nearN, iters;
 };
 
+// A point's mean position (a p) / a in the plain form.  Areas here have any exponent (a subnormal one's reciprocal
+// overflows, that of one above 2^126 is flushed), so the divisions are the compiler's.
+__device__ __forceinline__ V3<float> point_mean(float4 P) {
+  return V3<float>{(P.w * P.x) / P.w, (P.w * P.y) / P.w, (P.w * P.z) / P.w};
+}
+template <int KT, class KP>
+__device__ __forceinline__ void add_point_plain(AccP32& acc, const KP& kp, float4 P, float4 N, V3<float> mean, V3<float> q,
+                                                float f) {
+  const float a = P.w;
+  const float apx = a * P.x, apy = a * P.y, apz = a * P.z;
+  const float dx = mean.x - q.x, dy = mean.y - q.y, dz = mean.z - q.z;
+  const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
+  acc.w = fmaf(w, a, acc.w);
+  acc.px = fmaf(w, apx, acc.px);
+  acc.py = fmaf(w, apy, acc.py);
+  acc.pz = fmaf(w, apz, acc.pz);
+  acc.nx = fmaf(w, a * N.x, acc.nx);
+  acc.ny = fmaf(w, a * N.y, acc.ny);
+  acc.nz = fmaf(w, a * N.z, acc.nz);
+  acc.pn = fmaf(w, a * (P.x * N.x + P.y * N.y + P.z * N.z), acc.pn);
+  acc.pp = fmaf(w, a * (P.x * P.x + P.y * P.y + P.z * P.z), acc.pp);
+}
+
 // Contribution of one point (leaf member) with multiplier f, weight at the point's mean
 // position (a p) / a (Fastapss.cu:193; CPUUtils.cpp:455).
 template <int FORM, int KT, class KP>
@@ -130,19 +153,7 @@ __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const 
                                           V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
   const float4 P = tv.pts[j], N = tv.nrm[j];
   if constexpr (FORM == 0) {
-    const float a = P.w;
-    const float apx = a * P.x, apy = a * P.y, apz = a * P.z;
-    const float dx = quot(apx, a) - q.x, dy = quot(apy, a) - q.y, dz = quot(apz, a) - q.z;
-    const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
-    acc.w = fmaf(w, a, acc.w);
-    acc.px = fmaf(w, apx, acc.px);
-    acc.py = fmaf(w, apy, acc.py);
-    acc.pz = fmaf(w, apz, acc.pz);
-    acc.nx = fmaf(w, a * N.x, acc.nx);
-    acc.ny = fmaf(w, a * N.y, acc.ny);
-    acc.nz = fmaf(w, a * N.z, acc.nz);
-    acc.pn = fmaf(w, a * (P.x * N.x + P.y * N.y + P.z * N.z), acc.pn);
-    acc.pp = fmaf(w, a * (P.x * P.x + P.y * P.y + P.z * P.z), acc.pp);
+    add_point_plain<KT>(acc, kp, P, N, point_mean(P), q, f);
   } else if constexpr (FORM == 1) {
     // the fused operations are written out: every kernel that adds a point rounds alike
     const float dx = P.x - q.x, dy = P.y - q.y, dz = P.z - q.z;
@@ -182,14 +193,6 @@ template <int FORM> struct NodeMom { float4 m0, m1; };
 template <> struct NodeMom<0> { float4 m0, m1; float rA; };  // rA = 1 / A, correctly rounded
 template <> struct NodeMom<2> { double4 m0, m1; double A; };
 
-// Record `idx` of `bytes` bytes from `base`, with the byte offset formed in 32 bits (the tree
-// build guarantees node counts below 2^27), so the address is a scalar base plus one 32-bit
-// vector offset instead of 64-bit vector arithmetic.
-template <class T>
-__device__ __forceinline__ T ld_rec(const T* base, uint32_t idx) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (idx * (uint32_t)sizeof(T)));
-}
-
 template <int FORM>
 __device__ __forceinline__ NodeMom<FORM> load_mom(const TreeView& tv, uint32_t c) {
   NodeMom<FORM> r;
@@ -206,13 +209,20 @@ __device__ __forceinline__ NodeMom<FORM> load_mom(const TreeView& tv, uint32_t c
 }
 
 // Contribution of a node's moments with multiplier f, weight at its mean point.
-template <int FORM, int KT, class KP>
+// n / A from the stored reciprocal of A.  EXACT (trees whose areas may be subnormal, see walk_short): the
+// compiler's division.
+template <bool EXACT>
+__device__ __forceinline__ float quot_area(float n, float A, float rA) {
+  return EXACT ? n / A : quot_rcp(n, A, rA);
+}
+
+template <int FORM, int KT, bool EXACT = false, class KP>
 __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP& kp, const NodeMom<FORM>& mm, float Af,
                                         V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
   if constexpr (FORM == 0) {
     const float4 m0 = mm.m0, m1 = mm.m1;
-    const float dx = quot_rcp(m0.x, Af, mm.rA) - q.x, dy = quot_rcp(m0.y, Af, mm.rA) - q.y,
-                dz = quot_rcp(m0.z, Af, mm.rA) - q.z;
+    const float dx = quot_area<EXACT>(m0.x, Af, mm.rA) - q.x, dy = quot_area<EXACT>(m0.y, Af, mm.rA) - q.y,
+                dz = quot_area<EXACT>(m0.z, Af, mm.rA) - q.z;
     const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     acc.w = fmaf(w, Af, acc.w);
     acc.px = fmaf(w, m0.x, acc.px);
@@ -258,12 +268,12 @@ __device__ __forceinline__ void add_mom(typename FormT<FORM>::Acc& acc, const KP
 
 // add_mom as the (factor, value) pairs of its nine fused operations, in the order of the sums
 // (FP32 forms; the same roundings).
-template <int FORM, int KT, class KP>
+template <int FORM, int KT, bool EXACT, class KP>
 __device__ __forceinline__ void mom_pairs(float2* p, const KP& kp, const NodeMom<FORM>& mm, float Af, V3<float> q, float f) {
   const float4 m0 = mm.m0, m1 = mm.m1;
   if constexpr (FORM == 0) {
-    const float dx = quot_rcp(m0.x, Af, mm.rA) - q.x, dy = quot_rcp(m0.y, Af, mm.rA) - q.y,
-                dz = quot_rcp(m0.z, Af, mm.rA) - q.z;
+    const float dx = quot_area<EXACT>(m0.x, Af, mm.rA) - q.x, dy = quot_area<EXACT>(m0.y, Af, mm.rA) - q.y,
+                dz = quot_area<EXACT>(m0.z, Af, mm.rA) - q.z;
     const float w = f * weight32<KT>(kp, fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy))));
     p[0] = make_float2(w, Af);
     p[1] = make_float2(w, m0.x), p[2] = make_float2(w, m0.y), p[3] = make_float2(w, m0.z);
@@ -282,10 +292,10 @@ __device__ __forceinline__ void mom_pairs(float2* p, const KP& kp, const NodeMom
   }
 }
 
-template <int FORM, int KT, class KP>
+template <int FORM, int KT, bool EXACT = false, class KP>
 __device__ __forceinline__ void add_node(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv, uint32_t c,
                                          float Af, V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
-  add_mom<FORM, KT>(acc, kp, load_mom<FORM>(tv, c), Af, q, f);
+  add_mom<FORM, KT, EXACT>(acc, kp, load_mom<FORM>(tv, c), Af, q, f);
 }
 
 template <int FORM, int SEM, int KT, bool CNT, class KP>
@@ -306,21 +316,23 @@ __device__ __forceinline__ void add_leaf(typename FormT<FORM>::Acc& acc, const K
 // Traversal arithmetic per form.  The plain forms keep correctly rounded division and square root
 // (the reference's arithmetic); the compensated form, whose error budget is set by its FP64 fit and
 // compensated sums, takes the hardware reciprocal and square root (1 ulp).
-template <int FORM>
+template <int FORM, bool EXACT = false>
 __device__ __forceinline__ typename FormT<FORM>::T tdist(V3<typename FormT<FORM>::T> q, float4 g) {
   if constexpr (FORM != 2) {  // (the fused operations written out: every kernel rounds alike)
     const float dx = q.x - g.x, dy = q.y - g.y, dz = q.z - g.z;
     const float d2 = fmaf(dz, dz, fmaf(dx, dx, __fmul_rn(dy, dy)));
-    return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : root(d2);
+    return FORM == 1 ? __builtin_amdgcn_sqrtf(d2) : EXACT ? fsqrt(d2) : root(d2);
   } else {
     const double dx = q.x - (double)g.x, dy = q.y - (double)g.y, dz = q.z - (double)g.z;
     return root(dx * dx + dy * dy + dz * dz);
   }
 }
-template <int FORM, class T>
+template <int FORM, bool EXACT = false, class T>
 __device__ __forceinline__ T tratio(T a, T b) {  // a / b
   if constexpr (FORM == 1)
     return a * __builtin_amdgcn_rcpf(b);
+  else if constexpr (EXACT)
+    return a / b;
   else
     return quot(a, b);
 }
@@ -471,7 +483,7 @@ __device__ __forceinline__ uint32_t quad_lane(uint32_t v) {  // lane J of this l
 typedef const __attribute__((address_space(1))) void* GlobalPtr;
 typedef __attribute__((address_space(3))) void* LdsPtr;
 
-// WIDE: byte offsets of 64 bits (walk_narrow)
+// WIDE: 2^26 nodes or more, whose byte offsets need more than 32 bits
 template <int J, bool WIDE>
 __device__ __forceinline__ void stage_row(const char* rec, uint32_t idx, uint32_t lane, unsigned char* stage) {
   const uint32_t piece = (lane & 3u) * 16u;
@@ -490,7 +502,7 @@ __device__ __forceinline__ void stage_issue(const float4* rec, uint32_t idx, uin
 
 // Half a distance term that makes every blend factor 1 (a node above minDepth: no blending below it):
 // kNoBlend / (2 kNoBlend + anything a cloud spans) is 1/2 to the last bit, and its shares are 0 (areas'
-// reciprocals are held finite).  Not so over an infinite distance: walk_narrow.
+// reciprocals are held finite).  Not so over an infinite distance: walk_short.
 constexpr float kNoBlend = 1e30f;
 
 __device__ __forceinline__ void swap_regs(float& a, float& b) { asm("v_swap_b32 %0, %1" : "+v"(a), "+v"(b)); }
@@ -499,17 +511,23 @@ __device__ __forceinline__ void swap_regs(float4& a, float4& b) {
 }
 __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
-// Whether a wavefront takes the narrow walk (uniform; the wide one gives the same bits): the tree has fewer than
-// 2^26 nodes, whose byte offsets fit 32 bits, and, in the plain form, no query is so far away that its distances
-// overflow and meets nodes without blending (the compensated form has no fit there: its sum of squared offsets
+// Whether no node of the tree has a subnormal area: a point's is its leaf's squared diagonal, at most 2^-12 of the
+// root's (2 r), over the leaf's points.
+__device__ __forceinline__ bool areas_normal(const TreeView& tv) {
+  const float r = tv.geo[0].w;
+  return r * r >= (float)tv.n * 0x1p-104f;
+}
+// Whether a wavefront's plain walk may take the short quotients and roots and the large distance term (uniform):
+// the areas have normal reciprocals, and no query is so far away that its distances overflow and meets nodes
+// without blending.  The other walk (EXACT) holds everywhere and gives the same bits.  The compensated form has one
+// walk: it takes the hardware's reciprocals, and has no fit for such a query (its sum of squared offsets
 // overflows too).
 template <int FORM>
-__device__ __forceinline__ bool walk_narrow(const TreeView& tv, V3<float> q, uint32_t minDepth, bool live) {
-  bool narrow = tv.nn < (1u << 26);
-  if constexpr (FORM == 0) {
-    if (minDepth) narrow = narrow && !any_lane(live && !(fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fabsf(q.z)) < 1e18f));
-  }
-  return narrow;
+__device__ __forceinline__ bool walk_short(const TreeView& tv, V3<float> q, uint32_t minDepth, bool live) {
+  if constexpr (FORM == 1) return true;
+  bool ok = areas_normal(tv);
+  if (minDepth) ok = ok && !any_lane(live && !(fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fabsf(q.z)) < 1e18f));
+  return ok;
 }
 
 // What the walk relies on.  A near child's blend factor is exactly 1 (its distance is within its
@@ -519,7 +537,7 @@ __device__ __forceinline__ bool walk_narrow(const TreeView& tv, V3<float> q, uin
 // children in slot order, then its own (1 - b_c) share, then its first near child), and the
 // compensated form's block flushes come every kFlush iterations of the loop, which all lanes start
 // together, so a lane's sums depend on its own query only.
-template <int FORM, int SEM, int KT, bool CNT, bool WIDE, class KP>
+template <int FORM, int SEM, int KT, bool CNT, bool WIDE, bool EXACT, class KP>
 __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv,
                                                 V3<float> q, float cutoff, uint32_t minDepth, bool live,
                                                 WalkStack st, unsigned char* stage, int tid, Counters& ct) {
@@ -537,11 +555,11 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
   uint32_t active = live ? 1u : 0u;  // (a word: one compare makes the wavefront's mask of it)
   float dh = kNoBlend;  // half the current node's distance term
   if (minDepth == 0) {
-    const float d0 = tdist<FORM>(q, g0), rc = g0.w * cutoff;
+    const float d0 = tdist<FORM, EXACT>(q, g0), rc = g0.w * cutoff;
     dh = 0.5f * fabsf(d0 - rc);
     if (d0 > rc) {
       if (live) {
-        add_node<FORM, KT>(acc, kp, tv, 0, __uint_as_float(h0.z), q, 1.f);
+        add_node<FORM, KT, EXACT>(acc, kp, tv, 0, __uint_as_float(h0.z), q, 1.f);
         if constexpr (CNT) ct.far_ += 1;
       }
       active = 0u;
@@ -551,7 +569,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
   uint32_t first = h0.x, x = first, xEnd = active ? first + hdr_count(h0.y) : first, mask = 0, pend = 0;
   int lvl = 0;
   float Ai = __uint_as_float(h0.z), shareSum = 0.f;
-  float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)hdr_count(h0.y)) : rec[1].w;
+  float scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM, EXACT>(1.f, (float)hdr_count(h0.y)) : rec[1].w;
   NodeMom<FORM> own = load_mom<FORM>(tv, 0);
   const unsigned char* mine = stage + (lane & 3u) * kStageRow + (lane >> 2) * 64u;
   stage_issue<WIDE>(rec, x, lane, stage);
@@ -568,15 +586,15 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       mm.m1 = *reinterpret_cast<const float4*>(mine + 48);
       if constexpr (FORM == 0) mm.rA = __uint_as_float(h.w);
       float At = __uint_as_float(h.z);
-      const float over = tdist<FORM>(q, g) - g.w * cutoff;
+      const float over = tdist<FORM, EXACT>(q, g) - g.w * cutoff;
       bool contrib = false, multi = false;
       float f = 0.f;
       if (x < xEnd) {
         // X's blend factor against its parent (CPUUtils.cpp:489-497); far: beyond its cutoff
         const float dc = fmaxf(over, 0.f);
-        f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
-        if constexpr (FORM == 0 && WIDE) f = dh == kNoBlend ? 1.f : f;
-        const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : quot_rcp(At, Ai, scale));
+        f = fmaf(__builtin_amdgcn_cosf(tratio<FORM, EXACT>(dh, fmaf(2.f, dh, dc))), -0.5f, 0.5f);
+        if constexpr (EXACT) f = dh == kNoBlend ? 1.f : f;
+        const float share = SEM == MLOD_SEM_REF_CPU ? scale : (FORM == 1 ? At * scale : quot_area<EXACT>(At, Ai, scale));
         shareSum = fmaf(share, 1.f - f, shareSum);
         const bool leaf = (int32_t)h.y < 0;
         const bool single = h.y >= (kLeafBit | kSingleBit);
@@ -608,7 +626,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
           asm volatile("");  // (a uniform branch, not a select)
           dh = (int32_t)h.y >= blendKey ? dh : kNoBlend;
         }
-        scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(1.f, (float)(h.y & 15u)) : __uint_as_float(h.w);
+        scale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM, EXACT>(1.f, (float)(h.y & 15u)) : __uint_as_float(h.w);
       }
       uint32_t idx = x;
       if (active && x == xEnd) {
@@ -634,7 +652,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       // the next record's loads go out before this one's terms are formed (it has been read by now)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       stage_issue<WIDE>(rec, idx, lane, stage);
-      if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
+      if (contrib) add_mom<FORM, KT, EXACT>(acc, kp, mm, At, q, f);
       if (any_lane(multi)) {  // a leaf of several points (at the last level, or by the build's option)
         if (multi) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);
       }
@@ -726,7 +744,7 @@ __device__ __forceinline__ Record load_record(const float4* rec, uint32_t idx) {
                 reinterpret_cast<const float4*>(src)[2], reinterpret_cast<const float4*>(src)[3]};
 }
 
-template <int FORM, int SEM, int KT, bool WIDE, class KP>
+template <int FORM, int SEM, int KT, bool WIDE, bool EXACT, class KP>
 __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, const TreeView& tv, V3<float> q, float cutoff,
                                                uint32_t minDepth, bool live, GroupLds& lds) {
 #pragma clang fp contract(off)  // the fused operations are written out
@@ -750,10 +768,10 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
   uint32_t active = live ? 1u : 0u;
   float dh = kNoBlend;
   if (minDepth == 0) {
-    const float d0 = tdist<FORM>(q, g0), rc = g0.w * cutoff;
+    const float d0 = tdist<FORM, EXACT>(q, g0), rc = g0.w * cutoff;
     dh = 0.5f * fabsf(d0 - rc);
     if (d0 > rc) {
-      if (live) single_term([&](auto& a) { add_node<FORM, KT>(a, kp, tv, 0, A0, q, 1.f); });
+      if (live) single_term([&](auto& a) { add_node<FORM, KT, EXACT>(a, kp, tv, 0, A0, q, 1.f); });
       active = 0u;
     }
   }
@@ -776,7 +794,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     const NodeMom<FORM> ownP = own;
     const bool mineP = c < ncP, activeP = active != 0u;
     // --- near children, and the next node
-    const float over = tdist<FORM>(q, g) - g.w * cutoff;
+    const float over = tdist<FORM, EXACT>(q, g) - g.w * cutoff;
     const bool leaf = (int32_t)h.y < 0, single = h.y >= (kLeafBit | kSingleBit);
     const bool far = (int32_t)h.y >= blendKey && over > 0.f;
     const bool near = mineP && !leaf && !far;
@@ -813,21 +831,21 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     own = load_mom<FORM>(tv, node);
     rA = rec[4 * (size_t)node + 1].w;
     // --- the sums of the node that was tested
-    float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
-    if constexpr (FORM == 0 && WIDE) f = dhP == kNoBlend ? 1.f : f;
+    float f = fmaf(__builtin_amdgcn_cosf(tratio<FORM, EXACT>(dhP, fmaf(2.f, dhP, fmaxf(over, 0.f)))), -0.5f, 0.5f);
+    if constexpr (EXACT) f = dhP == kNoBlend ? 1.f : f;
     float share;
     if constexpr (SEM == MLOD_SEM_REF_CPU)
-      share = tratio<FORM>(1.f, (float)ncP);
+      share = tratio<FORM, EXACT>(1.f, (float)ncP);
     else if constexpr (FORM == 1)
       share = At * rAP;
     else
-      share = quot_rcp(At, AiP, rAP);
+      share = quot_area<EXACT>(At, AiP, rAP);
     const bool contrib = mineP && (far || single), multi = mineP && leaf && !single;
     {
       float2 p[10];
 #pragma unroll
       for (int t = 0; t < 10; ++t) p[t] = make_float2(0.f, 0.f);
-      if (contrib) mom_pairs<FORM, KT>(p, kp, mm, At, q, f);
+      if (contrib) mom_pairs<FORM, KT, EXACT>(p, kp, mm, At, q, f);
       if (mineP) p[9] = make_float2(share, 1.f - f);
       float4* out = reinterpret_cast<float4*>(lds.pair[lane]);
 #pragma unroll
@@ -892,7 +910,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     }
     if constexpr (FORM == 1) gs.cnt = terms >= kFlush ? terms - kFlush : terms;
     if (activeP) {
-      if (shareSum != 0.f) single_term([&](auto& x) { add_mom<FORM, KT>(x, kp, ownP, AiP, q, shareSum); });
+      if (shareSum != 0.f) single_term([&](auto& x) { add_mom<FORM, KT, EXACT>(x, kp, ownP, AiP, q, shareSum); });
       if constexpr (FORM == 1) {
         if (++gs.cnt == kFlush) gs.template flush<FORM>();
       }
@@ -926,10 +944,12 @@ __device__ __forceinline__ void traverse(typename FormT<FORM>::Acc& acc, const K
   } else {
     const WalkStack st{lds.first, lds.mask};
     unsigned char* stage = lds.stage[__builtin_amdgcn_readfirstlane(tid >> 6)];
-    if (walk_narrow<FORM>(tv, q, minDepth, live))
-      traverse_staged<FORM, SEM, KT, CNT, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
+    if (!walk_short<FORM>(tv, q, minDepth, live))
+      traverse_staged<FORM, SEM, KT, CNT, true, FORM == 0>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
+    else if (tv.nn < (1u << 26))
+      traverse_staged<FORM, SEM, KT, CNT, false, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
     else
-      traverse_staged<FORM, SEM, KT, CNT, true>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
+      traverse_staged<FORM, SEM, KT, CNT, true, false>(acc, kp, tv, q, cutoff, minDepth, live, st, stage, tid, ct);
   }
 }
 
@@ -985,7 +1005,7 @@ __device__ __forceinline__ NodeMom<FORM> load_mom_uni(const TreeView& tv, uint32
   return r;
 }
 
-template <int FORM, int SEM, int KT, bool CNT>
+template <int FORM, int SEM, int KT, bool CNT, bool EXACT>
 __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, const KParams& kp, const TreeView& tv,
                                               V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T cutoff,
                                               uint32_t minDepth, bool live, WaveStack<typename FormT<FORM>::T> st,
@@ -1004,9 +1024,9 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
   T m = T(1), distP = T(-1), shareSum = T(0);
   uint32_t nearb = 0;
   if (act) {
-    const T d0 = tdist<FORM>(q, g0);
+    const T d0 = tdist<FORM, EXACT>(q, g0);
     if (minDepth == 0 && d0 > (T)g0.w * cutoff) {
-      add_mom<FORM, KT>(acc, kp, load_mom_uni<FORM>(tv, 0u), __uint_as_float(h0.z), q, T(1));
+      add_mom<FORM, KT, EXACT>(acc, kp, load_mom_uni<FORM>(tv, 0u), __uint_as_float(h0.z), q, T(1));
       if constexpr (CNT) ct.far_ += 1;
       act = false;
     } else {
@@ -1019,7 +1039,7 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
   uint32_t first = h0.x, nc = hdr_count(h0.y), k = 0, un = 0, pend = 0;
   int lvl = 0;
   float Ai = __uint_as_float(h0.z);
-  T shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(T(1), (T)nc) : tratio<FORM>(T(1), (T)Ai);
+  T shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM, EXACT>(T(1), (T)nc) : tratio<FORM, EXACT>(T(1), (T)Ai);
   NodeMom<FORM> momX = load_mom_uni<FORM>(tv, 0);
   while (true) {
     if constexpr (CNT) ++waveIters;
@@ -1042,13 +1062,13 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
       bool nearc = false;
       if (act) {
         if constexpr (CNT) ct.iters += 1, ct.tested += 1;
-        const T dxq = tdist<FORM>(q, gx);
+        const T dxq = tdist<FORM, EXACT>(q, gx);
         const T rc = (T)gx.w * cutoff;
         const T dp = blendNode ? distP : T(-1);
         T beta = T(1);
         if (dp >= T(0)) {
           const T dc = fmax(dxq - rc, T(0));
-          beta = blend(tratio<FORM>(dp, dp + dc));
+          beta = blend(tratio<FORM, EXACT>(dp, dp + dc));
         }
         const T mx = m * beta;
         if (blendNode) {
@@ -1076,7 +1096,7 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
       }
       contrib = blendNode && shareSum != T(0);
     }
-    if (contrib) add_mom<FORM, KT>(acc, kp, mm, At, q, f);
+    if (contrib) add_mom<FORM, KT, EXACT>(acc, kp, mm, At, q, f);
     if constexpr (FORM == 1) {
       if (act && ++itc == kFlush) {
         acc.flush();
@@ -1135,12 +1155,12 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
     const uint4 hx = ld_uni(tv.hdr, xn);
     momX = load_mom_uni<FORM>(tv, xn);
     if (act) {
-      const T dxq = tdist<FORM>(q, gx);
+      const T dxq = tdist<FORM, EXACT>(q, gx);
       const T rc = (T)gx.w * cutoff;
       T beta = T(1);
       if (dp >= T(0)) {
         const T dc = fmax(dxq - rc, T(0));
-        beta = blend(tratio<FORM>(dp, dp + dc));
+        beta = blend(tratio<FORM, EXACT>(dp, dp + dc));
       }
       m = mp * beta;
       distP = fabs(dxq - rc);
@@ -1153,7 +1173,7 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
     shareSum = T(0);
     blendNode = hdr_depth(hx.y) >= minDepth;
     Ai = __uint_as_float(hx.z);
-    shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM>(T(1), (T)nc) : tratio<FORM>(T(1), (T)Ai);
+    shareScale = SEM == MLOD_SEM_REF_CPU ? tratio<FORM, EXACT>(T(1), (T)nc) : tratio<FORM, EXACT>(T(1), (T)Ai);
   }
 }
 
@@ -1344,10 +1364,12 @@ __global__ __launch_bounds__(64) void k_project_group(TreeView tv, KParams kp, f
     GroupSums gs;
     gs.init();
     const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
-    if (walk_narrow<FORM>(tv, qf, minDepth, live))
-      traverse_group<FORM, SEM, KT, false>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
+    if (!walk_short<FORM>(tv, qf, minDepth, live))
+      traverse_group<FORM, SEM, KT, true, FORM == 0>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
+    else if (tv.nn < (1u << 26))
+      traverse_group<FORM, SEM, KT, false, false>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
     else
-      traverse_group<FORM, SEM, KT, true>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
+      traverse_group<FORM, SEM, KT, true, false>(gs, kp, tv, qf, cutoff, minDepth, live, lds);
     lds.sum[grp][c] = FORM == 0 ? (double)gs.l0 : gs.k0.val();
     if (c == 0) lds.sum[grp][8] = FORM == 0 ? (double)gs.l8 : gs.k8.val();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1394,7 +1416,10 @@ __global__ __launch_bounds__(PBS) void k_project_wave(TreeView tv, KParams kp, f
       qt = V3<T>{qd.x, qd.y, qd.z};
     else
       qt = V3<T>{qf.x, qf.y, qf.z};
-    traverse_wave<FORM, SEM, KT, CNT>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
+    if (FORM != 0 || areas_normal(tv))
+      traverse_wave<FORM, SEM, KT, CNT, false>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
+    else
+      traverse_wave<FORM, SEM, KT, CNT, FORM == 0>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
     if constexpr (FORM == 1) acc.flush();
     if (live) fit_step<FORM, SEM>(acc, qd, qf, stepMax, nout);
   }
@@ -1552,6 +1577,7 @@ __global__ __launch_bounds__(PBS) void k_global_plain(TreeView tv, KParams kp, f
                                                 const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit,
                                                 uint32_t nIter, float stepMax) {
   __shared__ float4 sP[PBS], sN[PBS];
+  __shared__ V3<float> sM[PBS];
   const int tid = threadIdx.x;
   const uint32_t i = blockIdx.x * PBS + tid;
   const bool active = i < m && !(limit < m && perm[i] >= limit);
@@ -1567,17 +1593,12 @@ __global__ __launch_bounds__(PBS) void k_global_plain(TreeView tv, KParams kp, f
       if (base + tid < tv.n) {
         sP[tid] = tv.pts[base + tid];
         sN[tid] = tv.nrm[base + tid];
+        sM[tid] = point_mean(sP[tid]);
       }
       __syncthreads();
       const uint32_t cnt = min((uint32_t)PBS, tv.n - base);
-      if (active) {
-        TreeView lv = tv;
-        lv.pts = sP;
-        lv.nrm = sN;
-        for (uint32_t j = 0; j < cnt; ++j) {
-          add_point<0, KT>(acc, kp, lv, j, qf, 1.f);
-        }
-      }
+      if (active)
+        for (uint32_t j = 0; j < cnt; ++j) add_point_plain<KT>(acc, kp, sP[j], sN[j], sM[j], qf, 1.f);
     }
     fit_step<0, MLOD_SEM_REF_CPU>(acc, qd, qf, stepMax, nout);
   }
