@@ -519,18 +519,18 @@ __global__ __launch_bounds__(NBS) void k_ball_wave(TreeView tv, const float* __r
   }
 }
 
-// One step from FP64 sums over the neighbours in the global frame (CPUUtils.cpp:719-735): the
+// One step from FP64 sums over the neighbours (CPUUtils.cpp:719-735) about `o`, which is 0 in the FP64 form; the
 // compensated form moves them to the query's frame.
 template <int FORM>
-__device__ __forceinline__ void fit_sums(const double* S, V3<double>& qd, V3<float> qf, float4& nout) {
+__device__ __forceinline__ void fit_sums(const double* S, V3<float> o, V3<double>& qd, V3<float> qf, float4& nout) {
   V3<double> p, n;
   float kind;
   const V3<double> sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
   if constexpr (FORM == 1) {
-    const V3<double> q{qf.x, qf.y, qf.z};
+    const V3<double> q{(double)qf.x - o.x, (double)qf.y - o.y, (double)qf.z - o.z};
     fit_aliased<double>(S[0], V3<double>{sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0]}, sn, S[7] - dot3(q, sn),
                         S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0], V3<double>{0, 0, 0}, p, n, kind);
-    qd = V3<double>{q.x + p.x, q.y + p.y, q.z + p.z};
+    qd = V3<double>{(double)qf.x + p.x, (double)qf.y + p.y, (double)qf.z + p.z};
   } else {
     fit_aliased<double>(S[0], sp, sn, S[7], S[8], qd, p, n, kind);
     qd = p;
@@ -556,7 +556,10 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its wavefront's other
 // queries.  That holds for finite moments only (0 * NaN and 0 * infinity are NaN), so a cloud with a point that is
 // not finite goes to k_ball_wave, which leaves out what a ball does not hold (adding such points apart in this
-// kernel took 14 more registers, a wavefront a SIMD, and 7 % of every other cloud's time).  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
+// kernel took 14 more registers, a wavefront a SIMD, and 7 % of every other cloud's time).  The compensated form's sums are about a point of the cloud,
+// the middle one in the tree's order, and moved to the query at the end: that costs 1e-16 of the squared distance
+// between the two over the neighbourhood's, where the global frame costs it of the squared coordinates (a cloud 1e4
+// of its sizes from the origin, four sigmas of a twentieth: normals off by 1e-6, with the middle point 1e-7).  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
 // ones.  r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k 1.3;
 // FP64, 100k queries 1.6 (1.3 with weights.h's exponential).  Wavefronts of 64 queries (unions of four
 // times the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
@@ -585,6 +588,8 @@ __global__ __launch_bounds__(NBS) void k_ball_sums(TreeView tv, const float* __r
   float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
   bool done = !mine;
   const float r = sqrtf(r2f) * kSlack;
+  const float4 mid = tv.pts[tv.n >> 1];
+  const V3<float> o = FORM == 1 ? V3<float>{mid.x, mid.y, mid.z} : V3<float>{0.f, 0.f, 0.f};  // the sums' origin
   float4* pts = sPts[wv];
   double (*mom)[9] = sMom[wv];
   for (uint32_t it = 0; it < nIter; ++it) {
@@ -613,7 +618,8 @@ __global__ __launch_bounds__(NBS) void k_ball_sums(TreeView tv, const float* __r
             const uint32_t nb = min(64u, b - base);
             const bool in = (uint32_t)lane < nb;  // past the end: the first point with no moments
             const float4 P = tv.pts[base + (in ? (uint32_t)lane : 0u)], N = tv.nrm[base + (in ? (uint32_t)lane : 0u)];
-            const double e = in ? 1.0 : 0.0, x = P.x, y = P.y, z = P.z, nx = N.x, ny = N.y, nz = N.z;
+            const double e = in ? 1.0 : 0.0, x = (double)P.x - o.x, y = (double)P.y - o.y, z = (double)P.z - o.z;
+            const double nx = N.x, ny = N.y, nz = N.z;
             pts[lane] = P;
             mom[lane][0] = e;
             mom[lane][1] = e * x, mom[lane][2] = e * y, mom[lane][3] = e * z;
@@ -692,7 +698,7 @@ __global__ __launch_bounds__(NBS) void k_ball_sums(TreeView tv, const float* __r
         double S[9];
 #pragma unroll
         for (int c = 0; c < 9; ++c) S[c] = mom[lane][c];
-        fit_sums<FORM>(S, qd, qf, nout);
+        fit_sums<FORM>(S, o, qd, qf, nout);
       }
     }
     wave_order();

@@ -1440,14 +1440,15 @@ __global__ __launch_bounds__(PBS) void k_project_wave(TreeView tv, KParams kp, f
 }
 
 // ----------------------------------------------------------------------------- global APSS
-// One projection step from the nine sums over all neighbours, in the global frame in FP64:
-// {sum w, sum w p, sum w n, sum w p.n, sum w |p|^2}.  The compensated form moves them to the query's
-// frame (in FP64 that costs 1e-16 |q|^2 against the kernel's width squared).
+// One projection step from the nine sums over all neighbours in FP64, {sum w, sum w p, sum w n, sum w p.n,
+// sum w |p|^2}, about `o`, which is 0 in the FP64 form.  The compensated form takes them about a point of the cloud
+// and moves them to the query's frame (that costs 1e-16 of the squared distance between the two against the
+// kernel's width squared).
 template <int FORM, int SEM>
-__device__ __forceinline__ void fit_sums(const double* S, V3<double>& qd, float stepMax, float4& nout) {
+__device__ __forceinline__ void fit_sums(const double* S, V3<float> o, V3<double>& qd, float stepMax, float4& nout) {
   const V3<float> qf{(float)qd.x, (float)qd.y, (float)qd.z};
   if constexpr (FORM == 1) {
-    const V3<double> q{qf.x, qf.y, qf.z}, sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
+    const V3<double> q{(double)qf.x - o.x, (double)qf.y - o.y, (double)qf.z - o.z}, sp{S[1], S[2], S[3]}, sn{S[4], S[5], S[6]};
     const double R[9] = {S[0], sp.x - q.x * S[0], sp.y - q.y * S[0], sp.z - q.z * S[0], sn.x, sn.y, sn.z, S[7] - dot3(q, sn),
                          S[8] - 2.0 * dot3(q, sp) + dot3(q, q) * S[0]};
     fit_total<1, SEM>(R, qd, qf, stepMax, nout);
@@ -1490,6 +1491,8 @@ __global__ __launch_bounds__(W * 64) void k_global(TreeView tv, KParams kp, floa
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, row = lane & 15u, kk = lane >> 4, col = min(row, 8u);
   const uint32_t i = blockIdx.x * kGlobalQ + tid;
   const bool active = tid < kGlobalQ && i < m && !(limit < m && perm[i] >= limit);
+  const float4 mid = tv.pts[tv.n >> 1];
+  const V3<float> o = FORM == 1 ? V3<float>{mid.x, mid.y, mid.z} : V3<float>{0.f, 0.f, 0.f};  // the sums' origin
   V3<double> qd{0, 0, 0};  // (of the first 16 threads)
   float4 nout = make_float4(0.f, 0.f, 0.f, 0.f);
   if (active) {
@@ -1513,7 +1516,7 @@ __global__ __launch_bounds__(W * 64) void k_global(TreeView tv, KParams kp, floa
       for (uint32_t t = tid; t < end; t += W * 64) {
         const bool in = t < cnt;  // past the end: the tile's first point with no moments
         const float4 P = tv.pts[base + (in ? t : 0u)], N = tv.nrm[base + (in ? t : 0u)];
-        const double a = in ? (double)P.w : 0.0, x = P.x, y = P.y, z = P.z;
+        const double a = in ? (double)P.w : 0.0, x = (double)P.x - o.x, y = (double)P.y - o.y, z = (double)P.z - o.z;
         sP[t] = P;
         sF[t][0] = a;
         sF[t][1] = a * x, sF[t][2] = a * y, sF[t][3] = a * z;
@@ -1562,7 +1565,7 @@ __global__ __launch_bounds__(W * 64) void k_global(TreeView tv, KParams kp, floa
       sS[t / 9u][t % 9u] = x;
     }
     __syncthreads();
-    if (tid < kGlobalQ) fit_sums<FORM, MLOD_SEM_REF_CPU>(sS[tid], qd, stepMax, nout);
+    if (tid < kGlobalQ) fit_sums<FORM, MLOD_SEM_REF_CPU>(sS[tid], o, qd, stepMax, nout);
   }
   if (active) {
     q[i] = make_float4((float)qd.x, (float)qd.y, (float)qd.z, 0.f);
