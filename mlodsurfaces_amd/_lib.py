@@ -54,6 +54,7 @@ SIGNATURES = {
     "mlod_last_error": (C.c_char_p, []),
     "mlod_tree_create": (C.c_int, [_f, _f, C.c_uint32, C.POINTER(BuildOptsC), _vp, C.POINTER(_vp)]),
     "mlod_tree_create_device": (C.c_int, [_vp, _vp, C.c_uint32, C.POINTER(BuildOptsC), _vp, C.POINTER(_vp)]),
+    "mlod_memory_trim": (C.c_int, []),
     "mlod_tree_destroy": (C.c_int, [_vp]),
     "mlod_tree_get_info": (C.c_int, [_vp, C.POINTER(TreeInfoC)]),
     "mlod_set_kernel": (C.c_int, [_vp, C.POINTER(KernelC)]),

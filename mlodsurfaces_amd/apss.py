@@ -22,9 +22,15 @@ import numpy as np
 from . import _lib
 from ._lib import check, lib
 
-__all__ = ["Kernel", "APSSOctree", "APSS", "Fastapss", "GlobalAPSS", "MlodError"]
+__all__ = ["Kernel", "APSSOctree", "APSS", "Fastapss", "GlobalAPSS", "MlodError", "trim_memory"]
 
 MlodError = _lib.MlodError
+
+
+def trim_memory():
+    """Gives the device memory that the library keeps from freed octrees and queries (at most 1/64 of a
+    device's) back to the devices, e.g. for torch's allocator in the same process."""
+    check(lib().mlod_memory_trim())
 
 
 def _f32(a, name):

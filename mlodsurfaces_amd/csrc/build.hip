@@ -605,7 +605,7 @@ int dalloc(T** p, size_t count, uint64_t* bytes) {
   const size_t b = std::max<size_t>(count, 1) * sizeof(T);
   hipError_t e = dev_malloc(p, b);
   if (e != hipSuccess) return fail(MLOD_ERR_OOM, "hipMalloc of " + std::to_string(b) + " bytes failed");
-  if (bytes) *bytes += b;
+  if (bytes) *bytes += dev_block_bytes(*p);
   return MLOD_OK;
 }
 

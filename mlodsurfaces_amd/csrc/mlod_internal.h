@@ -187,6 +187,9 @@ __device__ __forceinline__ uint32_t xcd_block() {
 // hipFree does; several blocks given back together wait once.
 hipError_t dev_malloc_bytes(void** p, size_t bytes);
 void dev_free(void* const* ps, size_t n);
+hipError_t dev_malloc_raw(void** p, size_t bytes);  // past the cache (which is given back if need be); hipFree
+size_t dev_block_bytes(void* p);                    // what a block of dev_malloc holds
+void dev_trim();
 template <class T>
 inline hipError_t dev_malloc(T** p, size_t bytes) {
   return dev_malloc_bytes(reinterpret_cast<void**>(p), bytes);

@@ -246,7 +246,7 @@ namespace {
 
 template <class T>
 hipError_t dmalloc(T** p, size_t n) {
-  return hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T));
+  return dev_malloc_raw((void**)p, std::max<size_t>(n, 1) * sizeof(T));
 }
 template <class T>
 hipError_t hmalloc(T** p, size_t n) {
@@ -300,7 +300,7 @@ hipError_t alloc_stream(Stream& b, uint32_t cap) {
       (e = dmalloc(&b.dBlk, nblk)))
     return e;
   if ((e = rocprim::radix_sort_pairs(nullptr, b.sortBytes, b.dKey, b.dKey2, b.dIdx, b.dPerm, cap, 0, 40, b.s))) return e;
-  return hipMalloc(&b.sortTmp, b.sortBytes + 16);
+  return dev_malloc_raw(&b.sortTmp, b.sortBytes + 16);
 }
 
 void free_pool(mlod_server* S) {
