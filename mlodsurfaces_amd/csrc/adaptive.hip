@@ -59,14 +59,14 @@ struct GenState {
   uint32_t flags;
 };
 
-// An open-addressing table of keys, empty slots kNone, at least twice as many slots as keys are offered
-// (a probe so ends); the keys that enter it first go to `out`, in no particular order.  Most offers are
+// An open-addressing table of keys, empty slots kNone, twice as many slots as keys are offered (a probe so
+// ends; with the list of those that enter, 24 bytes an offer, what sorting them takes); the keys that enter it first go to `out`, in no particular order.  Most offers are
 // repeats (a cell's 64 slots hold some 10 new ones), which one load settles; sorting them all took up to
 // 20 launches and four waits a set.  generate() on 1M points, ms with each set sorted / hashed: depth 5 5.7 /
 // 4.3, 7 18.6 / 15.1, 8 36.4 / 31.1, 9 88 / 77, 10 294 / 260, 11 1086 / 967 (33M cells).
 struct CellSet {
   uint64_t* table;
-  uint64_t mask;  // slots - 1, slots a power of two
+  uint64_t slots;  // even
   uint64_t* out;
   GenState* st;
 };
@@ -76,15 +76,14 @@ __global__ __launch_bounds__(BS) void k_clear_set(CellSet set) {
   const uint64_t i0 = (uint64_t)blockIdx.x * BS + threadIdx.x;
   if (i0 == 0) set.st->count = 0;
   ulonglong2* t = reinterpret_cast<ulonglong2*>(set.table);
-  for (uint64_t i = i0; i <= set.mask / 2; i += stride) t[i] = make_ulonglong2(kNone, kNone);
+  for (uint64_t i = i0; i < set.slots / 2; i += stride) t[i] = make_ulonglong2(kNone, kNone);
 }
 
 // True for the one offer of `key` that enters it.
 __device__ __forceinline__ bool set_enter(const CellSet& set, uint64_t key) {
-  uint64_t h = key * 0x9e3779b97f4a7c15ull;
-  h ^= h >> 32;
-  for (;; ++h) {
-    unsigned long long* slot = reinterpret_cast<unsigned long long*>(set.table + (h & set.mask));
+  uint64_t h = __umul64hi(key * 0x9e3779b97f4a7c15ull, set.slots);
+  for (;; h = h + 1 < set.slots ? h + 1 : 0) {
+    unsigned long long* slot = reinterpret_cast<unsigned long long*>(set.table + h);
     // most offers find their key with a load (a stale one is settled by the exchange)
     const uint64_t seen = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (seen == key) return false;
@@ -350,9 +349,7 @@ struct mlod_generator {
   mlod_tree* tree = nullptr;
   mlod::KeyVec leaves, total;   // results, sorted and unique
   mlod::KeyVec a, b, c;         // work sets
-  mlod::KeyVec table;           // slots of the set that is being made
-  void* sortTmp = nullptr;
-  size_t sortBytes = 0;
+  mlod::KeyVec table;           // slots of the set that is being made, or a sort's temporary storage
   mlod::GenState* dState = nullptr;
   float* dXyz = nullptr;        // centres of the leaves (n x 3), valid after mlod_generator_centres
   size_t xyzCap = 0;
@@ -375,19 +372,14 @@ int KeyVec_append(KeyVec& v, const uint64_t* src, size_t m, hipMemcpyKind kind, 
   return MLOD_OK;
 }
 
-int ensure_sort_tmp(mlod_generator* g, size_t n, hipStream_t s) {
+int ensure_sort_tmp(mlod_generator* g, size_t n, size_t* bytes, hipStream_t s) {
   size_t need = 0, need2 = 0;
   MLOD_HIP(rocprim::radix_sort_keys(nullptr, need, (uint64_t*)nullptr, (uint64_t*)nullptr, n, 0, 64, s));
   MLOD_HIP(rocprim::unique(nullptr, need2, (uint64_t*)nullptr, (uint64_t*)nullptr, (uint64_t*)nullptr, n,
                            rocprim::equal_to<uint64_t>(), s));
   need = std::max(need, need2);
-  if (need <= g->sortBytes) return MLOD_OK;
-  MLOD_HIP(hipStreamSynchronize(s));
-  if (g->sortTmp) dev_free(g->sortTmp);
-  g->sortTmp = nullptr;
-  g->sortBytes = 0;
-  if (dev_malloc(&g->sortTmp, need + 256) != hipSuccess) return fail(MLOD_ERR_OOM, "adaptive octree: sort buffer");
-  g->sortBytes = need;
+  if (int r = g->table.reserve((need + 7) / 8, 0, s)) return r;
+  *bytes = g->table.cap * 8;
   return MLOD_OK;
 }
 
@@ -413,12 +405,13 @@ int sort_unique(mlod_generator* g, KeyVec& in, size_t n, KeyVec& out, size_t* m,
     return MLOD_OK;
   }
   if (n > 0xffffffffu) return fail(MLOD_ERR_UNSUPPORTED, "adaptive octree: more than 2^32 cells in one set");
-  if (int r = ensure_sort_tmp(g, n, s)) return r;
+  size_t tmp = 0;
+  if (int r = ensure_sort_tmp(g, n, &tmp, s)) return r;
   if (int r = out.reserve(n, 0, s)) return r;
-  size_t bytes = g->sortBytes;
-  MLOD_HIP(rocprim::radix_sort_keys(g->sortTmp, bytes, in.p, out.p, n, 0, 64, s));
-  bytes = g->sortBytes;
-  MLOD_HIP(rocprim::unique(g->sortTmp, bytes, out.p, in.p, &g->dState->count, n, rocprim::equal_to<uint64_t>(), s));
+  size_t bytes = tmp;
+  MLOD_HIP(rocprim::radix_sort_keys(g->table.p, bytes, in.p, out.p, n, 0, 64, s));
+  bytes = tmp;
+  MLOD_HIP(rocprim::unique(g->table.p, bytes, out.p, in.p, &g->dState->count, n, rocprim::equal_to<uint64_t>(), s));
   uint64_t cnt = 0, last = 0;
   const int flagged = read_state(g, &cnt, s);  // (the set is handed over all the same)
   if (flagged && flagged != MLOD_ERR_UNSUPPORTED) return flagged;
@@ -437,11 +430,10 @@ int sort_unique(mlod_generator* g, KeyVec& in, size_t n, KeyVec& out, size_t* m,
 // An empty set for `offers` keys, its cells to go to `out`.
 int begin_set(mlod_generator* g, size_t offers, KeyVec& out, CellSet* set, hipStream_t s) {
   if (offers > 0xffffffffu) return fail(MLOD_ERR_UNSUPPORTED, "adaptive octree: more than 2^32 cells in one set");
-  uint64_t slots = 4096;
-  while (slots < 2 * offers) slots *= 2;
+  const uint64_t slots = 2 * std::max<uint64_t>(offers, 2048);
   if (int r = out.reserve(offers, 0, s)) return r;
   if (int r = g->table.reserve(slots, 0, s)) return r;
-  *set = CellSet{g->table.p, slots - 1, out.p, g->dState};
+  *set = CellSet{g->table.p, slots, out.p, g->dState};
   k_clear_set<<<std::min<uint32_t>(blocks(slots / 2), 2048u), BS, 0, s>>>(*set);
   MLOD_HIP(hipGetLastError());
   return MLOD_OK;
@@ -641,7 +633,7 @@ int mlod_generator_destroy(mlod_generator* g) {
   if (!g) return MLOD_OK;
   (void)hipDeviceSynchronize();
   g->leaves.release(), g->total.release(), g->a.release(), g->b.release(), g->c.release(), g->table.release();
-  void* p[] = {g->sortTmp, g->dState, g->dXyz, g->dStage};
+  void* p[] = {g->dState, g->dXyz, g->dStage};
   dev_free(p, sizeof(p) / sizeof(p[0]));
   delete g;
   return MLOD_OK;
