@@ -109,7 +109,6 @@ struct QueryState {
   float4* qn;        // normals of the last step
   uint32_t* perm;    // sorted position -> caller's index
   float* stage;      // m x 3 staging for un-permuted download
-  float* hstage;     // pinned host staging (m x 3 x 2)
   uint32_t m = 0, cap = 0;
 };
 

@@ -1697,7 +1697,9 @@ void launch_batch_all(const ReqDesc* r, const uint2* blocks, uint32_t nblk, floa
 // the lane walk and is done in a third of its time while the chip has room for them.  Three steps on 1M
 // points, four sigmas, FP32C, us with a lane / a group: 4k queries 1140 / 427, 16k 1178 / 537, 32k
 // 1180 / 905, 48k 1271 / 1212, 64k 1289 / 1464; plain FP32, rational, cutoff 3, torus: 32k 5412 / 3097,
-// 48k 5673 / 4314, 64k 5807 / 5470.
+// 48k 5673 / 4314, 64k 5807 / 5470.  It is the uploaded queries that count, not those a call asks for: a few
+// of a large upload are walked a lane each, beside lanes that have nothing to do (they lie anywhere along the
+// curve, and wavefronts without one end at once).
 constexpr uint32_t kGroupMax = 49152;
 
 template <int FORM, int SEM, int KT, bool CNT>
