@@ -123,10 +123,15 @@ struct Counters {
   uint32_t far_, leafPts, tested, nearN, iters;
 };
 
-// A point's mean position (a p) / a in the plain form.  Areas here have any exponent (a subnormal one's reciprocal
-// overflows, that of one above 2^126 is flushed), so the divisions are the compiler's.
+// A point's mean position (a p) / a in the plain form.  EXACT: areas of any exponent (a subnormal one's reciprocal
+// overflows, that of one above 2^126 is flushed), the compiler's division; see areas_normal.
+template <bool EXACT>
 __device__ __forceinline__ V3<float> point_mean(float4 P) {
-  return V3<float>{(P.w * P.x) / P.w, (P.w * P.y) / P.w, (P.w * P.z) / P.w};
+  const float a = P.w, apx = a * P.x, apy = a * P.y, apz = a * P.z;
+  if constexpr (EXACT)
+    return V3<float>{apx / a, apy / a, apz / a};
+  else
+    return V3<float>{quot(apx, a), quot(apy, a), quot(apz, a)};
 }
 template <int KT, class KP>
 __device__ __forceinline__ void add_point_plain(AccP32& acc, const KP& kp, float4 P, float4 N, V3<float> mean, V3<float> q,
@@ -148,12 +153,12 @@ __device__ __forceinline__ void add_point_plain(AccP32& acc, const KP& kp, float
 
 // Contribution of one point (leaf member) with multiplier f, weight at the point's mean
 // position (a p) / a (Fastapss.cu:193; CPUUtils.cpp:455).
-template <int FORM, int KT, class KP>
+template <int FORM, int KT, bool EXACT, class KP>
 __device__ __forceinline__ void add_point(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv, uint32_t j,
                                           V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f) {
   const float4 P = tv.pts[j], N = tv.nrm[j];
   if constexpr (FORM == 0) {
-    add_point_plain<KT>(acc, kp, P, N, point_mean(P), q, f);
+    add_point_plain<KT>(acc, kp, P, N, point_mean<EXACT>(P), q, f);
   } else if constexpr (FORM == 1) {
     // the fused operations are written out: every kernel that adds a point rounds alike
     const float dx = P.x - q.x, dy = P.y - q.y, dz = P.z - q.z;
@@ -298,17 +303,17 @@ __device__ __forceinline__ void add_node(typename FormT<FORM>::Acc& acc, const K
   add_mom<FORM, KT, EXACT>(acc, kp, load_mom<FORM>(tv, c), Af, q, f);
 }
 
-template <int FORM, int SEM, int KT, bool CNT, class KP>
+template <int FORM, int SEM, int KT, bool CNT, bool EXACT = false, class KP>
 __device__ __forceinline__ void add_leaf(typename FormT<FORM>::Acc& acc, const KP& kp, const TreeView& tv, uint4 h,
                                          V3<typename FormT<FORM>::T> q, typename FormT<FORM>::T f, Counters& ct) {
   const uint32_t first = h.x, cnt = hdr_count(h.y);
   if constexpr (SEM == MLOD_SEM_REF_CPU) {
     // apssStats of a leaf is assigned, not summed, per point: only the last point stays
     // (CPUUtils.cpp:448-457).
-    add_point<FORM, KT>(acc, kp, tv, first + cnt - 1, q, f);
+    add_point<FORM, KT, EXACT>(acc, kp, tv, first + cnt - 1, q, f);
     if constexpr (CNT) ct.leafPts += 1;
   } else {
-    for (uint32_t j = first; j < first + cnt; ++j) add_point<FORM, KT>(acc, kp, tv, j, q, f);
+    for (uint32_t j = first; j < first + cnt; ++j) add_point<FORM, KT, EXACT>(acc, kp, tv, j, q, f);
     if constexpr (CNT) ct.leafPts += cnt;
   }
 }
@@ -511,11 +516,12 @@ __device__ __forceinline__ void swap_regs(float4& a, float4& b) {
 }
 __device__ __forceinline__ bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0ull; }
 
-// Whether no node of the tree has a subnormal area: a point's is its leaf's squared diagonal, at most 2^-12 of the
-// root's (2 r), over the leaf's points.
-__device__ __forceinline__ bool areas_normal(const TreeView& tv) {
-  const float r = tv.geo[0].w;
-  return r * r >= (float)tv.n * 0x1p-104f;
+// Whether the areas of all points and nodes are from 2^-126 to 2^126, where they have normal reciprocals: a point's
+// is its leaf's squared diagonal, at least 2^-12 of the root's (2 r), over the leaf's points; the points' sum is
+// the root's.
+__host__ __device__ __forceinline__ bool areas_normal(float radius, uint32_t points) {
+  const float r2 = radius * radius, n = (float)points;
+  return r2 >= n * 0x1p-104f && r2 * n <= 0x1p124f;
 }
 // Whether a wavefront's plain walk may take the short quotients and roots and the large distance term (uniform):
 // the areas have normal reciprocals, and no query is so far away that its distances overflow and meets nodes
@@ -525,7 +531,7 @@ __device__ __forceinline__ bool areas_normal(const TreeView& tv) {
 template <int FORM>
 __device__ __forceinline__ bool walk_short(const TreeView& tv, V3<float> q, uint32_t minDepth, bool live) {
   if constexpr (FORM == 1) return true;
-  bool ok = areas_normal(tv);
+  bool ok = areas_normal(tv.geo[0].w, tv.n);
   if (minDepth) ok = ok && !any_lane(live && !(fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fabsf(q.z)) < 1e18f));
   return ok;
 }
@@ -546,7 +552,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
   const float4* __restrict__ rec = FORM == 0 ? tv.recP : tv.recC;
   const uint4 h0 = tv.hdr[0];
   if (hdr_leaf(h0.y)) {  // a one-leaf tree (uniform)
-    if (live) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h0, q, 1.f, ct);
+    if (live) add_leaf<FORM, SEM, KT, CNT, EXACT>(acc, kp, tv, h0, q, 1.f, ct);
     if constexpr (FORM == 1) acc.flush();
     return;
   }
@@ -654,7 +660,7 @@ __device__ __forceinline__ void traverse_staged(typename FormT<FORM>::Acc& acc, 
       stage_issue<WIDE>(rec, idx, lane, stage);
       if (contrib) add_mom<FORM, KT, EXACT>(acc, kp, mm, At, q, f);
       if (any_lane(multi)) {  // a leaf of several points (at the last level, or by the build's option)
-        if (multi) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h, q, f, ct);
+        if (multi) add_leaf<FORM, SEM, KT, CNT, EXACT>(acc, kp, tv, h, q, f, ct);
       }
     }
     if constexpr (FORM == 1) acc.flush();
@@ -760,7 +766,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
     pick_sum<FORM>(a, c, gs.l0, gs.l8);
   };
   if (hdr_leaf(h0.y)) {  // a one-leaf tree (uniform)
-    if (live) single_term([&](auto& a) { add_leaf<FORM, SEM, KT, false>(a, kp, tv, h0, q, 1.f, ct); });
+    if (live) single_term([&](auto& a) { add_leaf<FORM, SEM, KT, false, EXACT>(a, kp, tv, h0, q, 1.f, ct); });
     gs.template flush<FORM>();
     return;
   }
@@ -902,7 +908,7 @@ __device__ __forceinline__ void traverse_group(GroupSums& gs, const KP& kp, cons
         const uint4 hj = make_uint4((uint32_t)__shfl((int)h.x, (int)(base + j), 64), (uint32_t)__shfl((int)h.y, (int)(base + j), 64), 0u, 0u);
         const float fj = __shfl(f, (int)(base + j), 64);
         const bool mj = __shfl((int)multi, (int)(base + j), 64) != 0;
-        if (mj) single_term([&](auto& t) { add_leaf<FORM, SEM, KT, false>(t, kp, tv, hj, q, fj, ct); });
+        if (mj) single_term([&](auto& t) { add_leaf<FORM, SEM, KT, false, EXACT>(t, kp, tv, hj, q, fj, ct); });
       }
       if constexpr (FORM == 1) {
         if (due == kGroup) gs.template flush<FORM>();
@@ -1015,7 +1021,7 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
   uint32_t itc = 0;  // the lane's own iterations since the last block flush (compensated form)
   const uint4 h0 = ld_uni(tv.hdr, 0u);
   if (hdr_leaf(h0.y)) {
-    if (live) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, h0, q, T(1), ct);
+    if (live) add_leaf<FORM, SEM, KT, CNT, EXACT>(acc, kp, tv, h0, q, T(1), ct);
     return;
   }
   const float4 g0 = ld_uni(tv.geo, 0u);
@@ -1076,7 +1082,7 @@ __device__ __forceinline__ void traverse_wave(typename FormT<FORM>::Acc& acc, co
           shareSum += (T(1) - beta) * share;
         }
         const bool far = !leaf && deep && dxq > rc;
-        if (leaf && !single) add_leaf<FORM, SEM, KT, CNT>(acc, kp, tv, hx, q, mx, ct);
+        if (leaf && !single) add_leaf<FORM, SEM, KT, CNT, EXACT>(acc, kp, tv, hx, q, mx, ct);
         nearc = !leaf && !far;
         if (nearc) nearb |= 1u << k;
         if constexpr (CNT) {
@@ -1386,7 +1392,7 @@ __global__ __launch_bounds__(64) void k_project_group(TreeView tv, KParams kp, f
 
 // k_project with the wave-shared walk: every lane of a wavefront calls the walk (lanes without a
 // query take part in no node), so the walk's control flow stays wave-uniform.
-template <int FORM, int SEM, int KT, bool CNT>
+template <int FORM, int SEM, int KT, bool CNT, bool EXACT>
 __global__ __launch_bounds__(PBS) void k_project_wave(TreeView tv, KParams kp, float4* __restrict__ q,
                                                       float4* __restrict__ qn, const uint32_t* __restrict__ perm,
                                                       uint32_t m, uint32_t limit, uint32_t nIter, float stepMax,
@@ -1416,10 +1422,7 @@ __global__ __launch_bounds__(PBS) void k_project_wave(TreeView tv, KParams kp, f
       qt = V3<T>{qd.x, qd.y, qd.z};
     else
       qt = V3<T>{qf.x, qf.y, qf.z};
-    if (FORM != 0 || areas_normal(tv))
-      traverse_wave<FORM, SEM, KT, CNT, false>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
-    else
-      traverse_wave<FORM, SEM, KT, CNT, FORM == 0>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
+    traverse_wave<FORM, SEM, KT, CNT, EXACT>(acc, kp, tv, qt, (T)cutoff, minDepth, live, st, tid, wv, ct, waveIters);
     if constexpr (FORM == 1) acc.flush();
     if (live) fit_step<FORM, SEM>(acc, qd, qf, stepMax, nout);
   }
@@ -1596,7 +1599,7 @@ __global__ __launch_bounds__(PBS) void k_global_plain(TreeView tv, KParams kp, f
       if (base + tid < tv.n) {
         sP[tid] = tv.pts[base + tid];
         sN[tid] = tv.nrm[base + tid];
-        sM[tid] = point_mean(sP[tid]);
+        sM[tid] = point_mean<true>(sP[tid]);
       }
       __syncthreads();
       const uint32_t cnt = min((uint32_t)PBS, tv.n - base);
@@ -1707,16 +1710,21 @@ int launch_one(const mlod_tree* t, const KParams& kp, uint32_t limit, uint32_t n
                unsigned long long* counters, hipStream_t s) {
   const uint32_t m = t->qs.m;
   if (m == 0) return MLOD_OK;
-  if (t->traversal == MLOD_TRAVERSAL_WAVE)
-    k_project_wave<FORM, SEM, KT, CNT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(
-        t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth, counters);
-  else if (FORM != 2 && !CNT && m <= kGroupMax)
+  if (t->traversal == MLOD_TRAVERSAL_WAVE) {
+    if (FORM != 0 || areas_normal(t->radius, t->n))
+      k_project_wave<FORM, SEM, KT, CNT, false><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(
+          t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth, counters);
+    else
+      k_project_wave<FORM, SEM, KT, CNT, FORM == 0><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(
+          t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth, counters);
+  } else if (FORM != 2 && !CNT && m <= kGroupMax) {
     k_project_group<FORM == 2 ? 1 : FORM, SEM, KT><<<(m + kGroups - 1) / kGroups, 64, 0, s>>>(
         t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m, limit, nIter, stepMax, t->cutoff, t->min_depth);
-  else
+  } else {
     k_project<FORM, SEM, KT, CNT><<<(m + PBS - 1) / PBS, PBS, 0, s>>>(t->view(), kp, t->qs.q, t->qs.qn, t->qs.perm, m,
                                                                        limit, nIter, stepMax, t->cutoff, t->min_depth,
                                                                        counters);
+  }
   return MLOD_OK;
 }
 
