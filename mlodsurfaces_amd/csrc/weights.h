@@ -127,6 +127,31 @@ __device__ __forceinline__ void weights32(const KP& k, const float (&d2)[U], flo
 #pragma unroll
       for (int u = 0; u < U; ++u) w[u] = w[u] == 0.f ? k.c : w[u];
     }
+  } else if constexpr (KT == MLOD_KERNEL_SINGULAR) {
+    if ((__float_as_uint(k.c) & 0x7fffffffu) > 0x0da24260u) {  // as weight32's, for all of them at once
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = quot(k.cp4, fmaf(d2[u], 0.25f, k.c4));
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = k.cp / (d2[u] + k.c);
+    }
+    if (k.eint > 0) {
+      float r[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) r[u] = 1.f;
+      for (int e = k.eint; e; e >>= 1) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (e & 1) r[u] *= w[u];
+          w[u] *= w[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = r[u];
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = __builtin_amdgcn_exp2f(k.e * __builtin_amdgcn_logf(w[u]));
+    }
   } else {
 #pragma unroll
     for (int u = 0; u < U; ++u) w[u] = weight32<KT>(k, d2[u]);
