@@ -16,6 +16,7 @@
 //     recC float4 x4 {geo}, {first, code, A, 1/A}, {pbar, C}, {N, V}      the same for the compensated
 //                                              form: centred moments (mean point, sum a n,
 //                                              sum a (p - pbar).n, sum a |p - pbar|^2)
+//            In both 1/A is held finite for a subnormal A.
 //            A walk that needs a whole node takes it in one 64-byte segment.
 //     momD double4 x2 + double                plain moments in FP64
 //   points, in leaf (sorted) order: pts float4 {p, a}, nrm float4 {n, 0}; order maps a

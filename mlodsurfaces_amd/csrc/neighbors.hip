@@ -18,7 +18,7 @@
 // leaves first and the k-th distance bound tightens early); small subtrees are scanned as
 // contiguous point ranges.  Candidates within the bound are buffered in LDS and merged, by all lanes
 // of a wavefront together, into a sorted array of 64-bit keys in registers (distance bits << 32 |
-// sorted point index).  The kernel is bound by vector instructions (VALU 94 % busy, k = 32): merging
+// sorted point index).  The kernel is bound by vector instructions (VALU 93 % busy, k = 32): merging
 // together runs the insertion about as often as the fullest lane needs it instead of once per point
 // that any lane takes (k = 32, 5M points, 4M queries, FP32C: 12.0 ms a step with 64-bit integer
 // compares, 7.7 with keys as doubles, 5.9 with the buffers).  Ball: one walk per wavefront over the union of
@@ -547,22 +547,23 @@ __device__ __forceinline__ void wave_order() {
 
 typedef double Acc4 __attribute__((ext_vector_type(4)));
 
-// The compensated and FP64 forms: a wavefront walks the union of 16 queries' balls, the sums on the matrix
-// cores.  A range's points go to LDS 64 at a time with their nine moments {1, p, n, p.n, |p|^2} in
-// FP64; then, four points a step and four steps at once, each lane weighs one (query lane % 16, point
-// lane / 16) pair a step, a pair outside its ball with weight 0, and an FP64 16x16x4 matrix
-// instruction adds the 64 weights times the points' moments.  A pair so costs its distance, test and
-// weight and none of the nine sums.  The ranges and the steps within them are the tree's, whatever the
-// queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its wavefront's other
-// queries.  That holds for finite moments only (0 * NaN and 0 * infinity are NaN), so a cloud with a point that is
-// not finite goes to k_ball_wave, which leaves out what a ball does not hold (adding such points apart in this
-// kernel took 14 more registers, a wavefront a SIMD, and 7 % of every other cloud's time).  The compensated form's sums are about a point of the cloud,
-// the middle one in the tree's order, and moved to the query at the end: that costs 1e-16 of the squared distance
-// between the two over the neighbourhood's, where the global frame costs it of the squared coordinates (a cloud 1e4
-// of its sizes from the origin, four sigmas of a twentieth: normals off by 1e-6, with the middle point 1e-7).  Bound by the weights' vector instructions at high query counts, by the walk's loads at low
-// ones.  r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k 1.3;
-// FP64, 100k queries 1.6 (1.3 with weights.h's exponential).  Wavefronts of 64 queries (unions of four
-// times the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
+// The compensated and FP64 forms: a wavefront walks the union of 16 queries' balls, the sums on the matrix cores. A
+// range's points go to LDS 64 at a time with their nine moments {1, p, n, p.n, |p|^2} in FP64; then, four points a
+// step and four steps at once, each lane weighs one (query lane % 16, point lane / 16) pair a step, a pair outside
+// its ball with weight 0, and an FP64 16x16x4 matrix instruction adds the 64 weights times the points' moments. A
+// pair so costs its distance, test and weight and none of the nine sums. The ranges and the steps within them are
+// the tree's, whatever the queries, and a zero weight leaves a sum as it is: a query's sums do not depend on its
+// wavefront's other queries. That holds for finite moments only (0 * NaN and 0 * infinity are NaN), so a cloud with
+// a point that is not finite goes to k_ball_wave, which leaves out what a ball does not hold (adding such points
+// apart in this kernel took 14 more registers, a wavefront a SIMD, and 7 % of every other cloud's time). The
+// compensated form's sums are about a point of the cloud, the middle one in the tree's order, and moved to the
+// query at the end: that costs 1e-16 of the squared distance between the two over the neighbourhood's, where the
+// global frame costs it of the squared coordinates (a cloud 1e4 of its sizes from the origin, four sigmas of a
+// twentieth: normals off by up to 1e-6, with the middle point 4e-8). Bound by the weights' vector instructions at high
+// query counts (500k: VALU 68 % busy, exponentials at a quarter of the rate; the matrix units 18 %), by the walk's
+// loads at low ones. r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k
+// 1.3; FP64, 100k queries 1.6 (1.3 with weights.h's exponential). Wavefronts of 64 queries (unions of four times
+// the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.
 constexpr uint32_t kBallQ = 16;            // queries a wavefront
 constexpr uint32_t kScanPointsBall = 512;  // subtrees up to this size are taken as one range (256: 1.65 ms, 1024: 1.57)
 

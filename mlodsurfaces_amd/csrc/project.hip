@@ -1472,7 +1472,8 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // their moments formed once per tile.
 // Step g of a tile belongs to slice g % 16; a wavefront holds 16 / W slices apart, and the slices are
 // added in order at the end, so the result does not depend on W.
-// Bound by the weights' vector instructions.  30k points, four sigmas, FP32C: 20k queries 6.0 -> 0.76 ms,
+// Bound by the weights' vector instructions (VALU 72 % busy, exponentials at a quarter of the rate; the matrix
+// units 33 %).  30k points, four sigmas, FP32C: 20k queries 6.0 -> 0.76 ms,
 // 500 queries 6.0 -> 0.19 (one lane per query left the chip two thirds empty, and each pair paid nine
 // compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries: 20.1 -> 1.05.
 // The fit uses the 1e-12 plane threshold of GlobalAPSS.cu:143 (the REF_CPU fit).
@@ -1577,7 +1578,9 @@ __global__ __launch_bounds__(W * 64) void k_global(TreeView tv, KParams kp, floa
 }
 
 // The plain FP32 form of global APSS: the reference's own sums, in FP32 and in point order, one lane per
-// query over point tiles in LDS.
+// query over point tiles in LDS, a point's mean divided out once a tile.  Bound by vector instructions and, up to
+// some 100k queries, by the chip being part empty: 20k queries, 30k points, four sigmas 5.3 ms (5.7 with the mean
+// formed for every pair), rational kernel 8.1 (9.4).
 template <int KT>
 __global__ __launch_bounds__(PBS) void k_global_plain(TreeView tv, KParams kp, float4* __restrict__ q, float4* __restrict__ qn,
                                                 const uint32_t* __restrict__ perm, uint32_t m, uint32_t limit,

@@ -13,11 +13,13 @@ namespace {
 // 8.1 ms a step, the same bits).  An approximation within an ulp, its residual by one fused operation,
 // which is exact, and one fused correction (Markstein, "Computation of elementary functions on the IBM
 // RISC System/6000 processor", 1990).  The expansions spend the rest on operands at the ends of the
-// exponent range.  Here the divisor is zero, from 2^-126 to 2^126 (a smaller one's reciprocal overflows, a larger one's is flushed) or
-// infinite, and the quotient is right where it and the residual are normal (above some 2^-100), and within an ulp
-// below; zeros, infinities and NaN go through the hardware's fix-up.  The square root is right from 2^-100 on,
+// exponent range.  Here the divisor is zero, infinite, or from 2^-126 to 2^126 (a smaller one's reciprocal
+// overflows, a larger one's is flushed), and the quotient is right where it and the residual are normal
+// (above some 2^-100), and within an ulp below; zeros, infinities and NaN go through the hardware's
+// fix-up.  The square root is right from 2^-100 on,
 // checked for every float there; below it loses up to an ulp, and a subnormal argument (a distance
-// under 1e-19) is returned as it is.
+// under 1e-19) is returned as it is.  Where areas or distances may lie outside, the plain walk has a variant with
+// the compiler's (walk_short in project.hip).
 __device__ __forceinline__ float quot_rcp(float n, float d, float r) {  // n / d, r = 1 / d correctly rounded
   const float q = __fmul_rn(n, r);
   return fmaf(fmaf(-d, q, n), r, q);
