@@ -560,7 +560,7 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // query at the end: that costs 1e-16 of the squared distance between the two over the neighbourhood's, where the
 // global frame costs it of the squared coordinates (a cloud 1e4 of its sizes from the origin, four sigmas of a
 // twentieth: normals off by up to 1e-6, with the middle point 4e-8). Bound by the weights' vector instructions at high
-// query counts (500k: VALU 68 % busy, exponentials at a quarter of the rate; the matrix units 18 %), by the walk's
+// query counts (500k: 58 % of the SIMDs' cycles, the matrix instructions 18 %), by the walk's
 // loads at low ones. r = 3 sigma0, 1M points (about 300 a ball), FP32C: 500k queries 4.8 -> 1.5 ms, 20k 1.0, 2k
 // 1.3; FP64, 100k queries 1.6 (1.3 with weights.h's exponential). Wavefronts of 64 queries (unions of four times
 // the surface, four times fewer wavefronts): 2.9, 3.1, 10.6, 4.6; of 32: 1.8, 1.5, 2.7, 2.5.

@@ -364,8 +364,8 @@ struct WalkStack {
 // such node is next.
 //
 // Bound by FP64 vector instructions (276 an iteration against 370: weights.h has the exponential, quotients and
-// roots, blend() the cosine, and no multiplier), with the L1 72 % busy beside them.  1M points, 400k queries, two steps, six sigmas:
-// 8.0 -> 4.75 ms; 1k queries 2.1 -> 1.3; a rational kernel, 400k queries, 7.4 -> 3.8.
+// roots, blend() the cosine, and no multiplier), with the L1 72 % busy beside them.  1M points, 400k queries,
+// two steps, six sigmas: 8.0 -> 4.75 ms; 1k queries 2.1 -> 1.3; a rational kernel, 400k queries, 7.4 -> 3.8.
 constexpr double kNoBlend64 = 1e300;  // a distance term that makes every blend factor exactly 1 (above minDepth)
 template <int FORM, int SEM, int KT, bool CNT, class KP>
 __device__ __forceinline__ void traverse_loads(AccP64& acc, const KP& kp, const TreeView& tv, V3<double> q, double cutoff,
@@ -1472,10 +1472,10 @@ typedef double Acc4 __attribute__((ext_vector_type(4)));
 // their moments formed once per tile.
 // Step g of a tile belongs to slice g % 16; a wavefront holds 16 / W slices apart, and the slices are
 // added in order at the end, so the result does not depend on W.
-// Bound by the weights' vector instructions (VALU 72 % busy, exponentials at a quarter of the rate; the matrix
-// units 33 %).  30k points, four sigmas, FP32C: 20k queries 6.0 -> 0.76 ms,
-// 500 queries 6.0 -> 0.19 (one lane per query left the chip two thirds empty, and each pair paid nine
-// compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries: 20.1 -> 1.05.
+// Bound by the weights' vector instructions and the FP64 products (56 % and 33 % of the SIMDs' cycles).  30k
+// points, four sigmas, FP32C: 20k queries 6.0 -> 0.80 ms, 500 queries 6.0 -> 0.19 (one lane per query left the
+// chip two thirds empty, and each pair paid nine compensated sums), 100k queries 6.4 -> 3.3; FP64, 8k queries:
+// 20.1 -> 1.05.
 // The fit uses the 1e-12 plane threshold of GlobalAPSS.cu:143 (the REF_CPU fit).
 constexpr int kGlobalQ = 16;
 constexpr int kSlices = 16;
