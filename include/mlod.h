@@ -108,11 +108,11 @@ int mlod_tree_create(const float* xyz, const float* nrm, uint32_t n, const mlod_
 /* Same from device-resident arrays. */
 int mlod_tree_create_device(const float* d_xyz, const float* d_nrm, uint32_t n, const mlod_build_opts* opts,
                             void* stream, mlod_tree** out);
-/* Fastapss::eraseFromGPU + APSS destructor (Fastapss.cu:486-511, GPUUtils.h:24). */
 /* The library keeps up to 1/64 of a device's memory in blocks that were freed, for its next allocations.
  * This gives them back to the device (all devices), for others in the process to use and before a
  * hipDeviceReset; allocations of the library do so by themselves when memory runs out. */
 int mlod_memory_trim(void);
+/* Fastapss::eraseFromGPU + APSS destructor (Fastapss.cu:486-511, GPUUtils.h:24). */
 int mlod_tree_destroy(mlod_tree* t);
 int mlod_tree_get_info(const mlod_tree* t, mlod_tree_info* out);
 
